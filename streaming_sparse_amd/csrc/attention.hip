@@ -34,8 +34,8 @@
 // The two key halves are merged through LDS at the end.
 #include "common.h"
 
+#include <algorithm>
 #include <atomic>
-
 #include <type_traits>
 
 using namespace ssa;
@@ -1037,59 +1037,74 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   }
 }
 
-// The split tiles' output: block (s, qw, dh) merges the K pieces of split
-// tile s (tile g = s % NB of workgroup split_from + s / NB) for queries
-// 32 qw .. 32 qw + 31 and dims 64 dh .. 64 dh + 63 (O = sum_j O_j
-// 2^(m_j - M), l likewise, M = max_j m_j, in piece order) and writes
-// out = O / l.  Lane l holds the epilogue's lane layout; every load is
-// issued before the first use.
-template <int K, int NB>
-__global__ __launch_bounds__(64) void merge_kernel(const float* part, uint16_t* out, int split_from, int T,
-                                                   long long q_tok, long long q_head) {
-  const int lane = threadIdx.x, s = blockIdx.x >> 2, qw = (blockIdx.x >> 1) & 1, dh = blockIdx.x & 1;
+// The split tiles' output: block (s, qw, dt) merges the `pieces` pieces of
+// split tile s (tile g = s % NB of workgroup split_from + s / NB) for queries
+// 32 qw .. 32 qw + 31 and dims 32 dt .. 32 dt + 31 (O = sum_j O_j 2^(m_j - M),
+// l likewise, M = max_j m_j, in piece order) and writes out = O / l.  Lane l
+// holds the epilogue's lane layout.  Bound by the latency of its loads: the
+// m and l of every piece are requested together, then the O of kMergeAhead
+// pieces at a time, and a tile spreads over 8 waves.  MAXP: the most pieces
+// an instance takes.
+constexpr int kMaxPieces = 16;
+constexpr int kMergeAhead = 4;
+
+template <int NB, int MAXP>
+__global__ __launch_bounds__(64) void merge_kernel(const float* part, uint16_t* out, int split_from, int pieces,
+                                                   int T, long long q_tok, long long q_head) {
+  const int lane = threadIdx.x, s = blockIdx.x >> 3, qw = (blockIdx.x >> 2) & 1, dt = blockIdx.x & 3;
   const int r = lane & 31, hh = lane >> 5;
   const int TB = T / NB, g = s % NB;
   const int work = split_from + s / NB;
   const int h = work / TB, t = (work % TB) * NB + g;
-  float mj[K], lj[K];
-  f32x4 v[K][2][4];
+  const float* const base = part + ((long long)(s / NB) * pieces * NB + g) * kPieceFloats;
+  auto piece = [&](int j) { return base + (long long)j * (NB * kPieceFloats); };
+  float w[MAXP], lj[MAXP];
 #pragma unroll
-  for (int j = 0; j < K; ++j) {
-    const float* sj = part + (long long)(((s / NB) * K + j) * NB + g) * kPieceFloats;
-    mj[j] = sj[8192 + qw * 32 + r];
-    lj[j] = sj[8256 + qw * 32 + r];
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj)
-        v[j][x][jj] = *reinterpret_cast<const f32x4*>(sj + ((qw * 16 + (2 * dh + x) * 4 + jj) * 64 + lane) * 4);
+  for (int j = 0; j < MAXP; ++j) {
+    // a uniform branch: the loads of all pieces go out before the first use
+    w[j] = -INFINITY;
+    lj[j] = 0.0f;
+    if (j < pieces) {
+      w[j] = piece(j)[8192 + qw * 32 + r];
+      lj[j] = piece(j)[8256 + qw * 32 + r];
+    }
   }
-  float M = -INFINITY;
+  float M = w[0];
 #pragma unroll
-  for (int j = 0; j < K; ++j) M = fmaxf(M, mj[j]);
-  f32x4 acc[2][4] = {};
+  for (int j = 1; j < MAXP; ++j) M = fmaxf(M, w[j]);
   float L = 0.0f;
 #pragma unroll
-  for (int j = 0; j < K; ++j) {
-    const float a = __builtin_amdgcn_exp2f(mj[j] - M);
-    L += lj[j] * a;
+  for (int j = 0; j < MAXP; ++j) {
+    w[j] = __builtin_amdgcn_exp2f(w[j] - M);
+    L += lj[j] * w[j];
+  }
+  f32x4 acc[4] = {};
+  constexpr int kAhead = MAXP < kMergeAhead ? MAXP : kMergeAhead;
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+  for (int j0 = 0; j0 < MAXP; j0 += kAhead) {
+    if (j0 >= pieces) break;
+    f32x4 v[kAhead][4];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      // past the last piece: re-read it, its weight is zero
+      const float* sj = piece(min(j0 + j, pieces - 1)) + ((qw * 16 + dt * 4) * 64 + lane) * 4;
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) v[j][jj] = *reinterpret_cast<const f32x4*>(sj + jj * 256);
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j)
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[x][jj][c] += v[j][x][jj][c] * a;
+        for (int c = 0; c < 4; ++c) acc[jj][c] += v[j][jj][c] * w[j0 + j];
   }
   const float inv = 1.0f / L;
   uint16_t* op = out + (long long)(t * 64 + qw * 32 + r) * q_tok + (long long)h * q_head + 4 * hh;
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const u32x2 w = {pack_bf16(acc[x][jj][0] * inv, acc[x][jj][1] * inv),
-                       pack_bf16(acc[x][jj][2] * inv, acc[x][jj][3] * inv)};
-      *reinterpret_cast<u32x2*>(op + 32 * (2 * dh + x) + 8 * jj) = w;
-    }
+  for (int jj = 0; jj < 4; ++jj) {
+    const u32x2 o = {pack_bf16(acc[jj][0] * inv, acc[jj][1] * inv), pack_bf16(acc[jj][2] * inv, acc[jj][3] * inv)};
+    *reinterpret_cast<u32x2*>(op + 32 * dt + 8 * jj) = o;
+  }
 }
 
 // Detail operand tiles of one head per block row: rops[h, rt] for the
@@ -1099,6 +1114,18 @@ __global__ __launch_bounds__(kRepOpChunks) void rep_operands_kernel(const uint16
   const int rt = blockIdx.x, h = blockIdx.y, c = threadIdx.x;
   const u32x4 w = rep_operand_chunk(detail + (long long)h * HP * 24, P, rt, c);
   *reinterpret_cast<u32x4*>(rops + ((long long)h * RT + rt) * (kRepOpBytes / 2) + 8 * c) = w;
+}
+
+// Merges `pieces` pieces of each of `tiles` split tiles (NB per workgroup).
+template <int NB>
+void launch_merge(const AttnParams& p, int tiles, int split_from, int pieces, hipStream_t stream) {
+  const dim3 grid(8 * tiles), block(64);
+  if (pieces <= 2)
+    hipLaunchKernelGGL((merge_kernel<NB, 2>), grid, block, 0, stream, p.part, p.out, split_from, pieces, p.T, p.q_tok,
+                       p.q_head);
+  else
+    hipLaunchKernelGGL((merge_kernel<NB, kMaxPieces>), grid, block, 0, stream, p.part, p.out, split_from, pieces, p.T,
+                       p.q_tok, p.q_head);
 }
 
 // Compute units of the current device (cached per device).
@@ -1121,18 +1148,45 @@ int device_cus(int* out) {
 }
 
 // The split a call runs: the workgroups past the last multiple of the CU
-// count run as pieces, so the last round spreads over every CU.  The
-// general call (NB = 1, two workgroups per CU) splits them in 2; the
-// two-block call (NB = 2, one per CU) in 4.  Returns the number of split
-// workgroups (0: none), the pieces per workgroup and the workspace bytes.
-int split_plan(int wgs, int nb, int* split_wgs, int* k, long long* bytes) {
+// count run as k pieces of their unit lists, merged by merge_kernel.  Returns
+// the number of split workgroups (0: none), the pieces per workgroup and the
+// workspace bytes.
+//
+// The chip holds `slots` workgroups at once (the general call two per CU, the
+// two-block call one).  The last round holds wgs mod slots of them; where
+// that leaves a whole CU's worth of work the first `cus` run whole.  k is the
+// most pieces that still start together: a piece that waits for a slot costs
+// its prologue, its state (33 KB) and a second latency-bound walk.  Measured
+// (captured in a graph; W workgroups, units each; k = 1, 2 and the rule's):
+// general W 24 x 36: 31.5, 24.7, 16.6 us (k 9); W 48 x 91: 70.9, 45.9, 28.4
+// (k 10, with 11: 37.0); W 144 x 46: 39.3, 40.0, 34.3 (k 3, with 4: 44.0);
+// W 288 x 91: 105.2, 92.6, 89.5 (k 8); W 432 x 46: 64.3 (the rule's k 1),
+// 76.8; W 504 x 91: 132.0 (k 1), 142.0; W 576 x 91: 192.3, 164.9, 158.4;
+// W 864 x 91: 241.7, 227.7 (k 2), with 3: 235.8.  Two-block W 22 x 308:
+// 217.0, 117.4, 41.4 (k 11, with 12: 60.9); W 216 x 432: 378.4 (k 1), 391.7;
+// W 432 x 72: 135.4 (k 1), 152.2, with 4: 148.5.
+// Pieces hold at least kMinUnits units (W 24 x 36: 2 units each 20.8 us, 4
+// units 16.6).
+constexpr int kMinUnits = 4;
+
+int split_plan(int wgs, int nb, int units, int* split_wgs, int* k, long long* bytes) {
   int cus = 0;
   const int e = device_cus(&cus);
   if (e != (int)hipSuccess) return e;
-  const int r = wgs % cus;
-  *split_wgs = r;
-  *k = nb == 1 ? 2 : 4;
-  *bytes = (long long)r * *k * nb * kPieceFloats * 4;
+  const int slots = nb == 1 ? 2 * cus : cus;
+  const int last = wgs % slots, r = wgs % cus;
+  int pieces = 1;
+  if (r > 0) {
+    pieces = (last >= cus ? slots - cus : slots) / r;
+    pieces = std::min(std::min(pieces, kMaxPieces), std::max(1, units / kMinUnits));
+    // a long two-block list whose last round fills at most 3/4 of the CUs:
+    // its quarters run in three quarter rounds (W 432: 432 units 750.7 ->
+    // 741.0 us, 72 units 135.4 -> 148.5)
+    if (nb == 2 && pieces == 1 && 4 * r <= 3 * cus && units >= 288) pieces = 4;
+  }
+  *split_wgs = pieces > 1 ? r : 0;
+  *k = pieces;
+  *bytes = (long long)*split_wgs * pieces * nb * kPieceFloats * 4;
   return (int)hipSuccess;
 }
 
@@ -1144,6 +1198,9 @@ constexpr int kTwoTerm = 1, kDense = 2, kStaged = 4;
 bool dense_call(int flags, int count, int pages, int n_tokens) {
   return (flags & kDense) && count == pages && (n_tokens / 64) % 2 == 0;
 }
+
+// Units of a tile's list, at most: the listed pages and the rep tiles.
+int unit_bound(int pages, int count, int nb) { return nb == 2 ? pages : count + (pages + 15) / 16; }
 
 // Workspace bytes of a staged call: two piece states per tile.
 long long staged_bytes(int wgs) { return (long long)wgs * 2 * kPieceFloats * 4; }
@@ -1174,7 +1231,7 @@ long long ssa_attention_workspace_bytes(int n_tokens, int heads, int pages, int 
   const int nb = dense_call(flags, count, pages, n_tokens) ? 2 : 1;
   int r = 0, k = 1;
   long long bytes = 0;
-  if (split_plan(heads * (n_tokens / 64) / nb, nb, &r, &k, &bytes) != (int)hipSuccess) return -1;
+  if (split_plan(heads * (n_tokens / 64) / nb, nb, unit_bound(pages, count, nb), &r, &k, &bytes) != (int)hipSuccess) return -1;
   return bytes;
 }
 
@@ -1244,7 +1301,7 @@ int ssa_attention(const void* q, const void* k, const void* v, const void* keys,
   // the last multiple of the CU count run as pieces, merged by merge_kernel
   int r = 0, pieces = 1;
   long long need = 0;
-  const int e = split_plan(wgs, nb, &r, &pieces, &need);
+  const int e = split_plan(wgs, nb, unit_bound(pages, count, nb), &r, &pieces, &need);
   if (e != (int)hipSuccess) return e;
   if (staged) {
     // the exact pages of every tile, then the rep tiles of every tile, each
@@ -1257,8 +1314,7 @@ int ssa_attention(const void* q, const void* k, const void* v, const void* keys,
       hipLaunchKernelGGL((attn_kernel<false, 1, 1>), dim3(wgs), dim3(kThreads), 0, stream, p);
       hipLaunchKernelGGL((attn_kernel<false, 1, 2>), dim3(wgs), dim3(kThreads), 0, stream, p);
     }
-    hipLaunchKernelGGL((merge_kernel<2, 1>), dim3(4 * wgs), dim3(64), 0, stream, p.part, p.out, 0, p.T, p.q_tok,
-                       p.q_head);
+    launch_merge<1>(p, wgs, 0, 2, stream);
     return (int)hipGetLastError();
   }
   if (r > 0 && workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0) {
@@ -1272,17 +1328,13 @@ int ssa_attention(const void* q, const void* k, const void* v, const void* keys,
       hipLaunchKernelGGL((attn_kernel<true, 2>), grid, dim3(2 * kThreads), 0, stream, p);
     else
       hipLaunchKernelGGL((attn_kernel<false, 2>), grid, dim3(2 * kThreads), 0, stream, p);
-    if (p.split_k > 1)
-      hipLaunchKernelGGL((merge_kernel<4, 2>), dim3(4 * 2 * (wgs - p.split_from)), dim3(64), 0, stream, p.part,
-                         p.out, p.split_from, p.T, p.q_tok, p.q_head);
+    if (p.split_k > 1) launch_merge<2>(p, 2 * (wgs - p.split_from), p.split_from, p.split_k, stream);
   } else {
     if (flags & kTwoTerm)
       hipLaunchKernelGGL((attn_kernel<true, 1>), grid, dim3(kThreads), 0, stream, p);
     else
       hipLaunchKernelGGL((attn_kernel<false, 1>), grid, dim3(kThreads), 0, stream, p);
-    if (p.split_k > 1)
-      hipLaunchKernelGGL((merge_kernel<2, 1>), dim3(4 * (wgs - p.split_from)), dim3(64), 0, stream, p.part,
-                         p.out, p.split_from, p.T, p.q_tok, p.q_head);
+    if (p.split_k > 1) launch_merge<1>(p, wgs - p.split_from, p.split_from, p.split_k, stream);
   }
   return (int)hipGetLastError();
 }

@@ -617,6 +617,83 @@ def test_attention_split_short_lists(device):
         check_out(out, want, f"short list {table.flatten().tolist()}")
 
 
+@pytest.mark.parametrize("heads,blocks,pages,count,pieces", [
+    (1, 1, 40, 9, 3),       # 12 units at most: pieces of kMinUnits = 4
+    (1, 3, 290, 61, 16),    # 80 units: the most pieces a merge takes, five units each
+    (1, 23, 97, 20, 6),     # an odd window: 27 units, pieces of 4 and 6
+    (3, 57, 100, 14, 2),    # 171 tiles: two pieces each
+    (2, 150, 96, 12, 4),    # 300 tiles: the 44 past the CU count, bounded by their units
+])
+def test_attention_many_pieces(device, heads, blocks, pages, count, pieces):
+    """Calls that leave CUs idle split every tile into the pieces that start
+    together (256 CUs, two workgroups each): within the bar of the oracle on
+    the first, a middle and the last block, and of the same call run whole
+    within 1e-3 rel-L2 (two-term: output roundings that flip) or 5e-3 (single:
+    two roundings of the probabilities, 2.3e-3 each, against different
+    maxima), with -1 padding in some rows, so that lists are shorter than the
+    pieces were planned for."""
+    from streaming_sparse_amd import _lib
+    gen = torch.Generator().manual_seed(heads * 1000 + blocks)
+    n = 64 * blocks
+    q = torch.randn(1, n, heads, 128, generator=gen).bfloat16()
+    k = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    v = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    vp = v[0].transpose(0, 1).reshape(heads, pages, 64, 128)
+    basis = workload.pca_basis(vp.float())
+    s = workload.kmeans_summaries(k[0].transpose(0, 1).reshape(heads, pages, 64, 128), vp, basis,
+                                  torch.Generator().manual_seed(9))
+    gd = Summary(*(getattr(s, f).to(device) for f in Summary.FIELDS))
+    ids = torch.stack([torch.randperm(pages, generator=gen)[:count] for _ in range(heads * blocks)])
+    ids = ids.reshape(heads, blocks, count).int()
+    ids[:, ::3, count // 3:] = -1
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        tail = heads * blocks % 256
+        assert _lib.lib().ssa_attention_workspace_bytes(n, heads, pages, count, 1) == tail * pieces * 33280
+    args = (q.to(device), k.to(device), v.to(device), gd, basis.to(device), ids.to(device))
+    tiles = sorted({0, blocks // 2, blocks - 1})
+    want = ref.selected_attention(q, k, v, s, basis, ids, tiles=tiles).bfloat16()
+    rows = torch.cat([torch.arange(t * 64, (t + 1) * 64) for t in tiles])
+    for single in (False, True):
+        ws = Workspace()
+        whole = attention(*args, ws, split=False, single_av=single).clone()
+        out = attention(*args, ws, single_av=single).clone()
+        torch.cuda.synchronize()
+        assert ref.rel_l2(out.float().cpu(), whole.float().cpu()) <= (5e-3 if single else 1e-3)
+        check_out(out[:, rows], want[:, rows], f"{heads}x{blocks} tiles, {pieces} pieces, single={single}")
+
+
+@pytest.mark.parametrize("heads,blocks,pages,pieces", [(1, 2, 7, 1), (1, 6, 70, 16), (2, 22, 60, 11), (8, 72, 24, 6),
+                                                       (12, 72, 290, 4)])
+def test_dense_many_pieces(device, heads, blocks, pages, pieces):
+    """The two-block kernel's pieces: a list too short to split, the most
+    pieces, one round of eleven, a tail bounded by its units, and the long
+    list whose tail runs in quarters; against dense attention on the first
+    and last block, and against the same call run whole."""
+    from streaming_sparse_amd import _lib
+    gen = torch.Generator().manual_seed(heads * 100 + blocks)
+    n = 64 * blocks
+    q = torch.randn(1, n, heads, 128, generator=gen).bfloat16()
+    k = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    v = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    z = lambda *shape: torch.zeros(heads, pages, *shape, device=device, dtype=torch.bfloat16)
+    gd = Summary(z(4, 128), z(128), z(3, 8), z(4, 12))
+    basis = torch.zeros(heads, 128, 8, device=device, dtype=torch.bfloat16)
+    ids = torch.arange(pages).expand(heads, blocks, -1).int().contiguous().to(device)
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        tail = heads * blocks // 2 % 256
+        assert _lib.lib().ssa_attention_workspace_bytes(n, heads, pages, pages, 2) == \
+            (tail * pieces * 2 * 33280 if pieces > 1 else 0)
+    ws = Workspace()
+    args = (q.to(device), k.to(device), v.to(device), gd, basis, ids)
+    whole = attention(*args, ws, all_pages=True, single_av=True, split=False).clone()
+    out = attention(*args, ws, all_pages=True, single_av=True).clone()
+    torch.cuda.synchronize()
+    assert ref.rel_l2(out.float().cpu(), whole.float().cpu()) <= 5e-3     # single-term, as above
+    rows = torch.cat([torch.arange(64), torch.arange(n - 64, n)])
+    want = ref.dense_attention(q[:, rows], k, v).bfloat16()
+    check_out(out[:, rows], want, f"dense {heads}x{blocks} blocks, {pieces} pieces")
+
+
 @pytest.mark.parametrize("blocks", [256, 257])
 def test_attention_split_boundary(device, blocks):
     """Tile counts at the CU-count boundary (256 CUs): 256 tiles run whole,
