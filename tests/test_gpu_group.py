@@ -35,3 +35,39 @@ def test_group_order_matches_oracle(device, first_chunk, history):
         print(f"layer {layer} first_chunk={first_chunk} history={history}: {int(same.sum())}/12 heads identical",
               flush=True)
         assert torch.equal(got[layer].long(), want)
+
+
+@pytest.mark.parametrize("scale,offset", [(1.0, 0.0), (1.0, 48.0), (12.0, 0.0)])
+def test_group_order_one_row(device, scale, offset):
+    """One layer and head (the smallest batch), and the statistics that are
+    merged over token blocks where they could cancel: keys far from zero, and
+    scores of standard deviation 12, whose softmax leaves a few tokens."""
+    gen = torch.Generator().manual_seed(int(scale + offset))
+    k = (scale * torch.randn(1, 4608, 1, 128, generator=gen) + offset).bfloat16()
+    v = torch.randn(1, 4608, 1, 128, generator=gen).bfloat16()
+    w = group.GroupWeights.seeded(1, 1, 7, torch.device("cpu"))
+    g = group.GroupWeights(*(t.to(device) for t in (w.bank, w.group_v, w.gate)))
+    got = group.order(k.to(device), v.to(device), g).cpu()
+    want = og.group_order(k[0].transpose(0, 1), v[0].transpose(0, 1), w.bank[0], w.group_v[0], w.gate[0])
+    assert torch.equal(got[0].long(), want)
+
+
+@pytest.mark.parametrize("distinct", [1, 7, 512])
+def test_group_order_is_stable_on_duplicates(device, distinct):
+    """Equal tokens have equal projections at every level, so the stable
+    sorts keep them in token order, through every merge of sorted runs; with
+    one distinct token every direction is zero and the order is the
+    identity."""
+    gen = torch.Generator().manual_seed(distinct)
+    rows = torch.randint(0, distinct, (4608,), generator=gen)
+    k = torch.randn(distinct, 2, 128, generator=gen).bfloat16()[rows][None].contiguous()
+    v = torch.randn(distinct, 2, 128, generator=gen).bfloat16()[rows][None].contiguous()
+    w = group.GroupWeights.seeded(1, 2, 8, device)
+    got = group.order(k.to(device), v.to(device), w).cpu().long()
+    for h in range(2):
+        assert torch.equal(got[0, h].sort().values, torch.arange(4608))
+        for r in range(distinct):
+            mine = got[0, h][rows[got[0, h]] == r]
+            assert bool((mine[1:] > mine[:-1]).all())
+    if distinct == 1:
+        assert torch.equal(got[0, 0], torch.arange(4608))
