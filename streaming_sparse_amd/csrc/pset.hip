@@ -35,9 +35,9 @@ constexpr int kAnchors = 24;
 constexpr int kCurrent = 72;
 constexpr int kFeatures = 712;
 constexpr int kMaxHidden = 256;
-constexpr int kEncPages = 4;        // pages per encode workgroup (the first-layer weights stream
-                                    // through each workgroup once: 4 pages balance that against the FMAs)
-static_assert(kEncPages % 4 == 0, "pages go to the four waves in turn");
+constexpr int kEncRows = 16;        // pages (of any heads) per MLP workgroup
+constexpr int kEncThreads = 512;
+constexpr int kProjPages = 32;      // pages of one head per projection workgroup
 constexpr int kCoefStride = 128;    // bf16 per page: co[85] | 0 x 11 | A[32]
 constexpr int kCoefA = 96;
 constexpr int kCand = 48;           // 16 removes + 32 adds
@@ -53,7 +53,7 @@ struct EncodeParams {
   const double* B;
   uint16_t* coef;
   double *mean_b, *detail_b;
-  int EP, first, pages, hidden;
+  int EP, heads, first, pages, hidden;
 };
 
 // Per-layer tensors of a batched encode (blockIdx.z = layer): the summary
@@ -68,13 +68,59 @@ struct EncodeLayers {
 struct OneLayer {};
 
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+  return wave_reduce(v, [](float a, float b) { return a + b; });
 }
 
+// D[16x16] += A[16x4] * B[4x16], fp32.  Lane l: A row l % 16, k = l / 16; B
+// column l % 16, same k; D column l % 16, rows 4 (l / 16) + i for item i.
+__device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Four floats at 4-byte alignment.
+struct alignas(4) Row4 { float v[4]; };
+__device__ __forceinline__ Row4 row4(const float* p, int valid) {
+  Row4 r;
+  if (valid >= 4) {
+    r = *reinterpret_cast<const Row4*>(p);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.v[i] = i < valid ? p[i] : 0.f;
+  }
+  return r;
+}
+
+constexpr int kFeatPad = 716, kHidPad = 260;     // floats per row: 16-byte aligned, rows on distinct banks
+union EncSmem {
+  struct {
+    union {
+      alignas(16) float f[kEncRows][kFeatPad];   // features
+      alignas(16) float hid[kEncRows][kHidPad];  // hidden units, once the features are used
+    } u;
+    float l1[2][kEncRows][kHidPad];              // layer 1 sums of the two halves of the features
+  } m;
+  struct {
+    double B[kHeadDim][16];
+    double pb[8][16];                            // bf16(basis)^T B of the head
+    uint16_t mean[kProjPages][kHeadDim + 8];
+  } b;
+};
+
+// The encodings of pages of all heads: workgroups 2 t and 2 t + 1 run the
+// reader and the phi MLP of pages 16 t .. 16 t + 15 of the flat (head, page)
+// range, the workgroups after them meanB and detailB of 32 pages of one head.
+// The MLPs are products of 16 pages by 16 units on the fp32 matrix pipe (fp32
+// products and sums).  Layer 1: wave w takes hidden units 64 (w % 4) .. + 63
+// over half w / 4 of the 712 features; lane (c = l % 16, g = l / 16) loads
+// units 4 c .. 4 c + 3 of a feature's weight row (256 bytes per row and
+// wave), well ahead, each item one product.  Bound by the fp32 matrix rate,
+// 9.5 us per workgroup, on the 108 CUs that 72 x 12 pages fill, then by the
+// latency of the steps around it.  72 x 12 pages, as part of a correction
+// call: 42 us (4 pages and both MLPs per workgroup as vector FMAs at one wave
+// per SIMD, layer 2 as 256-long serial dot products, meanB after it) -> 17;
+// 432 x 12 pages 126 -> 80.
 template <class Layers>
-__global__ __launch_bounds__(256) void encode_kernel(EncodeParams p, Layers layers) {
+__global__ __launch_bounds__(kEncThreads) void encode_kernel(EncodeParams p, Layers layers) {
   if constexpr (std::is_same_v<Layers, EncodeLayers>) {
     const int l = blockIdx.z;
     p.keys = layers.keys[l];
@@ -86,123 +132,187 @@ __global__ __launch_bounds__(256) void encode_kernel(EncodeParams p, Layers laye
     p.mean_b = layers.mean_b[l];
     p.detail_b = layers.detail_b[l];
   }
-  __shared__ alignas(16) float f[kFeatures][kEncPages];
-  __shared__ alignas(16) float hid[2 * kMaxHidden][kEncPages];
-  __shared__ double pb[8][16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int h = blockIdx.y;
-  const int g0 = blockIdx.x * kEncPages;
-  const int npg = min(kEncPages, p.pages - g0);
-
-  // features: wave w normalises pages w, w + 4, ...
-  for (int j = 0; j < kEncPages / 4; ++j) {
-    const int pl = 4 * j + wave;
-    if (pl >= npg) break;
-    const long long pg = (long long)h * p.HP + p.first + g0 + pl;
-    float kv[8];
-    const u32x4 k4 = ldg16(p.keys + pg * 512 + lane * 8);
+  __shared__ EncSmem smem;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int total = p.heads * p.pages;
+  const int mlps = 2 * ((total + kEncRows - 1) / kEncRows);
+  if ((int)blockIdx.x >= mlps) {
+    auto& s = smem.b;
+    const int chunks = (p.pages + kProjPages - 1) / kProjPages;
+    const int h = (blockIdx.x - mlps) / chunks, g0 = ((blockIdx.x - mlps) % chunks) * kProjPages;
+    const int npg = min(kProjPages, p.pages - g0);
+    const long long page0 = (long long)h * p.HP + p.first + g0, enc0 = (long long)h * p.EP + p.first + g0;
+    for (int i = tid; i < kHeadDim * 16; i += kEncThreads) s.B[i >> 4][i & 15] = p.B[i];
+    for (int i = tid; i < npg * 16; i += kEncThreads)
+      *reinterpret_cast<u32x4*>(&s.mean[i >> 4][8 * (i & 15)]) = ldg16(p.mean + (page0 + (i >> 4)) * kHeadDim + 8 * (i & 15));
+    const int o = tid >> 2, part = tid & 3, e = tid & 15;
+    uint16_t bs[32];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      kv[2 * w] = bf16_lo(k4[w]);
-      kv[2 * w + 1] = bf16_hi(k4[w]);
+    for (int i = 0; i < 32; ++i) bs[i] = p.basis[((long long)h * kHeadDim + 4 * i + part) * 8 + (o >> 4)];
+    __syncthreads();
+    // four threads per element of pb, 32 of the 128 dims each
+    double pb = 0.0;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) pb = fma((double)bf16_to_f32(bs[i]), s.B[4 * i + part][o & 15], pb);
+    pb += xor_lane<1>(pb);
+    pb += xor_lane<2>(pb);
+    if (part == 0) s.pb[o >> 4][o & 15] = pb;
+    if ((tid >> 4) < npg) {
+      double acc = 0.0;
+#pragma unroll 16
+      for (int d = 0; d < kHeadDim; ++d) acc = fma((double)bf16_to_f32(s.mean[tid >> 4][d]), s.B[d][e], acc);
+      p.mean_b[(enc0 + (tid >> 4)) * 16 + e] = acc;
     }
-    float ks = 0.f;
+    __syncthreads();
+    for (int i = tid; i < npg * 48; i += kEncThreads) {
+      const int pl = i / 48, a = (i / 16) % 3;
+      double acc = 0.0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) ks += kv[i] * kv[i];
-    const uint32_t mw = *reinterpret_cast<const uint32_t*>(p.mean + pg * 128 + lane * 2);
-    const float m0 = bf16_lo(mw), m1 = bf16_hi(mw);
-    const float dv = lane < 24 ? bf16_to_f32(p.detail[pg * 24 + lane]) : 0.f;
-    const float sv = lane < 48 ? bf16_to_f32(p.stats[pg * 48 + lane]) : 0.f;
-    const float kd = sqrtf(wave_sum(ks) / 512.f) + 1e-4f;
-    const float md = sqrtf(wave_sum(m0 * m0 + m1 * m1) / 128.f) + 1e-4f;
-    const float dd = sqrtf(wave_sum(dv * dv) / 24.f) + 1e-4f;
-    const float sd = sqrtf(wave_sum(sv * sv) / 48.f) + 1e-4f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) f[lane * 8 + i][pl] = kv[i] / kd;
-    f[512 + 2 * lane][pl] = m0 / md;
-    f[512 + 2 * lane + 1][pl] = m1 / md;
-    if (lane < 24) f[640 + lane][pl] = dv / dd;
-    if (lane < 48) f[664 + lane][pl] = sv / sd;
+      for (int k = 0; k < 8; ++k)
+        acc += (double)bf16_to_f32(p.detail[(page0 + pl) * 24 + a * 8 + k]) * s.pb[k][i & 15];
+      p.detail_b[((enc0 + pl) * 3 + a) * 16 + (i & 15)] = acc;
+    }
+    return;
   }
-  // bf16(basis)^T B for this head
-  if (tid < 128) {
-    const int k = tid >> 4, e = tid & 15;
-    double acc = 0.0;
-#pragma unroll 32
-    for (int d = 0; d < 128; ++d)
-      acc += (double)bf16_to_f32(p.basis[((long long)h * 128 + d) * 8 + k]) * p.B[d * 16 + e];
-    pb[k][e] = acc;
+  auto& s = smem.m;
+  const bool phi = blockIdx.x & 1;
+  const int r0 = (blockIdx.x >> 1) * kEncRows;
+  const int nrow = min(kEncRows, total - r0);
+
+  // the first weight rows are requested before anything else
+  const int H = p.hidden, c = lane & 15, g = lane >> 4;
+  constexpr int kHalf = kFeatures / 2, kSteps = kHalf / 16;      // 356 = 22 x 16 + 4
+  static_assert(kHalf == 16 * kSteps + 4, "one product after the full steps");
+  constexpr int kAhead = 4;        // steps of weight rows in flight
+  const int unit = 64 * (wave & 3) + 4 * c, half = wave >> 2;
+  const int valid = H - unit;      // units past H load zero
+  const float* w1 = p.w1t + (long long)(half * kHalf) * 2 * H + (phi ? H : 0) + min(unit, H - 1);
+  Row4 wr[kAhead][4];
+  auto load = [&](int st, Row4 (&r)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = row4(w1 + (long long)(16 * min(st, kSteps - 1) + 4 * g + i) * 2 * H, valid);
+  };
+#pragma unroll
+  for (int st = 0; st < kAhead; ++st) load(st, wr[st]);
+  const Row4 last = row4(w1 + (long long)(16 * kSteps + g) * 2 * H, valid);
+
+  // features: wave w normalises rows 2 w and 2 w + 1 (rows past the last
+  // re-read it; their outputs are not written)
+  {
+    u32x4 k4[2];
+    uint32_t mw[2];
+    float dv[2], sv[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = min(r0 + 2 * wave + i, total - 1);
+      const long long pg = (long long)(r / p.pages) * p.HP + p.first + r % p.pages;
+      k4[i] = ldg16(p.keys + pg * 512 + lane * 8);
+      mw[i] = *reinterpret_cast<const uint32_t*>(p.mean + pg * 128 + lane * 2);
+      dv[i] = lane < 24 ? bf16_to_f32(p.detail[pg * 24 + lane]) : 0.f;
+      sv[i] = lane < 48 ? bf16_to_f32(p.stats[pg * 48 + lane]) : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float kv[8];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        kv[2 * w] = bf16_lo(k4[i][w]);
+        kv[2 * w + 1] = bf16_hi(k4[i][w]);
+      }
+      float ks = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ks += kv[j] * kv[j];
+      const float m0 = bf16_lo(mw[i]), m1 = bf16_hi(mw[i]);
+      const float kd = sqrtf(wave_sum(ks) / 512.f) + 1e-4f;
+      const float md = sqrtf(wave_sum(m0 * m0 + m1 * m1) / 128.f) + 1e-4f;
+      const float dd = sqrtf(wave_sum(dv[i] * dv[i]) / 24.f) + 1e-4f;
+      const float sd = sqrtf(wave_sum(sv[i] * sv[i]) / 48.f) + 1e-4f;
+      float* f = s.u.f[2 * wave + i];
+      *reinterpret_cast<f32x4*>(f + 8 * lane) = f32x4{kv[0] / kd, kv[1] / kd, kv[2] / kd, kv[3] / kd};
+      *reinterpret_cast<f32x4*>(f + 8 * lane + 4) = f32x4{kv[4] / kd, kv[5] / kd, kv[6] / kd, kv[7] / kd};
+      f[512 + 2 * lane] = m0 / md;
+      f[512 + 2 * lane + 1] = m1 / md;
+      if (lane < 24) f[640 + lane] = dv[i] / dd;
+      if (lane < 48) f[664 + lane] = sv[i] / sd;
+    }
   }
   __syncthreads();
 
-  // layer 1 of both MLPs: thread j -> reader hidden j and phi hidden j
-  const int H = p.hidden;
-  if (tid < H) {
-    float ar[kEncPages], ap[kEncPages];
+  // layer 1: step s, item i of its four products: features 16 s + 4 g + i of
+  // this half (the last step's one product: feature 352 + g)
+  {
+    if (64 * (wave & 3) < H) {
+      const float* x = &s.u.f[c][half * kHalf];
+      f32x4 acc[4] = {};
+#pragma unroll 1
+      for (int s0 = 0; s0 < kSteps; s0 += kAhead) {
 #pragma unroll
-    for (int i = 0; i < kEncPages; ++i) ar[i] = ap[i] = 0.f;
-    const float* wr = p.w1t + tid;
-    const float* wp = p.w1t + H + tid;
-    // 32 rows of the weights in flight per thread: the loop streams 1.46 MB
-    // of weights through each workgroup and waits on their latency otherwise
-#pragma unroll 32
-    for (int k = 0; k < kFeatures; ++k) {
-      const float a = wr[(long long)k * 2 * H], b = wp[(long long)k * 2 * H];
+        for (int k = 0; k < kAhead; ++k) {
+          if (s0 + k < kSteps) {
+            const f32x4 xv = *reinterpret_cast<const f32x4*>(x + 16 * (s0 + k) + 4 * g);
 #pragma unroll
-      for (int c = 0; c < kEncPages / 4; ++c) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(&f[k][4 * c]);
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          ar[4 * c + i] = fmaf(x[i], a, ar[4 * c + i]);
-          ap[4 * c + i] = fmaf(x[i], b, ap[4 * c + i]);
+              for (int t = 0; t < 4; ++t) acc[t] = mfma16(wr[k][i].v[t], xv[i], acc[t]);
+            load(s0 + k + kAhead, wr[k]);
+          }
         }
       }
-    }
-    const float br = p.b1[tid], bp = p.b1[H + tid];
+      {
+        const float xv = x[16 * kSteps + g];
 #pragma unroll
-    for (int i = 0; i < kEncPages; ++i) {
-      const float xr = ar[i] + br, xp = ap[i] + bp;
-      hid[tid][i] = 0.5f * xr * (1.0f + erff(xr * 0.70710678118654752f));
-      hid[H + tid][i] = 0.5f * xp * (1.0f + erff(xp * 0.70710678118654752f));
+        for (int t = 0; t < 4; ++t) acc[t] = mfma16(last.v[t], xv, acc[t]);
+      }
+      // acc[t] item i: page c, unit 64 (w % 4) + 4 (4 g + i) + t
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<f32x4*>(&s.l1[half][c][64 * (wave & 3) + 4 * (4 * g + i)]) =
+            f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
     }
+  }
+  // layer 2: 85 reader or 32 phi outputs per page; wave w takes outputs 16 w
+  // .. + 15 of all pages, hidden units 16 s + 4 g + i in product i of step s.
+  // Its weights are requested here, ahead of the hidden units.
+  const int outs = phi ? 32 : 85;
+  const int o = 16 * wave + c;
+  const float* w = (phi ? p.w2p : p.w2r) + (long long)min(o, outs - 1) * H;
+  Row4 w2[16];
+  if (16 * wave < outs) {
+#pragma unroll
+    for (int st = 0; st < 16; ++st) w2[st] = row4(w + 16 * st + 4 * g, H - 16 * st - 4 * g);
   }
   __syncthreads();
-
-  // layer 2: 85 reader + 32 phi outputs per page, rounded to bf16
-  for (int idx = tid; idx < 117 * kEncPages; idx += 256) {
-    const int o = idx / kEncPages, pl = idx % kEncPages;
-    if (pl >= npg) continue;
-    const bool rd = o < 85;
-    const float* w = rd ? p.w2r + (long long)o * H : p.w2p + (long long)(o - 85) * H;
-    const int off = rd ? 0 : H;
-    float acc = 0.f;
-    for (int j = 0; j < H; ++j) acc = fmaf(hid[off + j][pl], w[j], acc);
-    acc += rd ? p.b2r[o] : p.b2p[o - 85];
-    const long long base = ((long long)h * p.EP + p.first + g0 + pl) * kCoefStride;
-    p.coef[base + (rd ? o : kCoefA + o - 85)] = to_bf16(acc);
+  for (int i = tid; i < kEncRows * kMaxHidden; i += kEncThreads) {
+    const int r = i / kMaxHidden, j = i % kMaxHidden;
+    float y = 0.f;
+    if (j < H) {
+      const float x = (s.l1[0][r][j] + s.l1[1][r][j]) + p.b1[(phi ? H : 0) + j];
+      y = 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
+    }
+    s.u.hid[r][j] = y;
   }
-  for (int idx = tid; idx < 11 * kEncPages; idx += 256) {
-    const int pl = idx / 11;
-    if (pl < npg) p.coef[((long long)h * p.EP + p.first + g0 + pl) * kCoefStride + 85 + idx % 11] = 0;
-  }
-  // meanB and detailB (fp64)
-  for (int idx = tid; idx < kEncPages * 16; idx += 256) {
-    const int pl = idx >> 4, e = idx & 15;
-    if (pl >= npg) continue;
-    const long long pg = (long long)h * p.HP + p.first + g0 + pl;
-    double acc = 0.0;
-#pragma unroll 32
-    for (int d = 0; d < 128; ++d) acc += (double)bf16_to_f32(p.mean[pg * 128 + d]) * p.B[d * 16 + e];
-    p.mean_b[((long long)h * p.EP + p.first + g0 + pl) * 16 + e] = acc;
-  }
-  for (int idx = tid; idx < kEncPages * 48; idx += 256) {
-    const int pl = idx / 48, a = (idx / 16) % 3, e = idx & 15;
-    if (pl >= npg) continue;
-    const long long pg = (long long)h * p.HP + p.first + g0 + pl;
-    double acc = 0.0;
+  __syncthreads();
+  if (16 * wave >= outs) return;
+  f32x4 acc[4] = {};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) acc += (double)bf16_to_f32(p.detail[pg * 24 + a * 8 + k]) * pb[k][e];
-    p.detail_b[(((long long)h * p.EP + p.first + g0 + pl) * 3 + a) * 16 + e] = acc;
+  for (int st = 0; st < 16; ++st) {
+    const f32x4 xv = *reinterpret_cast<const f32x4*>(&s.u.hid[c][16 * st + 4 * g]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = mfma16(w2[st].v[i], xv[i], acc[i]);
+  }
+  if (c >= nrow) return;
+  const int r = r0 + c;
+  uint16_t* cf = p.coef + ((long long)(r / p.pages) * p.EP + p.first + r % p.pages) * kCoefStride;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int oo = 16 * wave + 4 * g + i;
+    if (oo < outs) {
+      const float y = ((acc[0][i] + acc[1][i]) + (acc[2][i] + acc[3][i])) + (phi ? p.b2p[oo] : p.b2r[oo]);
+      cf[phi ? kCoefA + oo : oo] = to_bf16(y);
+    } else if (!phi) {
+      cf[oo] = 0;       // 85 .. 95: padding between co and A
+    }
   }
 }
 
@@ -967,11 +1077,13 @@ int encode_launch(const EncodeLayers* layers, int nlayers, const void* keys, con
   p.first = first_page;
   p.pages = pages;
   p.hidden = hidden;
-  const dim3 grid((pages + kEncPages - 1) / kEncPages, heads, nlayers);
+  p.heads = heads;
+  const dim3 grid(2 * ((heads * pages + kEncRows - 1) / kEncRows) + heads * ((pages + kProjPages - 1) / kProjPages), 1,
+                  nlayers);
   if (layers)
-    hipLaunchKernelGGL((encode_kernel<EncodeLayers>), grid, dim3(256), 0, stream, p, *layers);
+    hipLaunchKernelGGL((encode_kernel<EncodeLayers>), grid, dim3(kEncThreads), 0, stream, p, *layers);
   else
-    hipLaunchKernelGGL((encode_kernel<OneLayer>), grid, dim3(256), 0, stream, p, OneLayer{});
+    hipLaunchKernelGGL((encode_kernel<OneLayer>), grid, dim3(kEncThreads), 0, stream, p, OneLayer{});
   return (int)hipGetLastError();
 }
 

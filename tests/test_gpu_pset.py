@@ -61,6 +61,36 @@ def test_encode_matches_oracle(device):
     assert (enc.coef[..., 85:96] == 0).all()
 
 
+@pytest.mark.parametrize("heads,pages,first,hidden", [
+    (1, 1, 0, 256),       # one row of one tile
+    (3, 5, 11, 256),      # a tile of 15 rows over three heads
+    (1, 17, 3, 200),      # a tile and one row; hidden units that end inside a wave's 64
+    (2, 33, 0, 33),       # an odd hidden width (no 16-byte weight rows), 33 pages = two projection chunks
+    (12, 3, 2, 1),        # the smallest hidden width
+])
+def test_encode_tiles_match_oracle(device, heads, pages, first, hidden):
+    """Encodings of pages [first, first + pages) at the edges of the 16-row
+    tiles over (head, page), of the 32-page projection chunks and of the
+    hidden width; the bar of test_encode_matches_oracle per value, and pages
+    outside the range untouched."""
+    x, _, _, _ = inputs(9)
+    w = workload.reader_weights(5, hidden)
+    cap = first + pages + 2
+    s = type(x.summary)(*(getattr(x.summary, f)[:heads, :cap].contiguous().to(device) for f in x.summary.FIELDS))
+    enc = pset.Encoding.empty(heads, cap, device)
+    pset.encode(s, x.basis[:heads].to(device), pset.Reader(w, device), out=enc, first=first, pages=pages)
+    torch.cuda.synchronize()
+    want = opset.encode(*(getattr(x.summary, f)[:heads, :cap] for f in x.summary.FIELDS), x.basis[:heads], w)
+    r = slice(first, first + pages)
+    for got, ref_v in ((enc.co[:, r].cpu(), want['co'][:, r]), (enc.A[:, r].cpu(), want['A'][:, r])):
+        err = (got.float() - ref_v.float()).abs()
+        assert bool((err <= ref_v.float().abs() * 2.0 ** -7 + 1e-6).all())
+    torch.testing.assert_close(enc.mean[:, r].cpu(), want['mean'][:, r], atol=1e-12, rtol=1e-12)
+    torch.testing.assert_close(enc.detail[:, r].cpu(), want['detail'][:, r], atol=1e-12, rtol=1e-12)
+    for t in (enc.coef, enc.mean, enc.detail):
+        assert bool((t[:, :first] == 0).all()) and bool((t[:, first + pages:] == 0).all())
+
+
 def _near_tie(scores, legal, rel=1e-3):
     """Rows whose decision is fragile: best two legal scores, or the best
     score and 0, within `rel` of the row's score scale."""
