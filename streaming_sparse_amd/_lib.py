@@ -12,6 +12,8 @@ import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libssattn.so")
 _lib = None
+_raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream', None) or \
+    (lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 _vp, _i, _ll, _f = ctypes.c_void_p, ctypes.c_int, ctypes.c_longlong, ctypes.c_float
 # return type of the entry points that do not return a status
@@ -74,7 +76,9 @@ def use(path):
 
 
 def ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """The tensor's device pointer as an int (None -> NULL); every entry point
+    declares its pointer arguments as void pointers, which take it as it is."""
+    return None if t is None else t.data_ptr()
 
 
 def ptrs(tensors):
@@ -84,7 +88,14 @@ def ptrs(tensors):
 
 
 def stream_handle(device=None):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current stream of `device` (default: the current device), as an
+    int.  A device with an index is asked for its raw stream directly: the
+    Stream object that torch.cuda.current_stream makes costs more than a
+    kernel launch."""
+    index = getattr(device, 'index', None)
+    if index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(index)
 
 
 def check(status: int, name: str):

@@ -13,10 +13,13 @@ class Workspace:
         self.entries = {}
 
     def tensor(self, name, shape, device, dtype):
-        key = (name, tuple(shape), torch.device(device), dtype)
-        if key not in self.entries:
-            self.entries[key] = torch.empty(shape, device=device, dtype=dtype)
-        return self.entries[key]
+        # torch.Size is a tuple: equal shapes are equal keys in either form
+        key = (name, shape if isinstance(shape, tuple) else tuple(shape),
+               device if isinstance(device, torch.device) else torch.device(device), dtype)
+        buf = self.entries.get(key)
+        if buf is None:
+            buf = self.entries[key] = torch.empty(shape, device=device, dtype=dtype)
+        return buf
 
     def bytes(self):
         return sum(x.numel() * x.element_size() for x in self.entries.values())

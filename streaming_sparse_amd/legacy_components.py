@@ -17,7 +17,9 @@ from .ops import Summary
 HEAD_DIM = 128
 
 
-_SUMMARY_INNER = (('keys', (4, HEAD_DIM)), ('mean', (HEAD_DIM,)), ('detail', (3, 8)), ('stats', (4, 12)))
+# field, inner shape, elements of a page, inner strides
+_SUMMARY_INNER = (('keys', (4, HEAD_DIM), 4 * HEAD_DIM, (HEAD_DIM, 1)), ('mean', (HEAD_DIM,), HEAD_DIM, (1,)),
+                  ('detail', (3, 8), 24, (8, 1)), ('stats', (4, 12), 48, (12, 1)))
 
 
 def _check_summary(s: Summary, h: int, p: int):
@@ -25,18 +27,14 @@ def _check_summary(s: Summary, h: int, p: int):
     is a bf16 [H, >=p, ...] page slice of a contiguous [H, Pcap, ...] slab
     (shape and stride arithmetic only: no tensor views are built)."""
     hp = s.head_pages
-    for name, inner in _SUMMARY_INNER:
+    for name, inner, n, strides in _SUMMARY_INNER:
         t = getattr(s, name)
-        if t.dtype != torch.bfloat16:
+        if t.dtype is not torch.bfloat16:
             raise TypeError(f"summary.{name} must be bf16")
-        shape, stride = t.shape, t.stride()
+        shape = t.shape
         if shape[0] != h or shape[1] < p:
             raise ValueError(f"summary.{name} shape {tuple(shape)} does not cover {h} heads x {p} pages")
-        want = [1] * len(inner)
-        for i in range(len(inner) - 2, -1, -1):
-            want[i] = want[i + 1] * inner[i + 1]
-        n = want[0] * inner[0]
-        if tuple(shape[2:]) != inner or list(stride[2:]) != want or stride[1] != n or stride[0] != hp * n:
+        if shape[2:] != inner or t.stride() != (hp * n, n) + strides:
             raise ValueError(f"summary.{name} must be a page slice of a contiguous [H,{hp},...] slab")
     return hp
 
@@ -91,7 +89,6 @@ the tail's _av at tuned_attention.py:16-18); True runs one bf16 product."""
 _WORKSPACE_BYTES = {}
 
 
-@torch.no_grad()
 def split_workspace(workspace, n_tokens, heads, pages, count, flags, device):
     """The attention call's workspace from `workspace`, or None when the call
     needs none: the tiles past the last multiple of the device's CU count

@@ -80,7 +80,6 @@ def _summary_ok(s: Summary):
     return hp
 
 
-@torch.no_grad()
 def encode(summary: Summary, basis: torch.Tensor, reader: Reader, out: Encoding | None = None,
            first: int = 0, pages: int | None = None) -> Encoding:
     """Encode pages [first, first + pages) of `summary` (a slab or a prefix
@@ -139,7 +138,6 @@ def encode_layers(summaries, bases, reader: Reader, outs, first: int, pages: int
     return outs
 
 
-@torch.no_grad()
 def correct(q, summary: Summary, encoding: Encoding, reader: Reader, risk, lse, mask, ids, own, heads,
             workspace=None, want_scores=False, no_alloc=False, probe_layout=None):
     """Full_Pset correction of the scoped `heads` in place on `mask` (uint8 or

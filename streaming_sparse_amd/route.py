@@ -46,7 +46,6 @@ def tier_count(tier: str, pages: int, n: int | None = None) -> int:
     raise ValueError(tier)
 
 
-@torch.no_grad()
 def route(q, summary, theta, *, tier='base', own=None, current_slots=None, n=None, workspace=None,
           want_mask=True, full_pset=None, encoding=None, reader=None, lse_out=None, rep_out=None, ties=None,
           tie_eps=1e-3):

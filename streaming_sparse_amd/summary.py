@@ -54,7 +54,6 @@ def _check_cache(k, v, first: int, pages: int):
     return h
 
 
-@torch.no_grad()
 def build(k, v, basis, init, out: Summary, first: int, pages: int, iters: int = 4, src=None) -> Summary:
     """k, v [1, 64P, H, 128] bf16 cache; basis [H,128,8]; init [H, pages, 4]
     initial k-means tokens (0..63) per page; out: a summary slab (or prefix
