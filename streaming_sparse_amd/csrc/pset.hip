@@ -41,7 +41,9 @@ constexpr int kProjPages = 32;      // pages of one head per projection workgrou
 constexpr int kCoefStride = 128;    // bf16 per page: co[85] | 0 x 11 | A[32]
 constexpr int kCoefA = 96;
 constexpr int kCand = 48;           // 16 removes + 32 adds
-constexpr int kCandVals = 34;       // lm, beta, approx[16], rp[16]
+constexpr int kCandVals = 34;       // doubles per probe and candidate in the caller's scratch
+constexpr int kCandStride = 26;     // doubles of a candidate: lm, beta (fp32), approx[16], rp[16] (fp32)
+constexpr int kRowDoubles = 16 * kCand * kCandVals;   // a row's scratch: its 16 x 48 candidates, then its partials
 constexpr int kPoolInts = 64;       // 48 candidate pages + 16 legal bit rows
 
 // ------------------------------------------------------------- encoding ----
@@ -349,8 +351,13 @@ __device__ __forceinline__ int own_page(const PsetParams& p, int h, int t) {
   return min(max(p.own ? p.own[(long long)h * p.T + t] : p.P - p.T + t, 0), p.P - 1);
 }
 
+template <int O>
+__device__ __forceinline__ unsigned long long xor_u64(unsigned long long v) {
+  const uint32_t lo = xor_lane<O>((uint32_t)v), hi = xor_lane<O>((uint32_t)(v >> 32));
+  return ((unsigned long long)hi << 32) | lo;
+}
+
 struct PoolSmem {
-  float risk[kMaxPages];
   uint8_t sel[kMaxPages];
   uint8_t isadd[kMaxPages];
   unsigned long long key[kMaxPages];
@@ -367,8 +374,9 @@ struct PoolSmem {
 // remove group and one add group: up to 8 movable removes, then the anchor
 // pages other than own; the unselected pages by descending risk, then the
 // selected pages in page order; the movable removes x the first 16 add
-// slots are legal.
-__global__ __launch_bounds__(256) void pset_pool_kernel(PsetParams p) {
+// slots are legal.  One key per thread; 3 heads x 72 blocks, kernel trace:
+// 9.5 us (two keys per thread, every step through LDS) -> 7.8 us.
+__global__ __launch_bounds__(kMaxPages) void pset_pool_kernel(PsetParams p) {
   __shared__ PoolSmem s;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int hs = blockIdx.x / p.T, t = blockIdx.x % p.T;
@@ -377,52 +385,63 @@ __global__ __launch_bounds__(256) void pset_pool_kernel(PsetParams p) {
   const long long rowoff = ((long long)h * p.T + t) * P;
   const int own = own_page(p, h, t);
   if (blockIdx.x == 0 && tid < 3) p.stats[tid] = tid == 1 ? (long long)p.HS * p.T : 0ll;
-  for (int i = tid; i < kMaxPages; i += 256) {
-    s.risk[i] = i < P ? p.risk[rowoff + i] : 0.f;
-    s.sel[i] = i < P ? (p.mask[rowoff + i] ? 1 : 0) : 1;
-    s.isadd[i] = 0;
-  }
+  const float risk = tid < P ? p.risk[rowoff + tid] : 0.f;
+  const bool sel = tid < P ? p.mask[rowoff + tid] != 0 : true;
+  s.sel[tid] = sel;
+  s.isadd[tid] = 0;
   if (tid < 4) s.cnt[tid] = 0;
   __syncthreads();
   const bool first = P == kCurrent;
-  for (int pg = tid; pg < kMaxPages; pg += 256) {
-    unsigned long long key = 0ull;
-    // a 72-page window counts every page in the history groups (4: removes,
-    // 2: adds), so its removes and adds each form one contiguous run; its
-    // adds range over all pages (an anchor page is selected in every mask
-    // the router writes)
-    if ((pg >= kAnchors || first) && pg < P) {
-      const int cur = first ? 0 : pg >= P - kCurrent;
-      const uint32_t ord = orderable(s.risk[pg]);
-      int group = 0;
-      uint32_t kv = 0;
-      if (s.sel[pg] && pg != own && pg >= kAnchors) {
-        group = cur ? 3 : 4;
-        kv = ~ord;
-      } else if (!s.sel[pg]) {
-        group = cur ? 1 : 2;
-        kv = ord;
-      }
-      if (group) {
-        key = ((unsigned long long)group << 60) | ((unsigned long long)kv << 20) | (unsigned long long)(1023 - pg);
-        atomicAdd(&s.cnt[4 - group], 1);
-      }
+  const int pg = tid;
+  unsigned long long key = 0ull;
+  int group = 0;
+  // a 72-page window counts every page in the history groups (4: removes,
+  // 2: adds), so its removes and adds each form one contiguous run; its
+  // adds range over all pages (an anchor page is selected in every mask
+  // the router writes)
+  if ((pg >= kAnchors || first) && pg < P) {
+    const int cur = first ? 0 : pg >= P - kCurrent;
+    const uint32_t ord = orderable(risk);
+    uint32_t kv = 0;
+    if (sel && pg != own && pg >= kAnchors) {
+      group = cur ? 3 : 4;
+      kv = ~ord;
+    } else if (!sel) {
+      group = cur ? 1 : 2;
+      kv = ord;
     }
-    s.key[pg] = key;
+    if (group) key = ((unsigned long long)group << 60) | ((unsigned long long)kv << 20) | (unsigned long long)(1023 - pg);
   }
-  __syncthreads();
+#pragma unroll
+  for (int g = 1; g <= 4; ++g) {
+    const int n = __popcll(__ballot(group == g));
+    if (lane == 0 && n) atomicAdd(&s.cnt[4 - g], n);
+  }
+  // descending bitonic sort, one key per thread: partner distances up to 32
+  // by lane exchanges, 64 to 256 through LDS
+  auto exchange = [&](int j, int k, unsigned long long other) {
+    const bool keep_max = ((tid & j) == 0) == ((tid & k) == 0);
+    if ((other > key) == keep_max) key = other;
+  };
+#pragma unroll 1
   for (int k = 2; k <= kMaxPages; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      const int lo = 2 * tid - (tid & (j - 1)), hi = lo + j;
-      const bool desc = (lo & k) == 0;
-      const unsigned long long a = s.key[lo], c = s.key[hi];
-      if ((a < c) == desc) {
-        s.key[lo] = c;
-        s.key[hi] = a;
-      }
+#pragma unroll 1
+    for (int j = k >> 1; j >= 64; j >>= 1) {
+      s.key[tid] = key;
       __syncthreads();
+      const unsigned long long other = s.key[tid ^ j];
+      __syncthreads();
+      exchange(j, k, other);
     }
+    if (k >= 64) exchange(32, k, xor_u64<32>(key));
+    if (k >= 32) exchange(16, k, xor_u64<16>(key));
+    if (k >= 16) exchange(8, k, xor_u64<8>(key));
+    if (k >= 8) exchange(4, k, xor_u64<4>(key));
+    if (k >= 4) exchange(2, k, xor_u64<2>(key));
+    exchange(1, k, xor_u64<1>(key));
   }
+  s.key[tid] = key;
+  __syncthreads();
   const int nmh = s.cnt[0], nmc = s.cnt[1], nuh = s.cnt[2], nuc = s.cnt[3];
   auto page_at = [&](int i) -> int { return 1023 - (int)(s.key[i] & 1023ull); };
   if (first) {
@@ -494,9 +513,9 @@ __global__ __launch_bounds__(256) void pset_pool_kernel(PsetParams p) {
         // -inf), zero values -- that adds nothing to any sum, while every
         // page outside the pool stays in the background.  The rows kernel
         // writes no endpoint data for it (no page maps to the slot).
-        double* c = p.cand + ((((long long)hs * p.T + t) * 16) * kCand + sl) * kCandVals;
+        double* c = p.cand + ((long long)hs * p.T + t) * kRowDoubles + sl * kCandStride;
         for (int m = 0; m < 16; ++m)
-          for (int v = 0; v < kCandVals; ++v) c[(long long)m * kCand * kCandVals + v] = v == 0 ? -INFINITY : 0.0;
+          for (int v = 0; v < kCandStride; ++v) c[(long long)m * kCand * kCandStride + v] = v == 0 ? -INFINITY : 0.0;
       }
     }
     int32_t* po = p.pool + ((long long)hs * p.T + t) * kPoolInts;
@@ -512,39 +531,102 @@ __global__ __launch_bounds__(256) void pset_pool_kernel(PsetParams p) {
 
 // ----------------------------------------------------------------- rows ----
 
-constexpr int kSplit = 2;          // page ranges per (head, pair of blocks)
-constexpr int kRowPart = 52;       // accH[16], accT[16], accB[16], sH, sT, sB, max logs
+constexpr int kSplit = 4;          // page ranges per (head, 4 blocks)
+constexpr int kRowBlocks = 4;      // query blocks (64 probes) per workgroup
+constexpr int kRowWaves = 8;
+constexpr int kPartVals = 35;      // B[16], T[16], their masses sB and sT, max log mass
+constexpr int kPartAt = 16 * kCand * kCandStride;     // [kSplit][kPartVals][16 probes], in a row's scratch
+static_assert(kPartAt + kSplit * kPartVals * 16 <= kRowDoubles, "the partials fit behind the candidates");
+// the caller's row buffer (unused: the partials lie behind the candidates)
+constexpr int kRowsSplit = 2, kRowsVals = 52;
 
 struct RowsSmem {
-  uint8_t sel[2][kMaxPages];
-  int8_t slot[2][kMaxPages];       // remove slot (0..15) of a pool page, or -1
-  int8_t aslot[2][kMaxPages];      // add slot (16..47), or -1: a 72-page pool may list a page in both
-  float u[32][8];
-  float L[32];
-  alignas(16) float coef[4][8][128];     // per-wave staging of a tile's 8 pages (fp32)
-  alignas(16) double md[4][8][64];       // meanB[16] | detailB[48]
-  double part[4][32][kRowPart];
+  uint8_t sel[kRowBlocks][kMaxPages];
+  int8_t slot[kRowBlocks][kMaxPages];       // remove slot (0..15) of a pool page, or -1
+  int8_t aslot[kRowBlocks][kMaxPages];      // add slot (16..47), or -1: a 72-page pool may list a page in both
+  float u[64][9];
+  float L[64];
+  alignas(16) uint8_t q[64 * 256];          // probe rows, chunk c of row r at chunk c ^ (r & 15)
+  double part[4][kPartVals][64];
 };
 
-// One workgroup per (scoped head, pair of blocks, page range): per probe
-// and page, the log mass lm = LSE_r z - LSE z, the readout (rp, beta), the
-// summary approximation, then partial mixture sums; candidate pages write
-// their endpoint data.
-__global__ __launch_bounds__(256) void pset_rows_kernel(PsetParams p) {
-  __shared__ RowsSmem s;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int NP = (p.T + 1) >> 1;
-  const int sp = blockIdx.x % kSplit;
-  const int pair_id = (blockIdx.x / kSplit) % NP;
-  const int hs = blockIdx.x / (kSplit * NP);
-  const int t0 = 2 * pair_id;
-  const int h = p.heads[hs];
-  const int P = p.P;
-  const int nrow = min(2, p.T - t0);
-  const int ntiles = (P + 7) >> 3;
-  const int tile0 = sp * ntiles / kSplit, tile1 = (sp + 1) * ntiles / kSplit;
+// 1 / x by the hardware reciprocal (1 ulp) and one Newton step.
+__device__ __forceinline__ float recip(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return fmaf(fmaf(-x, r, 1.0f), r, r);
+}
 
-  for (int i = tid; i < 2 * P; i += 256) {
+// tanh to within 1.6 ulp: below 0.625 an odd polynomial (a weighted
+// least-squares fit of (tanh x / x - 1) / x^2, 7e-9 relative), above it
+// 1 - 2 / (e^2x + 1).
+__device__ __forceinline__ float tanh_f32(float x) {
+  const float a = fabsf(x), t = x * x;
+  const float pl = fmaf(fmaf(fmaf(fmaf(-0.005515433382242918f, t, 0.020469674840569496f), t, -0.05368810519576073f), t,
+                             0.1333083212375641f), t, -0.3333325982093811f);
+  const float e = __builtin_amdgcn_exp2f(a * (2.0f * kLog2e));
+  const float big = fmaf(-2.0f, __builtin_amdgcn_rcpf(e + 1.0f), 1.0f);
+  return a < 0.625f ? fmaf(pl * t, x, x) : copysignf(big, x);
+}
+
+// A wave-uniform read-only value through the scalar cache.
+template <typename T>
+using Const = const __attribute__((address_space(4))) T;
+template <typename T>
+__device__ __forceinline__ Const<T>* scalar(const T* p) {
+  return (Const<T>*)(uintptr_t)p;
+}
+
+// One workgroup per (scoped head, 4 query blocks, page range): a lane holds
+// one of the 64 probes and a wave walks the pages of its tiles one at a time,
+// so everything that belongs to the page (meanB, detailB, the readout
+// coefficients) is wave-uniform and comes through the scalar cache into
+// scalar operands.  Per probe and page: the log mass lm = LSE_r z - LSE z,
+// the readout (rp, beta) and the summary approximation; candidate pages write
+// their endpoint data, the background pages (in no pool slot) enter the
+// mixture sums B (the current selection's weights) and T (every page exact),
+// which the scores kernel completes with the candidates.  Bound by vector
+// issue: ~440 fp32 and fp64 instructions per page and 64 probes, the fp64 ones
+// at half rate (with the page data always in the scalar cache the kernel is
+// 12% faster).  432 pages, 3 heads x 72 blocks, kernel trace: 94 us (32 probes
+// per wave, page data broadcast from LDS, three accumulated mixtures, 369
+// registers at one wave per SIMD) -> 54 us; the trace runs below the load
+// clock.
+__global__ __launch_bounds__(64 * kRowWaves, 2) void pset_rows_kernel(PsetParams p) {
+  __shared__ RowsSmem s;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int NG = (p.T + kRowBlocks - 1) / kRowBlocks;
+  const int sp = blockIdx.x % kSplit;
+  const int hs = blockIdx.x / (kSplit * NG), t0 = (blockIdx.x / kSplit % NG) * kRowBlocks;
+  const int h = __builtin_amdgcn_readfirstlane(p.heads[hs]);
+  const int P = p.P;
+  const int nrow = min(kRowBlocks, p.T - t0);
+
+  // this range's page data towards the L2 (768 bytes per page): the scalar
+  // loads of the page steps wait for each other, so none of them should be
+  // the first to miss.  The requests are dropped once the setup is done.
+  constexpr int kWaves = kSplit * kRowWaves, kWarm = (kMaxPages / kWaves + 7) / 8;
+  const int share = sp * kRowWaves + wave;
+  const int page0 = share * P / kWaves, page1 = (share + 1) * P / kWaves;
+  u32x4 warm[kWarm][3];
+#pragma unroll
+  for (int i = 0; i < kWarm; ++i) {
+    const int page = min(page0 + 8 * i + (lane >> 3), P - 1), c = lane & 7;
+    const long long pe = (long long)h * p.EP + page;
+    warm[i][0] = ldg16(p.coef + pe * kCoefStride + 16 * c);
+    warm[i][1] = *reinterpret_cast<const u32x4*>(p.mean_b + pe * 16 + 2 * c);
+    warm[i][2] = *reinterpret_cast<const u32x4*>(p.detail_b + pe * 48 + 6 * c);
+  }
+  // probe rows into LDS: row r = block r / 16, probe r % 16
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = (tid >> 4) + 32 * i, c = tid & 15;
+    const int tb = min(t0 + (r >> 4), p.T - 1);
+    const long long rr = p.gathered ? (r & 15) : probe_row(r & 15);
+    const uint16_t* qq = p.q + (long long)h * p.q_head + (long long)tb * p.q_block + rr * p.q_row;
+    *reinterpret_cast<u32x4*>(&s.q[r * 256 + ((c ^ (r & 15)) << 4)]) = ldg16(qq + 8 * c);
+  }
+  for (int i = tid; i < kRowBlocks * P; i += 64 * kRowWaves) {
     const int b = i / P, pg = i % P;
     const int tb = min(t0 + b, p.T - 1);
     s.sel[b][pg] = p.mask[((long long)h * p.T + tb) * P + pg] ? 1 : 0;
@@ -552,7 +634,7 @@ __global__ __launch_bounds__(256) void pset_rows_kernel(PsetParams p) {
     s.aslot[b][pg] = -1;
   }
   __syncthreads();
-  if (tid < 2 * kCand) {
+  if (tid < kRowBlocks * kCand) {
     const int b = tid / kCand, sl = tid % kCand;
     const int tb = min(t0 + b, p.T - 1);
     const int page = p.pool[((long long)hs * p.T + tb) * kPoolInts + sl];
@@ -561,226 +643,214 @@ __global__ __launch_bounds__(256) void pset_rows_kernel(PsetParams p) {
   // reader query u = Wq . probe (fp32) and the probe LSE from the router
   {
     const int pr = tid >> 3, i = tid & 7;
-    const int tb = min(t0 + (pr >> 4), p.T - 1);
-    const long long rr = p.gathered ? (pr & 15) : probe_row(pr & 15);
-    const uint16_t* qq = p.q + (long long)h * p.q_head + (long long)tb * p.q_block + rr * p.q_row;
     const f32x4* wr = reinterpret_cast<const f32x4*>(p.wq + i * 128);
-    u32x4 qv[16];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) qv[c] = ldg16(qq + 8 * c);
     float acc = 0.f;
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
+      const u32x4 qv = *reinterpret_cast<const u32x4*>(&s.q[pr * 256 + ((c ^ (pr & 15)) << 4)]);
       const f32x4 w0 = wr[2 * c], w1 = wr[2 * c + 1];
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        acc = fmaf(bf16_lo(qv[c][k]), w0[2 * k], acc);
-        acc = fmaf(bf16_hi(qv[c][k]), w0[2 * k + 1], acc);
-        acc = fmaf(bf16_lo(qv[c][2 + k]), w1[2 * k], acc);
-        acc = fmaf(bf16_hi(qv[c][2 + k]), w1[2 * k + 1], acc);
+        acc = fmaf(bf16_lo(qv[k]), w0[2 * k], acc);
+        acc = fmaf(bf16_hi(qv[k]), w0[2 * k + 1], acc);
+        acc = fmaf(bf16_lo(qv[2 + k]), w1[2 * k], acc);
+        acc = fmaf(bf16_hi(qv[2 + k]), w1[2 * k + 1], acc);
       }
     }
     s.u[pr][i] = acc;
-    if (i == 0) s.L[pr] = p.lse[((long long)h * p.T + tb) * 16 + (pr & 15)];
+    if (i == 0) s.L[pr] = p.lse[((long long)h * p.T + min(t0 + (pr >> 4), p.T - 1)) * 16 + (pr & 15)];
   }
-  const int pi = lane & 31, hh = lane >> 5;
-  const int blk = pi >> 4, m = pi & 15;
-  const int tq = min(t0 + blk, p.T - 1);
-  const long long row = p.gathered ? m : probe_row(m);
-  const uint16_t* qbase = p.q + (long long)h * p.q_head + (long long)tq * p.q_block + row * p.q_row;
-  u32x4 qop[8];
-#pragma unroll
-  for (int st = 0; st < 8; ++st) qop[st] = ldg16(qbase + 64 * hh + 8 * st);
   __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kWarm; ++i) asm volatile("" ::"v"(warm[i][0]), "v"(warm[i][1]), "v"(warm[i][2]));
+  const int blk = lane >> 4, m = lane & 15;
   float u[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) u[i] = s.u[pi][i];
-  const double L = (double)s.L[pi];
+  for (int i = 0; i < 8; ++i) u[i] = s.u[lane][i];
+  const double L = (double)s.L[lane];
   const uint16_t* rkh = p.rk + (long long)h * p.HP * 4 * kHeadDim;
   const float c2 = kLog2e / sqrtf((float)kHeadDim);    // logits in log2 units
   constexpr float kLn2 = 0.69314718055994531f;
+  double* const row = p.cand + ((long long)hs * p.T + min(t0 + blk, p.T - 1)) * kRowDoubles;
+  double* const mine = row + m * (kCand * kCandStride);
+  const bool live = blk < nrow;
 
-  double accH[16], accT[16], accB[16];
+  double accT[16], accB[16];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) accH[e] = accT[e] = accB[e] = 0.0;
-  double sH = 0.0, sT = 0.0, sB = 0.0, lmax = -INFINITY;
-  const long long row_id = ((long long)hs * p.T + tq) * 16 + m;
-  float* cw = &s.coef[wave][0][0];
-  double* mw = &s.md[wave][0][0];
-  // A tile's inputs (the 8 pages' coefficients and meanB | detailB, and its
-  // 32 rep keys) are loaded into registers one tile ahead: the loads of the
-  // wave's next tile are in flight while this tile's pages are computed.
-  u32x4 fa, fb, fm[4], fk[8];
-  auto fetch = [&](int tile) {
-    const int pl = lane >> 3, c = lane & 7;
-    const int page = min(tile * 8 + pl, P - 1);
-    const uint16_t* cf = p.coef + ((long long)h * p.EP + page) * kCoefStride + 16 * c;
-    const double* src = c < 2 ? p.mean_b + ((long long)h * p.EP + page) * 16 + 8 * c
-                               : p.detail_b + ((long long)h * p.EP + page) * 48 + 8 * (c - 2);
-    fa = ldg16(cf);
-    fb = ldg16(cf + 8);
-    const u32x4* s4 = reinterpret_cast<const u32x4*>(src);
+  for (int e = 0; e < 16; ++e) accT[e] = accB[e] = 0.0;
+  double sT = 0.0, sB = 0.0, lmax = -INFINITY;
+
+  // one page, its 4 rep logits of this lane's probe in z
+  auto page_step = [&](int page, const float (&zr)[4]) {
+    const long long pe = (long long)h * p.EP + page;
+    Const<uint32_t>* cw = scalar(reinterpret_cast<const uint32_t*>(p.coef + pe * kCoefStride));
+    Const<double>* mb = scalar(p.mean_b + pe * 16);
+    Const<double>* db = scalar(p.detail_b + pe * 48);
+    auto coef = [&](int i) { return i & 1 ? bf16_hi(cw[i >> 1]) : bf16_lo(cw[i >> 1]); };
+    // rep softmax of the page (fp32), page log mass in fp64
+    float z[4], w[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) fm[k] = s4[k];
-    const int row = min(tile * 32 + (lane & 31), P * 4 - 1);
-    const uint16_t* a = rkh + (long long)row * kHeadDim + 64 * hh;
+    for (int r = 0; r < 4; ++r) z[r] = zr[r] * c2;
+    const float zm = fmaxf(fmaxf(z[0], z[1]), fmaxf(z[2], z[3]));
+    float sw = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      w[r] = __builtin_amdgcn_exp2f(z[r] - zm);
+      sw += w[r];
+    }
+    const double lm = (double)((zm + __log2f(sw)) * kLn2) - L;
+    const float isw = recip(sw);       // sw is in [1, 4]
+    const double d0 = (w[0] + w[1] - w[2] - w[3]) * isw;
+    const double d1 = (w[0] - w[1] + w[2] - w[3]) * isw;
+    const double d2 = (w[0] - w[1] - w[2] + w[3]) * isw;
+    // readout: F_j = tanh(u . A_j), val = co_0 + sum_j F_j co_{j+1}
+    float F[4];
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      float acc = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc = fmaf(u[i], coef(kCoefA + 4 * i + jj), acc);
+      F[jj] = tanh_f32(acc);
+    }
+    float val[17];
+#pragma unroll
+    for (int k = 0; k < 17; ++k) {
+      float acc = 0.f;
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) acc = fmaf(F[jj], coef((jj + 1) * 17 + k), acc);
+      val[k] = coef(k) + acc;
+    }
+    const double le = lm + (double)val[16];
+    const bool sel = s.sel[blk][page];
+    const int sl = s.slot[blk][page], sa = s.aslot[blk][page];
+    const bool cand = sl >= 0 || sa >= 0;
+    const double lg = sel ? le : lm;
+    lmax = fmax(lmax, lg);
+    // a candidate's share of the sums is the scores kernel's
+    const double ex = cand ? 0.0 : (double)__builtin_amdgcn_exp2f((float)lg * kLog2e);
+    const double et = cand ? 0.0 : (double)__builtin_amdgcn_exp2f((float)le * kLog2e);
+    sB += ex;
+    sT += et;
+    double ap[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      ap[e] = mb[e] + (d0 * db[e] + d1 * db[16 + e] + d2 * db[32 + e]);
+      const double v = ap[e] + (double)val[e];
+      accB[e] += ex * (sel ? v : ap[e]);
+      accT[e] += et * v;
+    }
+    if (__any(cand && live)) {
+#pragma unroll 1
+      for (int k = 0; k < 2; ++k) {
+        const int at = k == 0 ? sl : sa;
+        if (at < 0 || !live) continue;
+        double* d = mine + at * kCandStride;
+        union { double v[2]; u32x4 w; } t;
+        t.v[0] = lm;
+        t.w[2] = __float_as_uint(val[16]);
+        t.w[3] = 0u;
+        *reinterpret_cast<u32x4*>(d) = t.w;
+#pragma unroll
+        for (int e = 0; e < 16; e += 2) {
+          t.v[0] = ap[e];
+          t.v[1] = ap[e + 1];
+          *reinterpret_cast<u32x4*>(d + 2 + e) = t.w;
+        }
+#pragma unroll
+        for (int e = 0; e < 16; e += 4)
+          *reinterpret_cast<f32x4*>(d + 18 + e / 2) = f32x4{val[e], val[e + 1], val[e + 2], val[e + 3]};
+      }
+    }
+  };
+
+  // the pages of this wave: an even share of the window, in tiles of 8 pages
+  // from its first one
+  const int pr = lane & 31, hh = lane >> 5;
+  u32x4 fk[8];
+  auto fetch = [&](int page) {
+    const uint16_t* a = rkh + (long long)min(page * 4 + pr, P * 4 - 1) * kHeadDim + 64 * hh;
 #pragma unroll
     for (int st = 0; st < 8; ++st) fk[st] = ldg16(a + 8 * st);
   };
-  if (tile0 + wave < tile1) fetch(tile0 + wave);
-  for (int tile = tile0 + wave; tile < tile1; tile += 4) {
-    // stage this tile's 8 pages: coefficients (bf16 -> fp32) and meanB | detailB
-    {
-      const int pl = lane >> 3, c = lane & 7;
-      float* d = cw + pl * 128 + 16 * c;
+  if (page0 < page1) fetch(page0);
+#pragma unroll 1
+  for (int tile = page0; tile < page1; tile += 8) {
+    // the tile's reps against probes 0..31 and 32..63
+    f32x16 sa = {}, sb = {};
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        d[2 * k] = bf16_lo(fa[k]);
-        d[2 * k + 1] = bf16_hi(fa[k]);
-        d[8 + 2 * k] = bf16_lo(fb[k]);
-        d[8 + 2 * k + 1] = bf16_hi(fb[k]);
-      }
-      u32x4* md = reinterpret_cast<u32x4*>(mw + pl * 64 + 8 * c);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) md[k] = fm[k];
+    for (int st = 0; st < 8; ++st) {
+      const int c = ((8 * hh + st) ^ (pr & 15)) << 4;
+      sa = mfma32(fk[st], *reinterpret_cast<const u32x4*>(&s.q[pr * 256 + c]), sa);
+      sb = mfma32(fk[st], *reinterpret_cast<const u32x4*>(&s.q[(32 + pr) * 256 + c]), sb);
     }
-    f32x16 S = {};
-#pragma unroll
-    for (int st = 0; st < 8; ++st) S = mfma32(fk[st], qop[st], S);
-    if (tile + 4 < tile1) fetch(tile + 4);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (tile + 8 < page1) fetch(tile + 8);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int pl = 2 * j + hh;
-      const int page = tile * 8 + pl;
-      if (page >= P) continue;
-      // rep softmax of the page (fp32), page log mass in fp64
-      float z[4], w[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) z[r] = S[4 * j + r] * c2;
-      const float zm = fmaxf(fmaxf(z[0], z[1]), fmaxf(z[2], z[3]));
-      float sw = 0.f;
+      // items 4 j .. 4 j + 3 hold page 2 j in lanes 0..31, page 2 j + 1 in
+      // lanes 32..63: the lane-half swap gives each page all 64 probes
+      float z0[4], z1[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        w[r] = __builtin_amdgcn_exp2f(z[r] - zm);
-        sw += w[r];
+        const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(sa[4 * j + r]), __float_as_uint(sb[4 * j + r]),
+                                                        false, false);
+        z0[r] = __uint_as_float(x[0]);
+        z1[r] = __uint_as_float(x[1]);
       }
-      const double lm = (double)((zm + __log2f(sw)) * kLn2) - L;
-      const float isw = 1.0f / sw;
-      const float c0 = (w[0] + w[1] - w[2] - w[3]) * isw;
-      const float c1 = (w[0] - w[1] + w[2] - w[3]) * isw;
-      const float cc2 = (w[0] - w[1] - w[2] + w[3]) * isw;
-      // readout: F_j = tanh(u . A_j), val = co_0 + sum_j F_j co_{j+1}
-      const float* cf = cw + pl * 128;
-      float F[4];
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        float acc = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc = fmaf(u[i], cf[kCoefA + 4 * i + jj], acc);
-        F[jj] = tanhf(acc);
-      }
-      float val[17];
-#pragma unroll
-      for (int k = 0; k < 17; ++k) {
-        float acc = 0.f;
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) acc = fmaf(F[jj], cf[(jj + 1) * 17 + k], acc);
-        val[k] = cf[k] + acc;
-      }
-      const double beta = (double)val[16];
-      const bool sel = s.sel[blk][page];
-      const int sl = s.slot[blk][page], sa = s.aslot[blk][page];
-      const bool bg = sl < 0 && sa < 0;      // a background page: in no pool slot
-      const double le = lm + beta;
-      const double lg = sel ? le : lm;
-      lmax = fmax(lmax, lg);
-      const double ex = (double)__builtin_amdgcn_exp2f((float)lg * kLog2e);
-      const double et = (double)__builtin_amdgcn_exp2f((float)le * kLog2e);
-      sH += ex;
-      sT += et;
-      if (bg) sB += ex;
-      const double* md = mw + pl * 64;
-      double* cd = (sl >= 0 && blk < nrow) ? p.cand + (row_id * kCand + sl) * kCandVals : nullptr;
-      double* ca = (sa >= 0 && blk < nrow) ? p.cand + (row_id * kCand + sa) * kCandVals : nullptr;
-      if (cd) {
-        cd[0] = lm;
-        cd[1] = beta;
-      }
-      if (ca) {
-        ca[0] = lm;
-        ca[1] = beta;
-      }
-      const double d0 = c0, d1 = c1, d2 = cc2;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const double ap = md[e] + (d0 * md[16 + e] + d1 * md[32 + e] + d2 * md[48 + e]);
-        const double rp = (double)val[e];
-        const double cur = sel ? ap + rp : ap;
-        accH[e] += ex * cur;
-        accT[e] += et * (ap + rp);
-        if (bg) accB[e] += ex * cur;
-        if (cd) {
-          cd[2 + e] = ap;
-          cd[18 + e] = rp;
-        }
-        if (ca) {
-          ca[2 + e] = ap;
-          ca[18 + e] = rp;
-        }
-      }
+      const int page = tile + 2 * j;
+      if (page < page1) page_step(page, z0);
+      if (page + 1 < page1) page_step(page + 1, z1);
     }
-    __builtin_amdgcn_wave_barrier();
   }
-  // reduce over the two page halves of a lane pair, then over waves
-#pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    accH[e] += __shfl_xor(accH[e], 32);
-    accT[e] += __shfl_xor(accT[e], 32);
-    accB[e] += __shfl_xor(accB[e], 32);
-  }
-  sH += __shfl_xor(sH, 32);
-  sT += __shfl_xor(sT, 32);
-  sB += __shfl_xor(sB, 32);
-  lmax = fmax(lmax, __shfl_xor(lmax, 32));
-  if (hh == 0) {
-    double* pw = s.part[wave][pi];
+  // sums over the workgroup's waves, by halves
+  auto vals = [&](auto f) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      pw[e] = accH[e];
-      pw[16 + e] = accT[e];
-      pw[32 + e] = accB[e];
+      f(e, accB[e]);
+      f(16 + e, accT[e]);
     }
-    pw[48] = sH;
-    pw[49] = sT;
-    pw[50] = sB;
-    pw[51] = lmax;
-  }
-  __syncthreads();
-  for (int i = tid; i < 32 * kRowPart; i += 256) {
-    const int pr = i / kRowPart, e = i % kRowPart;
-    if ((pr >> 4) >= nrow) continue;
-    double v = e == 51 ? -INFINITY : 0.0;
+    f(32, sB);
+    f(33, sT);
+  };
 #pragma unroll
-    for (int w = 0; w < 4; ++w) v = e == 51 ? fmax(v, s.part[w][pr][e]) : v + s.part[w][pr][e];
-    p.rows[((((long long)hs * p.T + t0 + (pr >> 4)) * 16 + (pr & 15)) * kSplit + sp) * kRowPart + e] = v;
+  for (int half = kRowWaves / 2; half > 0; half >>= 1) {
+    if (wave >= half && wave < 2 * half) {
+      double(*d)[64] = s.part[wave - half];
+      vals([&](int v, double& x) { d[v][lane] = x; });
+      d[34][lane] = lmax;
+    }
+    __syncthreads();
+    if (wave < half) {
+      double(*d)[64] = s.part[wave];
+      vals([&](int v, double& x) { x += d[v][lane]; });
+      lmax = fmax(lmax, d[34][lane]);
+    }
+    __syncthreads();
+  }
+  if (wave == 0 && live) {
+    double* d = row + kPartAt + sp * (kPartVals * 16) + m;
+    vals([&](int v, double& x) { d[16 * v] = x; });
+    d[16 * 34] = lmax;
   }
 }
 
 // --------------------------------------------------------------- scores ----
 
+constexpr int kPairs = 256;              // 16 removes x the 16 adds each may swap with
+constexpr int kScoreWaves = 8, kScoreThreads = 64 * kScoreWaves;
 struct ScoreSmem {
-  alignas(16) double cand[4][kCand][kCandVals];   // per wave: one probe's candidate endpoints
-  double V[4][16][kCand];                // endpoint vectors D(c - H) + e^(e-M) rp, [dim][candidate]
-  double S[4][kCand];                    // S_r (removes) / T_a (adds), shifted by the row max
-  double ex[4][kCand][2];                // e^(lm+beta-M), e^(lm-M) of each candidate
-  double Hs[4][48];                      // H[16] | E[16] | ob[16] of the probe
-  double sc[4][3];                       // B, shift M, unused
-  double acc[4][512];
-  alignas(16) double part[4][kSplit * kRowPart];   // the probe's split row partials
+  union {
+    alignas(16) double cand[kScoreWaves][kCand][kCandStride];   // per wave: one probe's candidate endpoints
+    double acc[kScoreWaves][kPairs];                            // its sums over probes, once they are done
+  } c;
+  double V[kScoreWaves][16][kCand];                // endpoint vectors D(c - H) + e^(e-M) rp, [dim][candidate]
+  double EV[kScoreWaves][kCand];                   // E . V of each candidate
+  double S[kScoreWaves][kCand];                    // S_r (removes) / T_a (adds), shifted by the row max
+  double ex[kScoreWaves][kCand][2];                // e^(lm+beta-M), e^(lm-M) of each candidate
+  double wt[kScoreWaves][kCand][2];                // its weight in H and in the target
+  double Hs[kScoreWaves][48];                      // H[16] | E[16] | ob[16] of the probe
+  double part[kScoreWaves][36];                    // the probe's background sums over the splits
   uint32_t legal[16];
+  uint8_t csel[kCand], cdup[kCand];      // candidate selected; an add page already listed as a remove
   int page[kMaxPages];                   // pool pages, then the compacted selection
   unsigned long long key[kMaxPages];     // LUT keys of the compacted selection
   float risk[kMaxPages];
@@ -789,143 +859,184 @@ struct ScoreSmem {
   int besti[4], bad[4];
 };
 
-// One workgroup per scoped (head, block); wave w takes probes w, w+4, ...
+// One workgroup per scoped (head, block); wave w takes probes w and w + 8
 // With every log mass shifted by the row max M, e^(-den) of a swap is
 // 1/(S_r + T_a) where S_r = B + sum_{k!=r} e^(er_k-M) + e^(lr_r-M) and
 // T_a = sum_{k!=a} e^(la_k-M) + e^(ea_a-M) (VR/scores.py:72-73), and each
 // endpoint delta of VR/scores.py:81-88 factors into e^(-den) times a
-// per-candidate vector, so delta(r,a) = (V_a - V_r) / (S_r + T_a).
-__global__ __launch_bounds__(256) void pset_scores_kernel(PsetParams p) {
+// per-candidate vector, so delta(r,a) = (V_a - V_r) / (S_r + T_a); a pair's
+// score then needs |V_a - V_r|^2 and the difference of the candidates' E . V.
+// Of the 16 x 32 pairs only those inside a partition can be legal (remove r
+// with adds 0..15 for r < 8, 16..31 otherwise; in a 72-page pool adds 0..15),
+// so a lane scores 4 pairs per probe, its sums in registers.  Bound by the
+// chain of dependent steps per probe, two probes per wave at two waves per
+// SIMD.  3 heads x 72 blocks, kernel trace: 48 us (all 512 pairs, three fp64
+// products per pair and dim, four probes per wave) -> 27 us.
+__global__ __launch_bounds__(kScoreThreads) void pset_scores_kernel(PsetParams p) {
   __shared__ ScoreSmem s;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int hs = blockIdx.x / p.T, t = blockIdx.x % p.T;
   const int h = p.heads[hs];
   const int P = p.P;
+  const bool first = P == kCurrent;
   const long long rowbase = (long long)hs * p.T + t;
+  const double* const row = p.cand + rowbase * kRowDoubles;
   const int32_t* po = p.pool + rowbase * kPoolInts;
-  if (tid < kCand) s.page[tid] = po[tid];
+  // A probe's candidates (48 x 26 doubles = 624 16-byte chunks) and split
+  // partials are loaded one probe ahead: the loads of probe m + 8 are in
+  // flight while probe m is scored.
+  constexpr int kChunks = kCand * kCandStride / 2, kLoads = (kChunks + 63) / 64;
+  u32x4 v[kLoads];
+  double pv[kSplit];
+  auto load_probe = [&](int m) {
+    const u32x4* cd = reinterpret_cast<const u32x4*>(row + m * (kCand * kCandStride));
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) v[k] = cd[min(lane + 64 * k, kChunks - 1)];
+#pragma unroll
+    for (int k = 0; k < kSplit; ++k) pv[k] = row[kPartAt + (k * kPartVals + min(lane, kPartVals - 1)) * 16 + m];
+  };
+  load_probe(w);
+  const int my_page = tid < kCand ? po[tid] : -1;
+  if (tid < kCand) s.page[tid] = my_page;
   if (tid < 16) s.legal[tid] = (uint32_t)po[kCand + tid];
-  for (int i = tid; i < P; i += 256) {
+  for (int i = tid; i < P; i += kScoreThreads) {
     const long long r = ((long long)h * p.T + t) * P + i;
     s.risk[i] = p.risk[r];
     s.sel[i] = p.mask[r] ? 1 : 0;
   }
-  for (int i = lane; i < 512; i += 64) s.acc[w][i] = 0.0;
-  // A probe's candidates (48 x 34 doubles = 816 16-byte chunks) and split row
-  // partials (kSplit x 52 doubles) are loaded one probe ahead: the loads of
-  // probe m + 4 are in flight while probe m is scored.
-  constexpr int kChunks = kSplit * kRowPart / 2;
-  constexpr int kRowLoads = (kChunks + 63) / 64;
-  u32x4 v[13], r[kRowLoads];
-  auto load_probe = [&](int m) {
-    const u32x4* cd = reinterpret_cast<const u32x4*>(p.cand + (rowbase * 16 + m) * kCand * kCandVals);
-#pragma unroll
-    for (int k = 0; k < 13; ++k) v[k] = cd[min(lane + 64 * k, 815)];
-    const u32x4* rs = reinterpret_cast<const u32x4*>(p.rows + (rowbase * 16 + m) * kSplit * kRowPart);
-#pragma unroll
-    for (int k = 0; k < kRowLoads; ++k) r[k] = rs[min(64 * k + lane, kChunks - 1)];
+  __syncthreads();
+  if (tid < kCand) {
+    // a 72-page pool may list an add page among its removes: counted once
+    bool dup = false;
+    if (tid >= 16)
+      for (int k = 0; k < 16; ++k) dup = dup || s.page[k] == my_page;
+    s.cdup[tid] = dup;
+    s.csel[tid] = my_page >= 0 && my_page < P && s.sel[my_page];
+  }
+  __syncthreads();
+  auto wave_fence = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
-  load_probe(w);
-  for (int m = w; m < 16; m += 4) {
-    // stage the probe's candidates and row state, then request the next probe's
+  // this lane's pairs: remove i, add j (slot 16 + j)
+  auto pair_of = [&](int pr, int& i, int& j) {
+    i = pr >> 4;
+    j = (pr & 15) + (!first && i >= 8 ? 16 : 0);
+  };
+  auto rp_of = [](const double* c, int e) { return (double)reinterpret_cast<const float*>(c + 18)[e]; };
+  double acc[kPairs / 64];
+#pragma unroll
+  for (int q = 0; q < kPairs / 64; ++q) acc[q] = 0.0;
+#pragma unroll 1
+  for (int m = w; m < 16; m += kScoreWaves) {
+    // stage the probe's candidates and background sums, then request the next probe's
     {
-      u32x4* dst = reinterpret_cast<u32x4*>(&s.cand[w][0][0]);
+      u32x4* dst = reinterpret_cast<u32x4*>(&s.c.cand[w][0][0]);
 #pragma unroll
-      for (int k = 0; k < 13; ++k) {
-        const int c = lane + 64 * k;
-        if (c < 816) dst[c] = v[k];
-      }
-      u32x4* pd = reinterpret_cast<u32x4*>(s.part[w]);
+      for (int k = 0; k < kLoads; ++k)
+        if (lane + 64 * k < kChunks) dst[lane + 64 * k] = v[k];
+      double x = pv[0];
 #pragma unroll
-      for (int k = 0; k < kRowLoads; ++k)
-        if (64 * k + lane < kChunks) pd[64 * k + lane] = r[k];
+      for (int k = 1; k < kSplit; ++k) x = lane == 34 ? fmax(x, pv[k]) : x + pv[k];
+      if (lane < kPartVals) s.part[w][lane] = x;
     }
-    if (m + 4 < 16) load_probe(m + 4);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (lane < 16) {
-      double aH = 0.0, aT = 0.0, aB = 0.0, zH = 0.0, zT = 0.0, zB = 0.0, lx = -INFINITY;
-#pragma unroll
-      for (int k = 0; k < kSplit; ++k) {
-        const double* r = s.part[w] + k * kRowPart;
-        aH += r[lane];
-        aT += r[16 + lane];
-        aB += r[32 + lane];
-        zH += r[48];
-        zT += r[49];
-        zB += r[50];
-        lx = fmax(lx, r[51]);
-      }
-      const double Hv = aH / zH;
-      s.Hs[w][lane] = Hv;
-      s.Hs[w][16 + lane] = aT / zT - Hv;
-      s.Hs[w][32 + lane] = aB / zB;
-      if (lane == 0) {
-        s.sc[w][0] = zB * exp(-lx);
-        s.sc[w][1] = lx;
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const double B = s.sc[w][0], M = s.sc[w][1];
-    // per candidate: endpoint vector and its share of the swap denominator
+    if (m + kScoreWaves < 16) load_probe(m + kScoreWaves);
+    wave_fence();
+    const double M = s.part[w][34], shift = exp(-M), B = s.part[w][32] * shift;
+    const double* c = s.c.cand[w][min(lane, kCand - 1)];
+    double EX = 0.0, LM = 0.0, D = 0.0;
     if (lane < kCand) {
-      const double* c = s.cand[w][lane];
-      const double lmk = c[0], bk = c[1];
-      const double EX = exp(lmk + bk - M), LM = exp(lmk - M);
-      const double D = fabs(bk) < 0.5 ? LM * expm1(fmin(fmax(bk, -0.5), 0.5)) : EX - LM;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) s.V[w][e][lane] = D * (c[2 + e] - s.Hs[w][e]) + EX * c[18 + e];
+      const double lmk = c[0], bk = (double)reinterpret_cast<const float*>(c + 1)[0];
+      EX = exp(lmk + bk - M);
+      LM = exp(lmk - M);
+      D = fabs(bk) < 0.5 ? LM * expm1(fmin(fmax(bk, -0.5), 0.5)) : EX - LM;
       s.ex[w][lane][0] = EX;
       s.ex[w][lane][1] = LM;
+      s.wt[w][lane][0] = s.cdup[lane] ? 0.0 : s.csel[lane] ? EX : LM;
+      s.wt[w][lane][1] = s.cdup[lane] ? 0.0 : EX;
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (lane < kCand) {
-      // leave-one-out sums over the other candidates of the same group
-      double loo = 0.0;
-      if (lane < 16) {
-        for (int k = 0; k < 16; ++k)
-          if (k != lane) loo += s.ex[w][k][0];
-        s.S[w][lane] = B + loo + s.ex[w][lane][1];
-      } else {
-        for (int k = 16; k < kCand; ++k)
-          if (k != lane) loo += s.ex[w][k][1];
-        s.S[w][lane] = loo + s.ex[w][lane][0];
+    wave_fence();
+    // H and the target: the background sums and the candidates (lane: dim
+    // l % 16, candidates 12 (l / 16) .. + 11)
+    {
+      const int e = lane & 15, g = lane >> 4;
+      double aH = 0.0, aT = 0.0, zH = 0.0, zT = 0.0;
+#pragma unroll
+      for (int k = 12 * g; k < 12 * g + 12; ++k) {
+        const double* ck = s.c.cand[w][k];
+        const double wh = s.wt[w][k][0], wx = s.wt[w][k][1], ap = ck[2 + e], full = ap + rp_of(ck, e);
+        aH = fma(wh, s.csel[k] ? full : ap, aH);
+        aT = fma(wx, full, aT);
+        zH += wh;
+        zT += wx;
+      }
+      aH += xor_lane<16>(aH);
+      aT += xor_lane<16>(aT);
+      zH += xor_lane<16>(zH);
+      zT += xor_lane<16>(zT);
+      aH += xor_lane<32>(aH);
+      aT += xor_lane<32>(aT);
+      zH += xor_lane<32>(zH);
+      zT += xor_lane<32>(zT);
+      const double bH = s.part[w][e], Hv = fma(bH, shift, aH) / (zH + B);
+      if (g == 0) {
+        s.Hs[w][e] = Hv;
+        s.Hs[w][16 + e] = fma(s.part[w][16 + e], shift, aT) / (fma(s.part[w][33], shift, zT)) - Hv;
+        s.Hs[w][32 + e] = bH / s.part[w][32];
       }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    uint32_t badmask = 0u;
-#pragma unroll 1
-    for (int q = 0; q < 8; ++q) {
-      const int pr = lane + 64 * q, i = pr >> 5, j = pr & 31;
-      const double den = s.S[w][i] + s.S[w][16 + j];
-      const double inv = 1.0 / den;
-      double ed = 0.0, dd = 0.0;
-      bool finite = isfinite(inv);
+    wave_fence();
+    // per candidate: endpoint vector, its E . V and its share of the swap
+    // denominator (leave-one-out sums over the other candidates of its group)
+    if (lane < kCand) {
+      double ev = 0.0;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const double d = (s.V[w][e][16 + j] - s.V[w][e][i]) * inv;
-        finite = finite && isfinite(d);
-        ed += s.Hs[w][16 + e] * d;
-        dd += d * d;
+        const double x = D * (c[2 + e] - s.Hs[w][e]) + EX * rp_of(c, e);
+        s.V[w][e][lane] = x;
+        ev = fma(s.Hs[w][16 + e], x, ev);
       }
+      s.EV[w][lane] = ev;
+      double loo = 0.0;
+      if (lane < 16) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) loo += k != lane ? s.ex[w][k][0] : 0.0;
+        s.S[w][lane] = B + loo + LM;
+      } else {
+#pragma unroll
+        for (int k = 16; k < kCand; ++k) loo += k != lane ? s.ex[w][k][1] : 0.0;
+        s.S[w][lane] = loo + EX;
+      }
+    }
+    wave_fence();
+    uint32_t badmask = 0u;
+#pragma unroll
+    for (int q = 0; q < kPairs / 64; ++q) {
+      int i, j;
+      pair_of(lane + 64 * q, i, j);
+      const double den = s.S[w][i] + s.S[w][16 + j];
+      const double inv = 1.0 / den;
+      double dd = 0.0;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const double d = s.V[w][e][16 + j] - s.V[w][e][i];
+        dd = fma(d, d, dd);
+      }
+      const double ed = (s.EV[w][16 + j] - s.EV[w][i]) * inv;
+      dd *= inv * inv;
       // the reference's "bad" branch: max logs - den > 80, or a non-finite delta
-      if (den < 1.8048513878454153e-35 || !finite) badmask |= 1u << q;
-      else s.acc[w][pr] += 2.0 * ed - dd;
+      if (den < 1.8048513878454153e-35 || !(isfinite(inv) && isfinite(ed) && isfinite(dd))) badmask |= 1u << q;
+      else acc[q] += 2.0 * ed - dd;
     }
     if (__any(badmask != 0u)) {
       // rare: the mixture after the swap rebuilt from the background and every
       // candidate (VR/scores.py:75-79), minus H
-#pragma unroll 1
-      for (int q = 0; q < 8; ++q) {
+#pragma unroll
+      for (int q = 0; q < kPairs / 64; ++q) {
         if (!((badmask >> q) & 1u)) continue;
-        const int pr = lane + 64 * q, i = pr >> 5, j = pr & 31;
+        int i, j;
+        pair_of(lane + 64 * q, i, j);
         const double den = s.S[w][i] + s.S[w][16 + j];
         double ed = 0.0, dd = 0.0;
 #pragma unroll 1
@@ -933,35 +1044,45 @@ __global__ __launch_bounds__(256) void pset_scores_kernel(PsetParams p) {
           double nw = B * s.Hs[w][32 + e];
 #pragma unroll 1
           for (int k = 0; k < kCand; ++k) {
-            const double* c = s.cand[w][k];
+            const double* ck = s.c.cand[w][k];
             const bool exact = k < 16 ? k != i : k == 16 + j;      // selected after the swap
-            nw += exact ? s.ex[w][k][0] * (c[2 + e] + c[18 + e]) : s.ex[w][k][1] * c[2 + e];
+            nw += exact ? s.ex[w][k][0] * (ck[2 + e] + rp_of(ck, e)) : s.ex[w][k][1] * ck[2 + e];
           }
           const double d = nw / den - s.Hs[w][e];
           ed += s.Hs[w][16 + e] * d;
           dd += d * d;
         }
-        s.acc[w][pr] += 2.0 * ed - dd;
+        acc[q] += 2.0 * ed - dd;
       }
     }
     __builtin_amdgcn_wave_barrier();
   }
+  __syncthreads();      // the candidates' space takes the sums
+#pragma unroll
+  for (int q = 0; q < kPairs / 64; ++q) s.c.acc[w][lane + 64 * q] = acc[q];
   __syncthreads();
   // legality, argmax (ties -> lowest pair index), finiteness
   double best = -INFINITY;
   int besti = 0x7fffffff;
   int bad = 0;
+  if (tid < kPairs) {
+    int i, j;
+    pair_of(tid, i, j);
+    const int flat = 32 * i + j;
+    double sc = 0.0;
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int flat = tid + 256 * q, i = flat >> 5, j = flat & 31;
-    double sc = (((s.acc[0][flat] + s.acc[1][flat]) + s.acc[2][flat]) + s.acc[3][flat]) / 16.0;
+    for (int k = 0; k < kScoreWaves; ++k) sc += s.c.acc[k][tid];
+    sc /= 16.0;
     if (!((s.legal[i] >> j) & 1u)) sc = -1e30;
     if (!isfinite(sc)) bad += 1;
-    else if (sc > best || (sc == best && flat < besti)) {
+    else {
       best = sc;
       besti = flat;
     }
-    if (p.scores) p.scores[rowbase * 512 + flat] = sc;
+    if (p.scores) {
+      p.scores[rowbase * 512 + flat] = sc;
+      p.scores[rowbase * 512 + (flat ^ 16)] = -1e30;     // across partitions: never legal
+    }
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
@@ -973,7 +1094,7 @@ __global__ __launch_bounds__(256) void pset_scores_kernel(PsetParams p) {
       besti = oi;
     }
   }
-  if (lane == 0) {
+  if (lane == 0 && w < kPairs / 64) {
     s.best[w] = best;
     s.besti[w] = besti;
     s.bad[w] = bad;
@@ -982,7 +1103,7 @@ __global__ __launch_bounds__(256) void pset_scores_kernel(PsetParams p) {
   best = s.best[0];
   besti = s.besti[0];
   bad = s.bad[0];
-  for (int k = 1; k < 4; ++k) {
+  for (int k = 1; k < kPairs / 64; ++k) {
     if (s.best[k] > best || (s.best[k] == best && s.besti[k] < besti)) {
       best = s.best[k];
       besti = s.besti[k];
@@ -1029,13 +1150,13 @@ __global__ __launch_bounds__(256) void pset_scores_kernel(PsetParams p) {
   const int nsel = s.besti[0];
   // key (orderable risk, 1023 - page): a higher key ranks first, ties go to
   // the lower page; a page's slot is the count of listed keys above its own
-  for (int i = tid; i < nsel; i += 256) {
+  for (int i = tid; i < nsel; i += kScoreThreads) {
     const int x = s.page[i];
     s.key[i] = ((unsigned long long)orderable(s.risk[x]) << 32) | (uint32_t)(1023 - x);
   }
   __syncthreads();
   if (tid == 0) ids[0] = own;
-  for (int i = tid; i < nsel; i += 256) {
+  for (int i = tid; i < nsel; i += kScoreThreads) {
     const unsigned long long kx = s.key[i];
     int rank = 0;
     for (int k = 0; k < nsel; ++k) rank += s.key[k] > kx;
@@ -1043,7 +1164,7 @@ __global__ __launch_bounds__(256) void pset_scores_kernel(PsetParams p) {
   }
   // a selection shorter than the table (quotas clamped to their partitions)
   // leaves -1 padding, as the router writes it
-  for (int i = 1 + nsel + tid; i < p.C; i += 256) ids[i] = -1;
+  for (int i = 1 + nsel + tid; i < p.C; i += kScoreThreads) ids[i] = -1;
 }
 
 // Both entry points: a non-null `layers` table runs `nlayers` layers in one
@@ -1179,10 +1300,10 @@ int pset_launch(const void* q, long long q_head_stride, long long q_block_stride
   p.T = blocks;
   p.P = pages;
   p.C = count;
-  const int np = (blocks + 1) / 2;
-  hipLaunchKernelGGL(pset_pool_kernel, dim3(n_heads * blocks), dim3(256), 0, stream, p);
-  hipLaunchKernelGGL(pset_rows_kernel, dim3(n_heads * np * kSplit), dim3(256), 0, stream, p);
-  hipLaunchKernelGGL(pset_scores_kernel, dim3(n_heads * blocks), dim3(256), 0, stream, p);
+  const int groups = (blocks + kRowBlocks - 1) / kRowBlocks;
+  hipLaunchKernelGGL(pset_pool_kernel, dim3(n_heads * blocks), dim3(kMaxPages), 0, stream, p);
+  hipLaunchKernelGGL(pset_rows_kernel, dim3(n_heads * groups * kSplit), dim3(64 * kRowWaves), 0, stream, p);
+  hipLaunchKernelGGL(pset_scores_kernel, dim3(n_heads * blocks), dim3(kScoreThreads), 0, stream, p);
   return (int)hipGetLastError();
 }
 
@@ -1195,7 +1316,7 @@ int pset_launch(const void* q, long long q_head_stride, long long q_block_stride
 // endpoint data and every row partial), so nothing in it must start at zero.
 constexpr int kScratchRows = 216;   // 3 heads x 72 query blocks
 constexpr size_t kCandRowBytes = (size_t)16 * kCand * kCandVals * sizeof(double);
-constexpr size_t kRowsRowBytes = (size_t)16 * kSplit * kRowPart * sizeof(double);
+constexpr size_t kRowsRowBytes = (size_t)16 * kRowsSplit * kRowsVals * sizeof(double);
 constexpr size_t kPoolRowBytes = (size_t)kPoolInts * sizeof(int32_t);
 constexpr size_t kScratchRowsOff = kScratchRows * kCandRowBytes;
 constexpr size_t kScratchPoolOff = kScratchRowsOff + kScratchRows * kRowsRowBytes;

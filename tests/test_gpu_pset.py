@@ -295,3 +295,46 @@ def test_pset_short_spares_matches_oracle(device):
     got_mask = mask.cpu()
     assert bool(((got_mask[hs] == want_mask[hs]).all(-1) | ties).all())
     assert (got_mask[..., P - 72:].sum(-1) == 66).all() and got_mask[..., :24].all()
+
+
+@pytest.mark.parametrize("blocks,pages", [(1, 113), (5, 117), (7, 130), (4, 216)])
+def test_pset_ragged_groups_match_oracle(device, blocks, pages):
+    """Query blocks that do not fill a workgroup's four (1, 5 and 7), windows
+    whose pages do not divide over the 32 waves of a group or into tiles of 8
+    (113 and 117 pages: 3 or 4 pages per wave; 130: 4 or 5), two scoped heads:
+    pools equal, scores within 1e-4 of the row scale, decisions and masks
+    equal off near ties."""
+    x, w, _, _ = inputs(9)
+    heads, scoped, n = 4, [0, 3], 30
+    s = type(x.summary)(*(getattr(x.summary, f)[:heads, :pages].contiguous() for f in x.summary.FIELDS))
+    q = x.q[:, -64 * blocks:, :heads].contiguous()
+    own = (torch.arange(blocks) + pages - blocks)[None].expand(heads, -1).contiguous()
+    gs = type(s)(*(getattr(s, f).to(device) for f in s.FIELDS))
+    reader = pset.Reader(w, device)
+    enc = pset.encode(gs, x.basis[:heads].to(device), reader)
+    # history quotas that leave the smallest windows history pages to swap
+    a = torch.full((heads,), 24, dtype=torch.int32)
+    lse = torch.empty(heads, blocks, 16, device=device)
+    ids, mask, risk, _ = route(q.to(device), gs, x.theta[:heads].to(device), tier='intersection', own=own.to(device),
+                               current_slots=a, n=n, lse_out=lse)
+    m0 = mask.clone().cpu()
+    stats, rows = pset.correct(q.to(device), gs, enc, reader, risk, lse, mask, ids, own.to(device), scoped,
+                               want_scores=True)
+    torch.cuda.synchronize()
+    pr = ref.probes(q)
+    z = ref.route_logits(pr, s.keys)
+    enc_o = dict(co=enc.co.cpu(), A=enc.A.cpu(), mean=enc.mean.cpu(), detail=enc.detail.cpu())
+    want_mask, orow, _ = opset.correct(pr.bfloat16().float(), z, risk.cpu(), m0, own, enc_o, w['wq'], scoped)
+    pool = rows['pool'].cpu()
+    assert torch.equal(pool[..., :16].long(), orow['remove'])
+    assert torch.equal(pool[..., 16:48].long(), orow['add'].masked_fill(orow['add'] == pages, -1))
+    legal = orow['legal'].reshape(len(scoped), blocks, 16, 32)
+    want_s = orow['scores']
+    scale = want_s.masked_fill(~legal, 0).abs().flatten(-2).amax(-1).clamp_min(1e-300)
+    err = ((rows['scores'].cpu() - want_s).abs().masked_fill(~legal, 0).flatten(-2).amax(-1) / scale)
+    print(f"{blocks} blocks, {pages} pages: scores max err / row scale {float(err.max()):.2e}", flush=True)
+    assert bool(legal.flatten(-2).any(-1).all()) and float(err.max()) < 1e-4 and int(stats[2]) == 0
+    ties = _near_tie(want_s, legal)
+    ex_g = rows['executed'].cpu().bool()
+    assert bool(((ex_g == orow['executed']) & (~ex_g | (rows['argmax'].cpu().long() == orow['argmax'])) | ties).all())
+    assert bool(((mask.cpu()[scoped] == want_mask[scoped]).all(-1) | ties).all())
