@@ -26,16 +26,16 @@
 //                    power step X^T (X d) is (X^T X) d: 32 x 32 per step
 //                    instead of a pass over the rows)
 //   keys_kernel, sort_kernel  grid (18, B), (B): level 0's projections, sort
-//   level_kernel     grid (3 B): level 1 (groups of 1536): Gram matrix,
-//                    direction, projections and sort; rows are read where
-//                    they lie, through the order of level 0
-//   fused_levels_kernel  grid (B x 9): levels 2..6 inside each 512-row group
+//   level_kernel     grid (3 B), (9 B): levels 1 and 2 (groups of 1536 and
+//                    512): Gram matrix, direction, projections and sort; rows
+//                    are read where they lie, through the previous order
+//   fused_levels_kernel  grid (B x 18): levels 3..6 inside each 256-row group
 //   frames_kernel    grid (B): the first chunk's stable partition by frame
 // 30 layers x 12 heads: 5.26 ms (a workgroup per row and seven passes over its
 // rows per level, sums over rows through serial LDS walks, bitonic sorts in
-// LDS) -> 2.04 ms: project 0.58, totals 0.01, features 0.24, level 0 0.24
-// (direction 0.014, keys 0.11, sort 0.11), level 1 0.19, fused levels 0.77.
-// One layer x 12 heads: 862 -> 242 us.
+// LDS) -> 1.92 ms: project 0.58, totals 0.01, features 0.24, level 0 0.24
+// (direction 0.014, keys 0.11, sort 0.11), level 1 0.20, level 2 0.17, fused
+// levels 0.48.  One layer x 12 heads: 862 -> 249 us.
 #include "common.h"
 
 #include <type_traits>
@@ -687,39 +687,41 @@ __global__ __launch_bounds__(576) void sort_kernel(GroupParams p) {
   rank_runs<kTokens / 512>(runs, wave, key, pos, lane, [&](int rank, uint32_t t) { o[rank] = (int32_t)t; });
 }
 
-// Level 1: each workgroup orders one group of 1536 rows of one b (the rows
-// ids[1][group] of x[0], read where they lie).  One pass for the group's Gram
-// matrix, about its middle row (near the mean along level 0's direction, so
-// the centring loses nothing), on the fp64 matrix pipe; one for the
-// projections; three waves sort runs of 512 and merge by rank.  Bound by
-// those two passes over the rows.
-constexpr int kMid = kTokens / 3;
-__global__ __launch_bounds__(512) void level_kernel(GroupParams p) {
+// Levels 1 and 2: each workgroup orders one group of N rows of one b (the
+// rows ids[src][group] of x[0], read where they lie).  One pass for the
+// group's Gram matrix, about its middle row (near the mean along the previous
+// level's direction, so the centring loses nothing), on the fp64 matrix pipe;
+// one for the projections; a wave sorts each run of 512, the runs merge by
+// rank.  Bound by those two passes over the rows.
+template <int N, int THREADS>
+__global__ __launch_bounds__(THREADS) void level_kernel(GroupParams p, int src) {
+  constexpr int kWaves = THREADS / 64, kHalf = kWaves / 2, kGroups = kTokens / N;
   __shared__ union {
-    double red[4][kGramAll];
-    unsigned long long runs[kMid / 512][512];
+    double red[kHalf][kGramAll];
+    unsigned long long runs[N / 512][512];
   } u;
-  __shared__ unsigned short tok[kMid];
+  __shared__ unsigned short tok[N];
   __shared__ double vec[kR], mean_s[kR], dir_s[kR];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int b = blockIdx.x / 3, gi = blockIdx.x % 3;
+  const int b = blockIdx.x / kGroups, gi = blockIdx.x % kGroups;
   const double* x = p.x[0] + (long long)b * kTokens * kR;
-  const long long row0 = (long long)b * kTokens + gi * kMid;
-  for (int i = tid; i < kMid; i += 512) tok[i] = (unsigned short)p.ids[1][row0 + i];
+  const long long row0 = (long long)b * kTokens + gi * N;
+  for (int i = tid; i < N; i += THREADS) tok[i] = (unsigned short)p.ids[src][row0 + i];
   __syncthreads();
   {
     const int c = lane & 15, g = lane >> 4;
-    const double* mid = x + (int)tok[kMid / 2] * kR;
+    const double* mid = x + (int)tok[N / 2] * kR;
     const double s0 = mid[c], s1 = mid[c + 16];
     Gram gram;
-    constexpr int kSteps = kMid / 8 / 4;     // four rows per step, 192 rows per wave
+    constexpr int kRows = N / kWaves, kSteps = kRows / 4;     // a wave's rows, four per step
+    static_assert(kSteps % 8 == 0, "eight steps at a time");
 #pragma unroll 1
     for (int i0 = 0; i0 < kSteps; i0 += 8) {
       double xl[8], xh[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const double* xr = x + (int)tok[192 * wave + 4 * (i0 + i) + g] * kR + c;
+        const double* xr = x + (int)tok[kRows * wave + 4 * (i0 + i) + g] * kR + c;
         xl[i] = xr[0];
         xh[i] = xr[16];
       }
@@ -727,16 +729,21 @@ __global__ __launch_bounds__(512) void level_kernel(GroupParams p) {
       for (int i = 0; i < 8; ++i) gram.add(xl[i] - s0, xh[i] - s1);
     }
     gram.fold();
-    if (wave >= 4) gram.store<false>(u.red[wave - 4], lane);
+    if (wave >= kHalf) gram.store<false>(u.red[wave - kHalf], lane);
     __syncthreads();
-    if (wave < 4) gram.store<true>(u.red[wave], lane);
+    if (wave < kHalf) gram.store<true>(u.red[wave], lane);
     __syncthreads();
-    for (int i = tid; i < kGramAll; i += 512) u.red[0][i] = (u.red[0][i] + u.red[1][i]) + (u.red[2][i] + u.red[3][i]);
+    for (int i = tid; i < kGramAll; i += THREADS) {
+      double v = u.red[0][i];
+#pragma unroll
+      for (int k = 1; k < kHalf; ++k) v += u.red[k][i];
+      u.red[0][i] = v;
+    }
     __syncthreads();
     if (wave == 0) {
-      const double d = power_direction(u.red[0], kMid, vec, lane);
+      const double d = power_direction(u.red[0], N, vec, lane);
       if (lane < kR) {
-        mean_s[lane] = mid[lane] + u.red[0][kGramDoubles + lane] / kMid;
+        mean_s[lane] = mid[lane] + u.red[0][kGramDoubles + lane] / N;
         dir_s[lane] = d;
       }
     }
@@ -750,25 +757,27 @@ __global__ __launch_bounds__(512) void level_kernel(GroupParams p) {
     dir[c] = dir_s[4 * q + c];
   }
   unsigned long long* keys = &u.runs[0][0];
+  constexpr int kSlots = THREADS / 8;      // rows at a time
+  static_assert(N / kSlots % 4 == 0, "four rows per thread at a time");
 #pragma unroll 1
-  for (int i0 = 0; i0 < kMid / 64; i0 += 4) {
+  for (int i0 = 0; i0 < N / kSlots; i0 += 4) {
     double xr[4][4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const double* xp = x + (int)tok[rs + 64 * (i0 + i)] * kR + 4 * q;
+      const double* xp = x + (int)tok[rs + kSlots * (i0 + i)] * kR + 4 * q;
 #pragma unroll
       for (int c = 0; c < 4; ++c) xr[i][c] = xp[c];
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const double pr = project_row(xr[i], mean, dir);
-      if (q == 0) keys[rs + 64 * (i0 + i)] = order_key(pr);
+      if (q == 0) keys[rs + kSlots * (i0 + i)] = order_key(pr);
     }
   }
   __syncthreads();
   unsigned long long key[8];
   uint32_t pos[8];
-  const bool sorts = wave < kMid / 512;
+  const bool sorts = wave < N / 512;
   if (sorts) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -781,13 +790,13 @@ __global__ __launch_bounds__(512) void level_kernel(GroupParams p) {
   }
   __syncthreads();
   if (!sorts) return;
-  int32_t* o = p.ids[0] + row0;
-  rank_runs<kMid / 512>(u.runs, wave, key, pos, lane, [&](int rank, uint32_t i) { o[rank] = (int32_t)tok[i]; });
+  int32_t* o = p.ids[src ^ 1] + row0;
+  rank_runs<N / 512>(u.runs, wave, key, pos, lane, [&](int rank, uint32_t i) { o[rank] = (int32_t)tok[i]; });
 }
 
-// Levels 2..6 of the balanced split in one workgroup per 512-row group (a
-// ninth of the chunk, as level 1 leaves it): the group's fp64 rows and token
-// ids stay in LDS; level l sorts every aligned block of n = 512 >> (l - 2)
+// Levels 3..6 of the balanced split in one workgroup per 256-row group (an
+// 18th of the chunk, as level 2 leaves it): the group's fp64 rows and token
+// ids stay in LDS; level l sorts every aligned block of n = 256 >> (l - 3)
 // rows by the block's own projection, all blocks at once, and a permutation
 // of row slots carries the order from level to level.  A level reads its rows
 // from LDS once: wave w holds rows 32 w .. 32 w + 31 of the order in
@@ -795,20 +804,22 @@ __global__ __launch_bounds__(512) void level_kernel(GroupParams p) {
 // .. 4 rg + 3, and the power steps, sums over rows by lane exchanges and,
 // where a block spans waves, one LDS round with one barrier each.  The sort
 // runs one element per thread, by lane exchanges up to distance 32.  The last
-// level writes the final order.  Bound by fp64 vector issue: per 30-layer
-// batch 0.77 ms, of which the power steps take about half and the sorts 0.2
-// (1.65 ms with every pass from LDS and its sums through a 64-deep serial LDS
-// walk).
-constexpr int kFuse = 512;
-constexpr int kFuseLevels = 5;
-constexpr int kFuseThreads = 1024;
+// level writes the final order.  Bound by fp64 vector issue, two workgroups
+// per CU: per 30-layer batch 0.48 ms, half of it power steps (with level 2 in
+// here too, 512 rows and one workgroup per CU: 0.77 ms against 0.48 + 0.17; at
+// the start 1.65 ms, with every pass from LDS and its sums through a 64-deep
+// serial LDS walk).
+constexpr int kFuse = 256;
+constexpr int kFuseLevels = 4;
+constexpr int kFuseThreads = 512;
+constexpr int kFuseWaves = kFuseThreads / 64;
 constexpr int kFusePad = kR + 2;   // doubles per LDS row
 
-__global__ __launch_bounds__(kFuseThreads, 1) void fused_levels_kernel(GroupParams p, int32_t* last_out) {
-  __shared__ alignas(16) double xs[kFuse][kFusePad];   // 136 KB: rows in level 2's input order
+__global__ __launch_bounds__(kFuseThreads, 4) void fused_levels_kernel(GroupParams p, int src, int32_t* last_out) {
+  __shared__ alignas(16) double xs[kFuse][kFusePad];   // 68 KB: rows in level 3's input order
   __shared__ unsigned short perm[2][kFuse];            // row slot at each position
   __shared__ unsigned short tok[kFuse];
-  __shared__ alignas(16) double part[2][16][kR];       // per wave, one of two buffers in turn
+  __shared__ alignas(16) double part[2][kFuseWaves][kR];       // per wave, one of two buffers in turn
   __shared__ unsigned long long key[kFuse];
   __shared__ unsigned short pos[kFuse];
   const int tid = threadIdx.x, lane = tid & 63, q = lane & 7, rg = lane >> 3;
@@ -816,7 +827,7 @@ __global__ __launch_bounds__(kFuseThreads, 1) void fused_levels_kernel(GroupPara
   const int b = blockIdx.x / (kTokens / kFuse), gi = blockIdx.x % (kTokens / kFuse);
   const long long row0 = (long long)b * kTokens + (long long)gi * kFuse;
   if (tid < kFuse) {
-    tok[tid] = (unsigned short)p.ids[0][row0 + tid];
+    tok[tid] = (unsigned short)p.ids[src][row0 + tid];
     perm[0][tid] = (unsigned short)tid;
   }
   __syncthreads();
@@ -826,9 +837,9 @@ __global__ __launch_bounds__(kFuseThreads, 1) void fused_levels_kernel(GroupPara
     const int c = tid & 15, r = tid >> 4;
     f32x4 v[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = reinterpret_cast<const f32x4*>(x + (int)tok[r + 64 * i] * kR)[c];
+    for (int i = 0; i < 8; ++i) v[i] = reinterpret_cast<const f32x4*>(x + (int)tok[r + 32 * i] * kR)[c];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) reinterpret_cast<f32x4*>(&xs[r + 64 * i][0])[c] = v[i];
+    for (int i = 0; i < 8; ++i) reinterpret_cast<f32x4*>(&xs[r + 32 * i][0])[c] = v[i];
   }
   __syncthreads();
   int cur = 0, buf = 0;
@@ -860,15 +871,10 @@ __global__ __launch_bounds__(kFuseThreads, 1) void fused_levels_kernel(GroupPara
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
-      // row group rg takes the block's waves rg mod nw (and rg + 8 of 16),
-      // then the row groups sum
+      // row group rg takes the block's wave rg mod nw, then the row groups sum
       const double* pw = part[buf][w0 + (rg & (nw - 1))] + 4 * q;
 #pragma unroll
       for (int c = 0; c < 4; ++c) a[c] = pw[c];
-      if (nw == 16) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) a[c] += pw[8 * kR + c];
-      }
       if (nw >= 2) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) a[c] = add_xor<8>(a[c]);
@@ -877,7 +883,7 @@ __global__ __launch_bounds__(kFuseThreads, 1) void fused_levels_kernel(GroupPara
 #pragma unroll
         for (int c = 0; c < 4; ++c) a[c] = add_xor<16>(a[c]);
       }
-      if (nw >= 8) {
+      if (nw == 8) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) a[c] = add_xor<32>(a[c]);
       }
@@ -955,7 +961,7 @@ __global__ __launch_bounds__(kFuseThreads, 1) void fused_levels_kernel(GroupPara
     }
     __syncthreads();
     // bitonic sort of every aligned block of n, ascending (the direction bit
-    // of the last stage is masked to the block): element tid of the first 512
+    // of the last stage is masked to the block): element tid of the first 256
     // threads
     unsigned long long k = ~0ull;
     uint32_t ps = (uint32_t)tid;
@@ -993,7 +999,7 @@ __global__ __launch_bounds__(kFuseThreads, 1) void fused_levels_kernel(GroupPara
     cur ^= 1;
     __syncthreads();
   }
-  // final order: position j is grouped page (gi * 512 + j) / 64, row j % 64
+  // final order: position j is grouped page (gi * 256 + j) / 64, row j % 64
   if (tid < kFuse) {
     const int in_head = gi * kFuse + tid, page = in_head / 64;
     const int dpage = p.page_dst ? min(max(p.page_dst[page], 0), kPages - 1) : page;   // clamped: memory safety
@@ -1065,11 +1071,12 @@ int ssa_group_order(const void* k, const void* v, long long layer_stride, long l
   hipLaunchKernelGGL(direction_kernel, rows_grid, threads, 0, stream, p);
   hipLaunchKernelGGL(keys_kernel, blocks, threads, 0, stream, p);
   hipLaunchKernelGGL(sort_kernel, rows_grid, dim3(576), 0, stream, p);          // -> ids[1]
-  hipLaunchKernelGGL(level_kernel, dim3(p.B * 3), dim3(512), 0, stream, p);     // ids[1] -> ids[0]
-  // levels 2..6 write the order (or the frame partition's input)
-  int32_t* last_out = first_chunk ? p.ids[1] : order;
-  hipLaunchKernelGGL(fused_levels_kernel, dim3(p.B * (kTokens / kFuse)), dim3(kFuseThreads), 0, stream, p, last_out);
-  if (first_chunk) hipLaunchKernelGGL(frames_kernel, dim3(p.B), dim3(256), 0, stream, p.ids[1], order);
+  hipLaunchKernelGGL((level_kernel<kTokens / 3, 512>), dim3(p.B * 3), dim3(512), 0, stream, p, 1);   // -> ids[0]
+  hipLaunchKernelGGL((level_kernel<kTokens / 9, 256>), dim3(p.B * 9), threads, 0, stream, p, 0);      // -> ids[1]
+  // levels 3..6 write the order (or the frame partition's input)
+  int32_t* last_out = first_chunk ? p.ids[0] : order;
+  hipLaunchKernelGGL(fused_levels_kernel, dim3(p.B * (kTokens / kFuse)), dim3(kFuseThreads), 0, stream, p, 1, last_out);
+  if (first_chunk) hipLaunchKernelGGL(frames_kernel, dim3(p.B), threads, 0, stream, p.ids[0], order);
   return (int)hipGetLastError();
 }
 
