@@ -35,7 +35,6 @@
 #include "common.h"
 
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 
 using namespace ssa;
@@ -1126,25 +1125,6 @@ void launch_merge(const AttnParams& p, int tiles, int split_from, int pieces, hi
   else
     hipLaunchKernelGGL((merge_kernel<NB, kMaxPieces>), grid, block, 0, stream, p.part, p.out, split_from, pieces, p.T,
                        p.q_tok, p.q_head);
-}
-
-// Compute units of the current device (cached per device).
-int device_cus(int* out) {
-  constexpr int kMaxDevices = 64;
-  static std::atomic<int> cus[kMaxDevices];
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return (int)e;
-  if (dev < 0 || dev >= kMaxDevices) return (int)hipErrorInvalidDevice;
-  int n = cus[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess) return (int)e;
-    n = n > 0 ? n : 1;
-    cus[dev].store(n, std::memory_order_relaxed);
-  }
-  *out = n;
-  return (int)hipSuccess;
 }
 
 // The split a call runs: the workgroups past the last multiple of the CU

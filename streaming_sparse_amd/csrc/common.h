@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 namespace ssa {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -214,6 +216,25 @@ __device__ __forceinline__ u32x4 rep_operand_chunk(const uint16_t* det, int P, i
     out[x] = packed;
   }
   return out;
+}
+
+// Compute units of the current device (cached per device).
+inline int device_cus(int* out) {
+  constexpr int kMaxDevices = 64;
+  static std::atomic<int> cus[kMaxDevices];
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return (int)e;
+  if (dev < 0 || dev >= kMaxDevices) return (int)hipErrorInvalidDevice;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return (int)e;
+    n = n > 0 ? n : 1;
+    cus[dev].store(n, std::memory_order_relaxed);
+  }
+  *out = n;
+  return (int)hipSuccess;
 }
 
 }  // namespace ssa

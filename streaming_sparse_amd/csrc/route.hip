@@ -13,8 +13,8 @@
 //          (VR/runtime.py:279-288) or fixed top-k (VR/fixed_page_select.py:8-47)
 //   ids  = own first, then descending risk                (VB/graph.py:210)
 //
-// Workgroup: 256 threads (4 waves) = 32 probes (2 query blocks) of one head.
-// Each wave takes every 4th tile of 32 reps (8 pages).  S^T = R . Probe^T runs
+// Workgroup: 4 or 8 waves = 32 probes (2 query blocks) of one head.  Each
+// wave takes every 4th or 8th tile of 32 reps (8 pages).  S^T = R . Probe^T runs
 // on v_mfma_f32_32x32x16_bf16, so a lane holds one probe and the 4 reps of
 // each of its pages: the page's features are lane-local.  One pass over the
 // reps: each lane keeps a running max and sum of exponentials of its probe,
@@ -31,11 +31,9 @@ using namespace ssa;
 
 namespace {
 
-constexpr int kThreads = 256;
 constexpr int kMaxPages = 512;
 constexpr int kAnchors = 24;
 constexpr int kCurrent = 72;
-constexpr int kTilesPerWave = kMaxPages / 32;   // tiles of 8 pages, every 4th to a wave
 
 // Phase stamps of a measurement build (-DSSA_ROUTE_STAMPS, see
 // streaming_sparse_amd/build.py): lane 0 of each wave of the first
@@ -48,7 +46,7 @@ constexpr int kStampBlocks = 1024, kStampSlots = 16;
 __device__ unsigned long long route_stamps[kStampBlocks * 4 * kStampSlots];
 #define ROUTE_STAMP(k)                                                                       \
   do {                                                                                       \
-    if ((threadIdx.x & 63) == 0 && blockIdx.x < kStampBlocks)                                \
+    if ((threadIdx.x & 63) == 0 && threadIdx.x < 256 && blockIdx.x < kStampBlocks)                                \
       route_stamps[(blockIdx.x * 4 + (threadIdx.x >> 6)) * kStampSlots + (k)] = __builtin_amdgcn_s_memtime(); \
   } while (0)
 #else
@@ -95,13 +93,14 @@ struct Sel {                   // selection state, aliasing the tile ring once t
   int list[2][kMaxPages];
 };
 
+template <int NW>
 struct Smem {
-  alignas(16) uint8_t ring[4][2][kSlotBytes];   // per-wave double buffer of rep tiles
-  float part[4][32][2];        // per-wave (max, sum) of each probe
-  float bmax[4];               // per-wave maximum of stats[p,1,11]
+  alignas(16) uint8_t ring[NW][2][kSlotBytes];   // per-wave double buffer of rep tiles
+  float part[NW][32][2];       // per-wave (max, sum) of each probe
+  float bmax[NW];              // per-wave maximum of stats[p,1,11]
   float risk[2][kMaxPages];
 };
-static_assert(sizeof(Sel) <= sizeof(Smem::ring), "selection state must fit in the tile ring");
+static_assert(sizeof(Sel) <= sizeof(Smem<4>::ring), "selection state must fit in the tile ring");
 
 // Maxima as trees of v_max3 / v_max.  The sources build with NaN-free
 // float semantics, so the compiler adds no quieting of matrix-pipe results
@@ -154,21 +153,23 @@ __device__ __forceinline__ unsigned long long xlane64(unsigned long long v, int 
   return ((unsigned long long)hi << 32) | lo;
 }
 
-// Descending bitonic sort of one row's 512 keys, held 4 per thread (element
-// 4*bt + i in key[i]) by the row's 128 threads (two waves): partner distance
-// 1 and 2 inside the thread, 4..128 by cross-lane shuffles inside the wave,
-// 256 through LDS (`xchg`, the row's 512 slots) between the two waves.  Every
-// thread of the workgroup calls it (both rows sort in lockstep; two barriers).
-__device__ __forceinline__ void sort512_desc(unsigned long long (&key)[4], int bt, unsigned long long* xchg) {
+// Descending bitonic sort of one row's 512 keys, held KPT (2 or 4) per thread
+// (element KPT * bt + i in key[i]) by the row's 512 / KPT threads: partner
+// distances below KPT inside the thread, up to 32 KPT by cross-lane
+// exchanges inside the wave, beyond through LDS (`xchg`, the row's 512 slots)
+// between the row's waves.  Every thread of the workgroup calls it (both rows
+// sort in lockstep).
+template <int KPT>
+__device__ __forceinline__ void sort512_desc(unsigned long long (&key)[KPT], int bt, unsigned long long* xchg) {
 #pragma unroll
   for (int k = 2; k <= kMaxPages; k <<= 1) {
 #pragma unroll
     for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j < 4) {
+      if (j < KPT) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < KPT; ++i) {
           if (i & j) continue;
-          const int e = 4 * bt + i;
+          const int e = KPT * bt + i;
           const bool desc = (e & k) == 0;
           const unsigned long long x = key[i], y = key[i | j];
           if ((x < y) == desc) {
@@ -177,31 +178,31 @@ __device__ __forceinline__ void sort512_desc(unsigned long long (&key)[4], int b
           }
         }
       } else {
-        unsigned long long other[4];
-        if (j <= 128) {
+        unsigned long long other[KPT];
+        if (j <= 32 * KPT) {
           const int lane = bt & 63;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            switch (j) {
-              case 4: other[i] = xlane64<1>(key[i], lane); break;
-              case 8: other[i] = xlane64<2>(key[i], lane); break;
-              case 16: other[i] = xlane64<4>(key[i], lane); break;
-              case 32: other[i] = xlane64<8>(key[i], lane); break;
-              case 64: other[i] = xlane64<16>(key[i], lane); break;
+          for (int i = 0; i < KPT; ++i) {
+            switch (j / KPT) {
+              case 1: other[i] = xlane64<1>(key[i], lane); break;
+              case 2: other[i] = xlane64<2>(key[i], lane); break;
+              case 4: other[i] = xlane64<4>(key[i], lane); break;
+              case 8: other[i] = xlane64<8>(key[i], lane); break;
+              case 16: other[i] = xlane64<16>(key[i], lane); break;
               default: other[i] = xlane64<32>(key[i], lane); break;
             }
           }
         } else {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) xchg[4 * bt + i] = key[i];
+          for (int i = 0; i < KPT; ++i) xchg[KPT * bt + i] = key[i];
           __syncthreads();
 #pragma unroll
-          for (int i = 0; i < 4; ++i) other[i] = xchg[(4 * bt + i) ^ j];
+          for (int i = 0; i < KPT; ++i) other[i] = xchg[(KPT * bt + i) ^ j];
           __syncthreads();
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int e = 4 * bt + i;
+        for (int i = 0; i < KPT; ++i) {
+          const int e = KPT * bt + i;
           const bool desc = (e & k) == 0;
           const bool keep_max = ((e & j) == 0) == desc;
           const unsigned long long x = key[i], y = other[i];
@@ -214,11 +215,11 @@ __device__ __forceinline__ void sort512_desc(unsigned long long (&key)[4], int b
 
 // Detail operand tiles written on the side by workgroups of their own,
 // appended to the router's grid: they take the slots of the CUs that hold
-// one router workgroup.  Thread c of block r writes chunk r * kThreads + c
+// one router workgroup.  Thread c of block r writes chunk r * threads + c
 // of the flat (head, tile, chunk) range.
-__device__ void rep_operand_block(const RouteParams& p, int r) {
+__device__ __forceinline__ void rep_operand_block(const RouteParams& p, int r, int threads) {
   const int tiles = (p.P + 15) >> 4;
-  const int f = r * kThreads + threadIdx.x;
+  const int f = r * threads + threadIdx.x;
   if (f >= p.H * tiles * kRepOpChunks) return;
   const int c = f % kRepOpChunks, ht = f / kRepOpChunks, h = ht / tiles, rt = ht % tiles;
   const u32x4 w = rep_operand_chunk(p.rdetail + (long long)h * p.HP * 24, p.P, rt, c);
@@ -227,12 +228,18 @@ __device__ void rep_operand_block(const RouteParams& p, int r) {
 
 __global__ __launch_bounds__(1) void zero_count_kernel(int32_t* count) { *count = 0; }
 
-__global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
-  __shared__ Smem s;
+// NW waves per workgroup: 4, two workgroups per CU, or 8, one per CU, where
+// the grid has no more workgroups than the chip has CUs (the tiles and the
+// selection then spread over twice the waves).
+template <int NW>
+__global__ __launch_bounds__(64 * NW, 2) void route_kernel(RouteParams p) {
+  constexpr int kThreads = 64 * NW, kRowThreads = kThreads / 2, kKeys = kMaxPages / kRowThreads;
+  constexpr int kTilesPerWave = kMaxPages / 8 / NW;     // tiles of 8 pages, every NW-th to a wave
+  __shared__ Smem<NW> s;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int NP = (p.T + 1) >> 1;
   if ((int)blockIdx.x >= p.H * NP) {
-    rep_operand_block(p, blockIdx.x - p.H * NP);
+    rep_operand_block(p, blockIdx.x - p.H * NP, kThreads);
     return;
   }
   const int work = xcd_remap(blockIdx.x, p.H * NP);
@@ -247,11 +254,11 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
   const int ntiles = (P + 7) >> 3;
   // logits in log2 units: z2 = q.k * log2(e) / sqrt(D); prob = 2^(z2 - max2) / den
   const float c2 = kLog2e / sqrtf((float)kHeadDim);
-  // Each wave owns tiles wave + 4 j (j < nmine) and a double buffer of them
+  // Each wave owns tiles wave + NW j (j < nmine) and a double buffer of them
   // in LDS: no other wave reads its slots, so its own load counter orders
-  // them.  A wave without tiles (P <= 24) re-reads the last tile and skips it.
-  const int nmine = __builtin_amdgcn_readfirstlane(max((ntiles - wave + 3) >> 2, 0));
-  auto mine = [&](int jj) { return min(wave + 4 * max(min(jj, nmine - 1), 0), ntiles - 1); };
+  // them.  A wave without tiles (a short window) re-reads the last tile and skips it.
+  const int nmine = __builtin_amdgcn_readfirstlane(max((ntiles - wave + NW - 1) / NW, 0));
+  auto mine = [&](int jj) { return min(wave + NW * max(min(jj, nmine - 1), 0), ntiles - 1); };
   lds_u8* const ring = (lds_u8*)&s.ring[wave][0][0];
   const uint32_t ring_addr = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)ring);
   // row offsets of a full tile in the instruction-offset form of dma_rows:
@@ -305,16 +312,17 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
       dma16(qb, off, ring_addr + kSlotBytes + jj * 1024);
     }
   }
-  // max_p stats[p,1,11] over the head's pages: wave w reads pages
-  // 128 w + lane and 128 w + 64 + lane (pages <= 512), the workgroup
-  // combines the four partial maxima in LDS before the tiles (each page's
+  // max_p stats[p,1,11] over the head's pages: wave w reads every NW-th 64
+  // pages' share (pages <= 512), the workgroup combines the partial maxima
+  // in LDS before the tiles (each page's
   // value is a lone 2-byte word, so a wave's loads cost the address unit one
   // cache line per lane: reading every page in every wave queued 8 such
   // loads per wave behind one another)
-  uint32_t bw[2];
+  constexpr int kBounds = kMaxPages / kThreads;
+  uint32_t bw[kBounds];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int pg = 128 * wave + 64 * i + lane;
+  for (int i = 0; i < kBounds; ++i) {
+    const int pg = 64 * (kBounds * wave + i) + lane;
     bw[i] = pg < P ? sth[(long long)pg * 48 + 23] : 0xff80u;
   }
   auto uniform = [](float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v))); };
@@ -332,7 +340,7 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
   asm volatile("" ::"s"(own_raw[0]), "s"(own_raw[1]), "s"(cur_raw));
   // the loads above are complete past this point
 #pragma unroll
-  for (int i = 0; i < 2; ++i) asm volatile("" ::"v"(bw[i]));
+  for (int i = 0; i < kBounds; ++i) asm volatile("" ::"v"(bw[i]));
   wait_loads();
   ROUTE_STAMP(1);   // the setup's loads are in
   // probe operand (B): dims 16*st + 8*hh + [0,8) of probe pi, the k order of
@@ -363,10 +371,15 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
   for (int g = 0; g < 8; ++g) qsum += q2[g];
   const float qn = sqrtf(qsum * kHeadDim) / sqrtf((float)kHeadDim);
 
-  float bmax = wave_reduce(fmaxf(bf16_to_f32(bw[0]), bf16_to_f32(bw[1])), [](float a, float b) { return fmaxf(a, b); });
+  float bmax = bf16_to_f32(bw[0]);
+#pragma unroll
+  for (int i = 1; i < kBounds; ++i) bmax = fmaxf(bmax, bf16_to_f32(bw[i]));
+  bmax = wave_reduce(bmax, [](float a, float b) { return fmaxf(a, b); });
   if (lane == 0) s.bmax[wave] = bmax;
   __syncthreads();
-  bmax = fmaxf(fmaxf(s.bmax[0], s.bmax[1]), fmaxf(s.bmax[2], s.bmax[3]));
+  bmax = s.bmax[0];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) bmax = fmaxf(bmax, s.bmax[w]);
 
   // One pass over the reps.  Each lane keeps a running max m and sum of
   // exponentials den of its probe over its reps; the features of a page are
@@ -420,7 +433,10 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
     rep_logits(av, qop, S);
   };
   const uint32_t lo_only = hh == 0 ? 0xffffffffu : 0u;
-  float mx = -INFINITY, den = 0.f;
+  // the running max starts finite: a lane half without a page in the wave's
+  // first tile (a window of 8 n + 1 pages) then keeps probabilities of zero
+  // instead of exponents of -inf + inf
+  float mx = -3.402823466e38f, den = 0.f;
   float vals[kTilesPerWave][4], mj[kTilesPerWave];
   ROUTE_STAMP(2);   // probe norms, B operands, first tiles issued
   auto soft = [&](f32x16 S, const TileStats& ts, int tile, float (&v4)[4], float& mt) {
@@ -484,8 +500,7 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
   {
     const float omx = xor_lane<32>(mx), oden = xor_lane<32>(den);
     const float mm = fmaxf(mx, omx);
-    const float mu = mm == -INFINITY ? 0.f : mm;   // a wave without tiles (P <= 24) has none
-    den = den * __builtin_amdgcn_exp2f(mx - mu) + oden * __builtin_amdgcn_exp2f(omx - mu);
+    den = den * __builtin_amdgcn_exp2f(mx - mm) + oden * __builtin_amdgcn_exp2f(omx - mm);
     mx = mm;
     if (hh == 0) {
       s.part[wave][pi][0] = mx;
@@ -495,10 +510,10 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
   __syncthreads();
   float MX = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) MX = fmaxf(MX, s.part[w][pi][0]);
+  for (int w = 0; w < NW; ++w) MX = fmaxf(MX, s.part[w][pi][0]);
   float DEN = 0.f;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) DEN += s.part[w][pi][1] * __builtin_amdgcn_exp2f(s.part[w][pi][0] - MX);
+  for (int w = 0; w < NW; ++w) DEN += s.part[w][pi][1] * __builtin_amdgcn_exp2f(s.part[w][pi][0] - MX);
   const float nlse = -(MX + __log2f(DEN));
   ROUTE_STAMP(4);   // probe totals
   if (p.lse && wave == 0 && hh == 0 && t0 + blk < p.T)
@@ -512,11 +527,9 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
     if (j < nmine) {
       const float f = __builtin_amdgcn_exp2f(mj[j] + nlse);
       const int tile = mine(j);
+      // pages past the window (of its last tile) land in slots nobody reads
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int page = tile * 8 + 2 * jj + hh;
-        if (page < P) tr[blk * kTrBlock + page * 16 + m] = vals[j][jj] * f;
-      }
+      for (int jj = 0; jj < 4; ++jj) tr[blk * kTrBlock + (tile * 8 + 2 * jj + hh) * 16 + m] = vals[j][jj] * f;
     }
   }
   __syncthreads();
@@ -540,11 +553,10 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
 
   // ---------------------------------------------------------------- select
   Sel& sl = *reinterpret_cast<Sel*>(&s.ring[0][0][0]);
-  // Row b is sorted by its 128 threads (tid / 128 = b), 512 64-bit keys,
-  // descending.  Key = (group << 62) | (orderable risk << 30) | (1023 - page):
+  // Row b is sorted by its half of the threads, 512 64-bit keys, descending.  Key = (group << 62) | (orderable risk << 30) | (1023 - page):
   // risk descending, ties -> lower page, and the group field orders the
   // partitions (base / top-k: one group).
-  const int b = tid >> 7, bt = tid & 127;
+  const int b = tid / kRowThreads, bt = tid % kRowThreads;
   int own[2];
   // own pages outside the window are clamped into it (memory safety of the
   // per-page state; a valid own is in [0, P))
@@ -565,10 +577,10 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
     A = min(max(araw, 0), ncur);
     nh = min(max(p.total - araw, 0), nhist);
   }
-  unsigned long long keys[4];
+  unsigned long long keys[kKeys];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int pg = 4 * bt + i;
+  for (int i = 0; i < kKeys; ++i) {
+    const int pg = kKeys * bt + i;
     unsigned long long key = 0ull;
     if (pg < P) {
       const unsigned long long ord = (unsigned long long)orderable(s.risk[b][pg]) << 30;
@@ -589,7 +601,7 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
   sort512_desc(keys, bt, sl.key[b]);
   ROUTE_STAMP(8);   // sorted
 #pragma unroll
-  for (int i = 0; i < 4; ++i) sl.key[b][4 * bt + i] = keys[i];
+  for (int i = 0; i < kKeys; ++i) sl.key[b][kKeys * bt + i] = keys[i];
   __syncthreads();
   // sl.key[b] sorted descending; the page of entry i is 1023 - (key & 1023)
   auto page_at = [&](int i) -> int { return 1023 - (int)(sl.key[b][i] & 1023ull); };
@@ -621,17 +633,17 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
     if (tie) p.tie_rows[atomicAdd(p.tie_count, 1)] = h * p.T + t0 + b;
   }
   int32_t* idsrow = p.ids ? p.ids + ((long long)h * p.T + t0 + b) * p.C : nullptr;
-  for (int pg = bt; pg < P; pg += 128) sl.sel[b][pg] = 0;
+  for (int pg = bt; pg < P; pg += kRowThreads) sl.sel[b][pg] = 0;
   __syncthreads();
   if (p.mode == 0) {
     // LUT = [own, 0..23, top C-25 candidates], already in order
-    for (int i = bt; i < p.C; i += 128) {
+    for (int i = bt; i < p.C; i += kRowThreads) {
       const int pg = i == 0 ? own[b] : (i <= kAnchors ? i - 1 : page_at(i - 1 - kAnchors));
       sl.sel[b][pg] = 1;
       if (row_ok && idsrow) idsrow[i] = pg;
     }
   } else if (p.mode == 2) {
-    for (int i = bt; i < p.C; i += 128) {
+    for (int i = bt; i < p.C; i += kRowThreads) {
       const int pg = page_at(i);
       sl.sel[b][pg] = 1;
       if (row_ok && idsrow) idsrow[i] = pg;
@@ -640,7 +652,7 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
     // quota: current top A at sorted [0, A) (own first), history top nh at
     // sorted [ncur, ncur + nh), anchors; list them, then order the LUT by risk
     const int nlist = kAnchors + A + nh;    // <= P
-    for (int i = bt; i < nlist; i += 128) {
+    for (int i = bt; i < nlist; i += kRowThreads) {
       const int pg = i < A ? page_at(i) : (i < A + nh ? page_at(ncur + i - A) : i - A - nh);
       sl.list[b][i] = pg;
       sl.sel[b][pg] = 1;
@@ -656,27 +668,27 @@ __global__ __launch_bounds__(kThreads, 2) void route_kernel(RouteParams p) {
       // their place.
       const bool own_listed = sl.sel[b][own[b]] != 0;
       const int nent = nlist + (own_listed ? 0 : 1);   // <= P
-      for (int i = bt; i < nent; i += 128) {
+      for (int i = bt; i < nent; i += kRowThreads) {
         const int pg = i < nlist ? sl.list[b][i] : own[b];
         if (i >= nlist) sl.list[b][i] = pg;
         sl.key[b][i] = pg == own[b] ? ~0ull
                                     : ((unsigned long long)orderable(s.risk[b][pg]) << 32) | (uint32_t)(1023 - pg);
       }
       __syncthreads();
-      for (int i = bt; i < nent; i += 128) {
+      for (int i = bt; i < nent; i += kRowThreads) {
         const unsigned long long kx = sl.key[b][i];
         int rank = 0;
 #pragma unroll 8
         for (int j = 0; j < nent; ++j) rank += sl.key[b][j] > kx;
         if (row_ok && rank < p.C) idsrow[rank] = sl.list[b][i];
       }
-      for (int i = nent + bt; i < p.C; i += 128)
+      for (int i = nent + bt; i < p.C; i += kRowThreads)
         if (row_ok) idsrow[i] = -1;
     }
   }
   __syncthreads();
   if (p.mask) {
-    for (int pg = bt; pg < P; pg += 128)
+    for (int pg = bt; pg < P; pg += kRowThreads)
       if (row_ok) p.mask[((long long)h * p.T + t0 + b) * P + pg] = sl.sel[b][pg];
   }
   ROUTE_STAMP(10);  // table, near-tie report and mask written
@@ -861,8 +873,21 @@ int ssa_route(const void* q, long long q_head_stride, long long q_block_stride, 
   // that a captured graph replays it
   if (tie_rows) hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, stream, tie_count);
   const int np = (blocks + 1) / 2;
-  const int nrv = rep_ops ? (heads * ((pages + 15) / 16) * kRepOpChunks + kThreads - 1) / kThreads : 0;
-  hipLaunchKernelGGL(route_kernel, dim3(heads * np + nrv), dim3(kThreads), 0, stream, p);
+  // A grid of at most one workgroup per CU runs 8 waves each (base route: 1
+  // head x 8 blocks, 180 pages 18.1 -> 12.7 us, 2 x 72, 432 pages 22.0 -> 18.0,
+  // 7 x 72, 300 pages 19.8 -> 18.1); beyond that two 4-wave workgroups share a
+  // CU, which 8 waves of either kind fill with their registers, and the wide
+  // ones would run one after the other.
+  int cus = 0;
+  const int e = device_cus(&cus);
+  if (e != (int)hipSuccess) return e;
+  const bool wide = heads * np <= cus;
+  const int threads = wide ? 512 : 256;
+  const int nrv = rep_ops ? (heads * ((pages + 15) / 16) * kRepOpChunks + threads - 1) / threads : 0;
+  if (wide)
+    hipLaunchKernelGGL(route_kernel<8>, dim3(heads * np + nrv), dim3(threads), 0, stream, p);
+  else
+    hipLaunchKernelGGL(route_kernel<4>, dim3(heads * np + nrv), dim3(threads), 0, stream, p);
   return (int)hipGetLastError();
 }
 

@@ -72,6 +72,29 @@ def test_risk_small_windows(device, pages):
     assert rel < 1e-4
 
 
+@pytest.mark.parametrize("blocks,pages", [(1, 8), (1, 9), (2, 20), (3, 57), (5, 72), (4, 97), (7, 216), (512, 100),
+                                          (514, 25), (514, 100)])
+def test_route_wide_and_narrow_workgroups(device, blocks, pages):
+    """One head with a grid of at most one workgroup per CU (256 CUs: 512
+    blocks) runs the router with 8 waves, 514 blocks with 4: windows that
+    leave waves of either kind without a tile, end in a partial tile (of one
+    page, as a wave's first tile: 9, 57 and 25) or fill it, odd block counts; risk within 1e-4 of the float64 oracle and the
+    top-k table ranked by that risk, own first, ties to the lower page."""
+    x = call_inputs(0, 9)
+    sub = x.summary.slice(0, pages)
+    s = Summary(*(getattr(sub, f)[:1].contiguous() for f in sub.FIELDS))
+    gs = Summary(*(getattr(s, f).to(device) for f in s.FIELDS))
+    q = x.q[:, :, :1].repeat(1, 8, 1, 1)[:, :64 * blocks].contiguous()
+    own = (torch.arange(blocks) % pages)[None]
+    ids, mask, risk, _ = route(q.to(device), gs, x.theta[:1].to(device), tier='topk', own=own.to(device))
+    pr = ref.probes(q)
+    want = ref.risk(pr, ref.route_logits(pr, s.keys, torch.float64), s.stats, x.theta[:1], dtype=torch.float64)
+    rel = float(((risk.cpu().double() - want).abs() / want.abs().clamp_min(1e-30)).max())
+    assert rel < 1e-4, rel
+    got_ids, got_mask = ref.select_topk(risk.cpu(), own, max(1, int(pages * 0.1)))
+    assert torch.equal(ids.cpu(), got_ids) and torch.equal(mask.cpu(), got_mask)
+
+
 @pytest.mark.parametrize("cfg,frames", [(0, 9), (1, 18)])
 def test_route_base_matches_oracle(device, cfg, frames):
     x = call_inputs(cfg, frames)
