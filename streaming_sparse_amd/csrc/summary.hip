@@ -26,6 +26,13 @@
 // ascending token order.  LDS stays under 40 KB so four workgroups share a
 // CU.
 //
+// Vector instructions bound it (the vector pipes are about two thirds busy
+// over the kernel's life), not the 1 KB per row that it moves: 72 pages of
+// 12 heads written through take 23.1 us, 11.3 us of it for their bytes.
+// Lane masks of the cluster sums are picked once per Lloyd step instead of
+// once per matrix step, and the detail formed once per wave instead of once
+// per lane: 23.6 -> 23.1 us.
+//
 // ssa_summary_write reads the page rows from the chunk's K/V instead and
 // writes them into the cache in the same pass (the window write that
 // precedes the summary recompute, VR/runtime.py:205-206).
@@ -76,6 +83,7 @@ struct SumSmem {
   } u;
   float kmean[128], vmean[128];
   float code[4][8];
+  alignas(16) float det[4][24];          // per wave: the bf16-rounded detail
 };
 
 __device__ __forceinline__ int word(int t, int w) { return t * 64 + (w ^ ((t & 15) << 2)); }
@@ -120,18 +128,26 @@ __device__ __forceinline__ u32x4 rows_operand(const uint32_t* rows, int dt, int 
   return u32x4{ua[0], ua[1], ub[0], ub[1]};
 }
 
-// A operand of the cluster sums: row m = lane % 32 is the 0/1 membership of
-// cluster m (m < 4) or all ones (m == 4: the page sum) or zero, over the
-// tokens of rows_operand's k order.
-__device__ __forceinline__ u32x4 member_operand(const uint64_t (&mk)[4], int ks, int lane) {
-  const int m = lane & 31, hh = lane >> 5;
-  const uint64_t msk = m < 4 ? mk[m] : (m == 4 ? ~0ull : 0ull);
-  const uint32_t bits = (uint32_t)((msk >> (16 * ks + 4 * hh)) & 0xFu) |
-                        ((uint32_t)((msk >> (16 * ks + 8 + 4 * hh)) & 0xFu) << 4);
+// Member mask of this lane's row of the cluster sums: row m = lane % 32 is
+// cluster m (m < 4), all tokens (m == 4: the page sum) or none.
+__device__ __forceinline__ uint64_t member_mask(const uint64_t (&mk)[4], int lane) {
+  const int m = lane & 31;
+  return m < 4 ? mk[m] : (m == 4 ? ~0ull : 0ull);
+}
+
+// A operand of the cluster sums: the 0/1 membership `mask` of this lane's row
+// over the tokens of rows_operand's k order (tokens 16 ks + 4 hh + 0..3, then
+// 8 further), each bit spread to a bf16 one by a sign-extended field.
+__device__ __forceinline__ u32x4 member_operand(uint64_t mask, int ks, int lane) {
+  const uint32_t half = ks & 2 ? (uint32_t)(mask >> 32) : (uint32_t)mask;
+  const uint32_t bits = half >> ((lane >> 5) << 2);
+  auto one = [&](int at) { return (uint32_t)((int32_t)(bits << (31 - at)) >> 31); };
   u32x4 w;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-    w[j] = ((bits >> (2 * j)) & 1u ? 0x3F80u : 0u) | ((bits >> (2 * j + 1)) & 1u ? 0x3F800000u : 0u);
+  for (int j = 0; j < 4; ++j) {
+    const int at = 16 * (ks & 1) + 8 * (j >> 1) + 2 * (j & 1);
+    w[j] = (one(at) & 0x3F80u) | (one(at + 1) & 0x3F800000u);
+  }
   return w;
 }
 
@@ -142,8 +158,9 @@ __device__ __forceinline__ u32x4 member_operand(const uint64_t (&mk)[4], int ks,
 // page sum of that dim in item 0.
 __device__ __forceinline__ f32x16 cluster_sums(const uint32_t* rows, const uint64_t (&mk)[4], int dt, int lane) {
   f32x16 c = {};
+  const uint64_t mask = member_mask(mk, lane);
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) c = mfma32(member_operand(mk, ks, lane), rows_operand(rows, dt, ks, lane), c);
+  for (int ks = 0; ks < 4; ++ks) c = mfma32(member_operand(mask, ks, lane), rows_operand(rows, dt, ks, lane), c);
   return c;
 }
 
@@ -367,21 +384,35 @@ __global__ __launch_bounds__(256, 4) void summary_kernel(SummaryParams p, Layers
     }
   }
   __syncthreads();
-  // detail = bf16(HAAR . code / 4), every wave
+  // detail = bf16(HAAR . code / 4): lane 8 a + kk of every wave forms one of
+  // the 24 (each lane forming all 24 took 12x the vector instructions), hands
+  // it to the wave's other lanes through LDS, and every lane then combines
+  // the three contrasts into the 8 coefficients of cluster r's basis rows
+  const long long pg = (long long)h * p.HP + page;
+  {
+    const int kk = lane & 7, a = min(lane >> 3, 2);
+    const float c0 = s.code[0][kk], c1 = s.code[1][kk], c2 = s.code[2][kk], c3 = s.code[3][kk];
+    const float b1 = a == 0 ? c1 : -c1, b2 = a == 1 ? c2 : -c2, b3 = a == 2 ? c3 : -c3;
+    const uint16_t d = to_bf16((((c0 + b1) + b2) + b3) / 4.f);
+    if (wave == 0 && lane < 24) p.detail[pg * 24 + lane] = d;
+    if (lane < 24) s.det[r][lane] = bf16_to_f32(d);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   float det[3][8];
 #pragma unroll
-  for (int a = 0; a < 3; ++a) {
+  for (int a = 0; a < 3; ++a)
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
-      const float v = (kHaar[a][0] * s.code[0][kk] + kHaar[a][1] * s.code[1][kk] + kHaar[a][2] * s.code[2][kk] +
-                       kHaar[a][3] * s.code[3][kk]) / 4.f;
-      det[a][kk] = bf16_to_f32(to_bf16(v));
+    for (int kk = 0; kk < 8; kk += 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(&s.det[r][8 * a + kk]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) det[a][kk + e] = v[e];
     }
-  }
-  const long long pg = (long long)h * p.HP + page;
-  if (wave == 0 && lane < 24) p.detail[pg * 24 + lane] = to_bf16(
-      (kHaar[lane >> 3][0] * s.code[0][lane & 7] + kHaar[lane >> 3][1] * s.code[1][lane & 7] +
-       kHaar[lane >> 3][2] * s.code[2][lane & 7] + kHaar[lane >> 3][3] * s.code[3][lane & 7]) / 4.f);
+  float coef[8];
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk)
+    coef[kk] = kHaar[0][r] * det[0][kk] + kHaar[1][r] * det[1][kk] + kHaar[2][r] * det[2][kk];
   // reps, reconstruction error, stats of cluster r
   float e8 = 0.f, e9 = 0.f;
   uint32_t pk_pair;
@@ -397,10 +428,7 @@ __global__ __launch_bounds__(256, 4) void summary_kernel(SummaryParams p, Layers
       const float mu = bf16_to_f32(to_bf16(s.vmean[d]));
       float acc = 0.f;
 #pragma unroll
-      for (int kk = 0; kk < 8; ++kk) {
-        const float c = kHaar[0][r] * det[0][kk] + kHaar[1][r] * det[1][kk] + kHaar[2][r] * det[2][kk];
-        acc = fmaf(c, j == 0 ? bas0[kk] : bas1[kk], acc);
-      }
+      for (int kk = 0; kk < 8; ++kk) acc = fmaf(coef[kk], j == 0 ? bas0[kk] : bas1[kk], acc);
       const float x8 = km - pk[j], x9 = vm[j] - (mu + acc);
       e8 = fmaf(x8, x8, e8);
       e9 = fmaf(x9, x9, e9);
