@@ -443,60 +443,68 @@ __device__ __forceinline__ void pv(const u32x4 (&pb)[2], const u32x4 (&pl)[2], c
 
 // Unit list of tile (t, h): its exact pages in LUT order, then the rep tiles
 // holding at least one page the table does not select (each carrying its
-// drop mask); maskw gets the 512-bit page mask.  LUT entries outside [0, P)
-// (the -1 padding of a shorter table) are not read: they add no exact unit
-// and select nothing.  A page listed twice is attended twice, as a LUT walk
-// does.  Called by every 4-wave workgroup's threads; wcount is 4 ints of LDS.
-// first: this thread's entry of the table's first kThreads entries, read by
-// the caller (lut_entry) before its other loads.
-__device__ __forceinline__ int lut_entry(const AttnParams& p, int h, int t, int i) {
-  return i < p.C ? p.ids[((long long)h * p.T + t) * p.C + i] : -1;
-}
-
+// drop mask).  LUT entries outside [0, P) (the -1 padding of a shorter table)
+// are not read: they add no exact unit and select nothing.  A page listed
+// twice is attended twice, as a LUT walk does.
+//
+// Every wave builds the whole list by itself (all write the same values to
+// `units`) with a page mask of its own, so the first K/V loads wait for the
+// table entries alone: not for the query rows, which a barrier's wait takes
+// in, nor for the other waves.  Latency bound it; a workgroup's list and
+// first loads together went from 10.4k to 8.4k cycles of the ~107k that half
+// a list of 83 units takes (185 tiles: 63.0 -> 62.1 us a call; 24 tiles of 36
+// units 16.3 -> 15.2; 864 tiles of 91 units 223 -> 221).
+//
 // STAGE 1 lists the exact pages only, STAGE 2 the rep tiles only (the two
 // launches of a staged call); STAGE 0 both.
+constexpr int kLutRows = kMaxCount / 64;   // table entries per lane, at most
+
+struct UnitCounts {
+  int nunits, nexact;
+};
+
+// Orders this wave's LDS writes before its lanes' later LDS reads.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <int STAGE>
-__device__ void own_units(const AttnParams& p, int h, int t, int tid, int first, int* units, uint32_t* maskw,
-                          int* wcount, int* nunits, int* nexact) {
-  const int lane = tid & 63, wave = tid >> 6;
-  if (tid < 16) maskw[tid] = 0u;
-  __syncthreads();
+__device__ __forceinline__ UnitCounts own_units(const AttnParams& p, int lane, const int (&lut)[kLutRows], int* units,
+                                                uint32_t* maskw) {
+  if (lane < 16) maskw[lane] = 0u;
+  wave_lds_fence();
   int base = 0;
-  for (int i0 = 0; i0 < p.C; i0 += kThreads) {
-    const int pg = i0 == 0 ? first : lut_entry(p, h, t, i0 + tid);
+#pragma unroll
+  for (int j = 0; j < kLutRows; ++j) {
+    if (64 * j >= p.C) break;
+    const int pg = lut[j];
     const bool ok = pg >= 0 && pg < p.P;
     const unsigned long long bal = __ballot(ok);
-    if (lane == 0) wcount[wave] = __popcll(bal);
-    __syncthreads();
-    int off = base;
-    for (int w = 0; w < wave; ++w) off += wcount[w];
     if (ok) {
-      if (STAGE != 2) units[off + __popcll(bal & ((1ull << lane) - 1ull))] = pg;
+      if (STAGE != 2) units[base + __popcll(bal & ((1ull << lane) - 1ull))] = pg;
       atomicOr(&maskw[pg >> 5], 1u << (pg & 31));
     }
-    base += wcount[0] + wcount[1] + wcount[2] + wcount[3];
-    __syncthreads();
+    base += (int)__popcll(bal);
   }
-  if (tid < 64) {
-    const int R = (p.P + 15) >> 4;
-    bool live = false;
-    uint32_t drop = 0xffffu;
-    if (lane < R) {
-      const int p0 = lane * 16;
-      const uint32_t word = (maskw[p0 >> 5] >> (p0 & 31)) & 0xffffu;
-      const int valid = min(16, p.P - p0);
-      const uint32_t vmask = valid >= 16 ? 0xffffu : ((1u << valid) - 1u);
-      drop = (word | ~vmask) & 0xffffu;
-      live = drop != 0xffffu;
-    }
-    const unsigned long long bal = __ballot(live);
-    const int rbase = STAGE == 2 ? 0 : base;
-    if (STAGE != 1 && live) units[rbase + __popcll(bal & ((1ull << lane) - 1ull))] = rep_unit(lane, drop);
-    if (lane == 0) {
-      *nunits = STAGE == 1 ? base : rbase + __popcll(bal);
-      *nexact = STAGE == 2 ? 0 : base;
-    }
+  wave_lds_fence();
+  const int R = (p.P + 15) >> 4;
+  bool live = false;
+  uint32_t drop = 0xffffu;
+  if (lane < R) {
+    const int p0 = lane * 16;
+    const uint32_t word = (maskw[p0 >> 5] >> (p0 & 31)) & 0xffffu;
+    const int valid = min(16, p.P - p0);
+    const uint32_t vmask = valid >= 16 ? 0xffffu : ((1u << valid) - 1u);
+    drop = (word | ~vmask) & 0xffffu;
+    live = drop != 0xffffu;
   }
+  const unsigned long long bal = __ballot(live);
+  const int rbase = STAGE == 2 ? 0 : base;
+  if (STAGE != 1 && live) units[rbase + __popcll(bal & ((1ull << lane) - 1ull))] = rep_unit(lane, drop);
+  wave_lds_fence();
+  return UnitCounts{STAGE == 1 ? base : rbase + (int)__popcll(bal), STAGE == 2 ? 0 : base};
 }
 
 // NB query blocks per workgroup (4 waves each).  NB = 1: the general call
@@ -514,11 +522,10 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   // rows one unit ahead.  Iteration i reads K slot (i+1)&1 and V slot i&1
   // while the loads of K unit i+2 and V unit i+1 land in the other slots.
   __shared__ alignas(16) uint8_t ring[4 * kBuf];   // K slot 0 | K slot 1 | V slot 0 | V slot 1
-  __shared__ int units[kMaxCount + kMaxRepTiles];
-  __shared__ uint32_t maskw[16];
+  __shared__ int units[NB == 1 ? kMaxCount + kMaxRepTiles : 1];
+  __shared__ uint32_t maskw[4][16];
   __shared__ float xm[NB][2][64], xl[NB][2][64];
-  __shared__ int nunits_s, nexact_s, wcount[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 #ifdef SSA_ATTN_STAMPS
   __shared__ unsigned long long stl[4][kAStampRec];
   auto stamp = [&](int slot, unsigned long long v) {
@@ -546,7 +553,15 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   const int h = work / TB, t = (work % TB) * NB + grp;
   // the table entries first: the unit list waits for them alone, not for
   // the query rows requested after them
-  const int first = NB == 1 ? lut_entry(p, h, t, tid) : -1;
+  int lut[kLutRows];
+  if (NB == 1) {
+    const int32_t* row = p.ids + ((long long)h * p.T + t) * p.C;
+#pragma unroll
+    for (int j = 0; j < kLutRows; ++j) {
+      lut[j] = -1;
+      if (64 * j < p.C && 64 * j + lane < p.C) lut[j] = row[64 * j + lane];
+    }
+  }
   // query operand: lane's query row, dims 16*st + 8*hh + [0,8); its latency
   // overlaps the unit list
   const int r = lane & 31, hh = lane >> 5;
@@ -555,16 +570,19 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   const uint16_t* qp = p.q + qrow * p.q_tok + (long long)h * p.q_head + 8 * hh;
 #pragma unroll
   for (int st = 0; st < 8; ++st) qop[st] = ldg16(qp + 16 * st);
-  if (NB == 1) {
-    own_units<STAGE>(p, h, t, tid, first, units, maskw, wcount, &nunits_s, &nexact_s);
-  } else {
-    // every page exact, no rep tiles: units are the pages in order
-    for (int i = tid; i < p.P; i += kThreads * NB) units[i] = i;
-    if (tid == 0) nunits_s = nexact_s = p.P;
-  }
-  __syncthreads();
+  const UnitOffsets page_off = unit_offsets(wave, lane, p.kv_tok, 63, NB, true);
+  const RepOffsets rep_off = rep_offsets(wave, lane, NB);
+  const UnitSources src = unit_sources(p, h);
+  // this lane's detail operand rows (rank r % 8 of its half's 12 pairs) in a
+  // rep tile's V slot
+  const uint32_t det_off = kDetailOff + ((pair * 2 + hh) * 8 + (r & 7)) * 32;
+  const uint32_t klane = k_base(pair, lane), vlane = v_base(pair, lane);
+  // two-block calls: every page exact, no rep tiles, units are the pages in
+  // order
+  UnitCounts count{p.P, p.P};
+  if constexpr (NB == 1) count = own_units<STAGE>(p, lane, lut, units, maskw[wave]);
   ATTN_TICK(1);
-  const int nunits = __builtin_amdgcn_readfirstlane(nunits_s);
+  const int nunits = __builtin_amdgcn_readfirstlane(count.nunits);
   // the piece state's slot: tile (work - split_from) of the split ones, or
   // every tile in a staged call
   const long long pslot = (long long)(((work - (STAGE ? 0 : p.split_from)) * nparts + piece) * NB + grp) * kPieceFloats;
@@ -593,19 +611,16 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   float ls = 0.f;
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) O[dt] = f32x16{};
-  const UnitOffsets page_off = unit_offsets(wave, lane, p.kv_tok, 63, NB, true);
-  const RepOffsets rep_off = rep_offsets(wave, lane, NB);
-  const UnitSources src = unit_sources(p, h);
-  // this lane's detail operand rows (rank r % 8 of its half's 12 pairs) in a
-  // rep tile's V slot
-  const uint32_t det_off = kDetailOff + ((pair * 2 + hh) * 8 + (r & 7)) * 32;
-  const uint32_t klane = k_base(pair, lane), vlane = v_base(pair, lane);
-  auto unit = [&](int i) { return __builtin_amdgcn_readfirstlane(units[i]); };
+  auto raw_unit = [&](int i) { return NB == 1 ? units[i] : i; };
+  auto unit = [&](int i) { return __builtin_amdgcn_readfirstlane(raw_unit(i)); };
   // prologue: K and V of unit ibeg, K of unit ibeg+1 in flight (unit i in
   // slots i & 1); S of unit ibeg and its max
   issue_rows<NB>(p, src, unit(ibeg), 0, wave, lane, page_off, rep_off, kslot(ibeg & 1));
   issue_rows<NB>(p, src, unit(ibeg), 1, wave, lane, page_off, rep_off, vslot(ibeg & 1));
   issue_rows<NB>(p, src, unit(min(ibeg + 1, iend - 1)), 0, wave, lane, page_off, rep_off, kslot((ibeg + 1) & 1));
+  // the loads of unit ibeg's K have landed when no more than the later ones
+  // are left (a wave issues 4 / NB of its K rows, as many of a page's V rows,
+  // fewer of a rep tile's)
   wait_loads();
   __syncthreads();
   f32x16 S0 = s_tile(kslot(ibeg & 1), pair, lane, qop), S1;
@@ -617,7 +632,7 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   // Unit ids run ahead in registers (u0 = unit i); the id of unit i+3 is
   // read from LDS in step i-1, so the read completes at its barrier.
   int u0 = unit(ibeg), u1 = unit(min(ibeg + 1, iend - 1)), u2 = unit(min(ibeg + 2, iend - 1));
-  int u3raw = units[min(ibeg + 3, iend - 1)];
+  int u3raw = raw_unit(min(ibeg + 3, iend - 1));
 
   // P.V of exact page i (probabilities of Sc, V slot cur), with S(i+1) from
   // the other K slot and its max.  K: the kind of units i+1 and i+2.
@@ -873,7 +888,7 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
     u0 = u1;
     u1 = u2;
     u2 = u3;
-    u3raw = units[min(i + 4, iend - 1)];
+    u3raw = raw_unit(min(i + 4, iend - 1));
     wait_loads();
     ATTN_TICK(10 + 3 * (i - ibeg));
     __syncthreads();
@@ -886,7 +901,7 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   using AnyUnits = std::integral_constant<int, 2>;
   using Even = std::integral_constant<int, 0>;
   using Odd = std::integral_constant<int, 1>;
-  const int npages = nexact_s;
+  const int npages = __builtin_amdgcn_readfirstlane(count.nexact);
   int i = ibeg;
   for (; i + 2 < iend && i + 3 < npages; i += 2) {
     step(PageUnits{}, PageUnits{}, Even{}, i, S0, S1);
@@ -1057,6 +1072,17 @@ __global__ __launch_bounds__(64) void merge_kernel(const float* part, uint16_t* 
   const int h = work / TB, t = (work % TB) * NB + g;
   const float* const base = part + ((long long)(s / NB) * pieces * NB + g) * kPieceFloats;
   auto piece = [&](int j) { return base + (long long)j * (NB * kPieceFloats); };
+  constexpr int kAhead = MAXP < kMergeAhead ? MAXP : kMergeAhead;
+  f32x4 v[kAhead][4];
+  auto load = [&](int j0) {
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      // past the last piece: re-read it, its weight is zero
+      const float* sj = piece(min(j0 + j, pieces - 1)) + ((qw * 16 + dt * 4) * 64 + lane) * 4;
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) v[j][jj] = *reinterpret_cast<const f32x4*>(sj + jj * 256);
+    }
+  };
   float w[MAXP], lj[MAXP];
 #pragma unroll
   for (int j = 0; j < MAXP; ++j) {
@@ -1078,18 +1104,10 @@ __global__ __launch_bounds__(64) void merge_kernel(const float* part, uint16_t* 
     L += lj[j] * w[j];
   }
   f32x4 acc[4] = {};
-  constexpr int kAhead = MAXP < kMergeAhead ? MAXP : kMergeAhead;
 #pragma unroll
   for (int j0 = 0; j0 < MAXP; j0 += kAhead) {
     if (j0 >= pieces) break;
-    f32x4 v[kAhead][4];
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) {
-      // past the last piece: re-read it, its weight is zero
-      const float* sj = piece(min(j0 + j, pieces - 1)) + ((qw * 16 + dt * 4) * 64 + lane) * 4;
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) v[j][jj] = *reinterpret_cast<const f32x4*>(sj + jj * 256);
-    }
+    load(j0);
 #pragma unroll
     for (int j = 0; j < kAhead; ++j)
 #pragma unroll

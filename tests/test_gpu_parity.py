@@ -685,6 +685,35 @@ def test_attention_many_pieces(device, heads, blocks, pages, count, pieces):
         check_out(out[:, rows], want[:, rows], f"{heads}x{blocks} tiles, {pieces} pieces, single={single}")
 
 
+@pytest.mark.parametrize("pages,count", [(65, 1), (97, 63), (98, 64), (120, 65), (300, 129), (512, 448), (512, 512)])
+def test_attention_list_lengths(device, pages, count):
+    """Tables around the 64 entries that a wave reads at once, up to the longest:
+    scattered -1 padding, a page listed twice, and in the last block the first
+    page alone; within the bar of the oracle, staged or in one launch."""
+    gen = torch.Generator().manual_seed(pages + count)
+    heads, blocks = 1, 3
+    n = 64 * blocks
+    q = torch.randn(1, n, heads, 128, generator=gen).bfloat16()
+    k = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    v = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    vp = v[0].transpose(0, 1).reshape(heads, pages, 64, 128)
+    basis = workload.pca_basis(vp.float())
+    s = workload.kmeans_summaries(k[0].transpose(0, 1).reshape(heads, pages, 64, 128), vp, basis,
+                                  torch.Generator().manual_seed(9))
+    gd = Summary(*(getattr(s, f).to(device) for f in Summary.FIELDS))
+    ids = torch.stack([torch.randperm(pages, generator=gen)[:count] for _ in range(blocks)]).int()[None].contiguous()
+    ids[0, 1][torch.rand(count, generator=gen) < 0.4] = -1
+    ids[0, 1, -1] = ids[0, 1, 0] = 5
+    ids[0, 2] = -1
+    ids[0, 2, count // 2] = 0
+    want = ref.selected_attention(q, k, v, s, basis, ids).bfloat16()
+    args = (q.to(device), k.to(device), v.to(device), gd, basis.to(device), ids.to(device))
+    for single in (False, True):
+        for staged in (False, True):
+            out = attention(*args, Workspace(), single_av=single, staged=staged)
+            check_out(out, want, f"{pages} pages, {count} listed, single={single}, staged={staged}")
+
+
 @pytest.mark.parametrize("heads,blocks,pages,pieces", [(1, 2, 7, 1), (1, 6, 70, 16), (2, 22, 60, 11), (8, 72, 24, 6),
                                                        (12, 72, 290, 4)])
 def test_dense_many_pieces(device, heads, blocks, pages, pieces):
