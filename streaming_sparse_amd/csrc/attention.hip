@@ -524,7 +524,7 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   __shared__ alignas(16) uint8_t ring[4 * kBuf];   // K slot 0 | K slot 1 | V slot 0 | V slot 1
   __shared__ int units[NB == 1 ? kMaxCount + kMaxRepTiles : 1];
   __shared__ uint32_t maskw[4][16];
-  __shared__ float xm[NB][2][64], xl[NB][2][64];
+  __shared__ float xm[NB][2][2][64], xl[NB][2][2][64];   // [group][pair][query half][lane]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 #ifdef SSA_ATTN_STAMPS
   __shared__ unsigned long long stl[4][kAStampRec];
@@ -586,21 +586,19 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   // the piece state's slot: tile (work - split_from) of the split ones, or
   // every tile in a staged call
   const long long pslot = (long long)(((work - (STAGE ? 0 : p.split_from)) * nparts + piece) * NB + grp) * kPieceFloats;
-  if (STAGE != 0 && nunits == 0) {
-    // no unit of this stage (a table that selects every page, or lists none
-    // in the window): the empty state m = -inf, l = 0, O = 0
-    for (int i = tid; i < kPieceFloats; i += kThreads) p.part[pslot + i] = i >= 8192 && i < 8256 ? -INFINITY : 0.0f;
-    return;
-  }
   // this workgroup's units [ibeg, iend): a piece of the list when split,
   // starting at an even unit (so the slot of every step stays known at
-  // compile time).  A piece left empty (a list shorter than the pieces)
-  // walks unit ibeg and hands on an empty state instead (m = -inf, l = 0,
-  // O = 0).
+  // compile time)
   const int ibeg = STAGE ? 0 : 2 * (nunits * piece / (2 * nparts));
-  const int inext = (STAGE || piece + 1 == nparts) ? nunits : 2 * (nunits * (piece + 1) / (2 * nparts));
-  const bool empty = inext <= ibeg;
-  const int iend = empty ? ibeg + 1 : inext;
+  const int iend = (STAGE || piece + 1 == nparts) ? nunits : 2 * (nunits * (piece + 1) / (2 * nparts));
+  if (nparts > 1 && iend <= ibeg) {
+    // no unit of this piece (a list shorter than the pieces) or stage (a
+    // table that selects every page, or lists none in the window): the empty
+    // state m = -inf, l = 0, O = 0
+    float* const st = p.part + pslot;
+    for (int i = tid & (kThreads - 1); i < kPieceFloats; i += kThreads) st[i] = i >= 8192 && i < 8256 ? -INFINITY : 0.0f;
+    return;
+  }
   lds_u8* const kbase = (lds_u8*)ring;
   lds_u8* const vbase = (lds_u8*)ring + 2 * kBuf;
   auto kslot = [&](int slot) { return kbase + slot * kBuf; };
@@ -974,7 +972,7 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   }
   ATTN_TICK(4);
   __syncthreads();
-  // merge the two key halves: pair 1 hands (m, l, O) to pair 0 through LDS.
+  // merge the two key halves through LDS: (m, l) and half of O each way.
   // Lanes l and l ^ 32 hold the fp32 partial sums of one query's two 16-key
   // halves (ls).
   float l = 0.0f;
@@ -982,16 +980,22 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
     const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ls), __float_as_uint(ls), false, false);
     l += __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
-  // [group][qw][64 items][64 lanes] fp32 = 32 KB per group
-  float* xo = reinterpret_cast<float*>(ring) + grp * 8192;
-  if (pair == 1) {
-    float* d = xo + qw * 4096 + lane;
+  // Each pair finishes two of the four dim tiles and hands the other two to
+  // the other pair: [group][qw][pair][32 items][64 lanes] fp32, 32 KB per
+  // group.  All four waves so share the last sums and stores, which are
+  // bound by latency; nothing in them depends on a run-time choice per
+  // element (a test for an empty piece in each one waited for every LDS read
+  // by itself: 2.4 us of a piece's 17 us at 48 tiles of 66 units).  24 tiles
+  // of 36 units 17.2 -> 15.7 us, 48 of 66 25.6 -> 24.3, 185 of 83 62.3 -> 60.8.
+  float* const xo = reinterpret_cast<float*>(ring) + grp * 8192 + qw * 4096;
+  {
+    float* d = xo + pair * 2048 + lane;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int e = 0; e < 2; ++e)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) d[(16 * dt + i) * 64] = O[dt][i];
-    xm[grp][qw][lane] = rm.m;
-    xl[grp][qw][lane] = l;
+      for (int i = 0; i < 16; ++i) d[(16 * e + i) * 64] = pair == 0 ? O[2 + e][i] : O[e][i];
+    xm[grp][pair][qw][lane] = rm.m;
+    xl[grp][pair][qw][lane] = l;
   }
   __syncthreads();
 #ifdef SSA_ATTN_STAMPS
@@ -1004,49 +1008,50 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
       attn_stamps[((long long)blockIdx.x * 4 + wave) * kAStampRec + k] = stl[wave & 3][k];
   }
 #endif
-  if (pair == 1) return;
-  const float m1 = xm[grp][qw][lane], l1 = xl[grp][qw][lane];
+  const float m1 = xm[grp][pair ^ 1][qw][lane], l1 = xl[grp][pair ^ 1][qw][lane];
   const float m = rm.m;
   const float mt = fmaxf(m, m1);
   const float mu = mt == -INFINITY ? 0.0f : mt;
   const float a0 = __builtin_amdgcn_exp2f(m - mu), a1 = __builtin_amdgcn_exp2f(m1 - mu);
   const float lt = l * a0 + l1 * a1;
-  const float* d = xo + qw * 4096 + lane;
+  f32x16 R[2];     // dims 32 (2 pair + e) .. + 31 of both key halves
+  {
+    const float* d = xo + (pair ^ 1) * 2048 + lane;
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) R[e][i] = (pair == 0 ? O[e][i] : O[2 + e][i]) * a0 + d[(16 * e + i) * 64] * a1;
+  }
   // the lane's query, dim half and query half, re-formed here so that no
   // register holds them across the unit loop
   int lq = tid;
   asm volatile("" : "+v"(lq));
-  const int rq = lq & 31, hq = (lq >> 5) & 1, qq = (lq >> 6) & 1;
+  const int rq = lq & 31, hq = (lq >> 5) & 1;
   if (nparts > 1) {
     // a piece: its unnormalised state (the two key halves merged) for
     // merge_kernel, in this epilogue's lane layout
-    float* slot = p.part + pslot;
+    float* st = p.part + pslot;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int e = 0; e < 2; ++e)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        f32x4 po;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) po[c] = empty ? 0.0f : O[dt][4 * j + c] * a0 + d[(16 * dt + 4 * j + c) * 64] * a1;
-        *reinterpret_cast<f32x4*>(slot + ((qq * 16 + dt * 4 + j) * 64 + lq % 64) * 4) = po;
-      }
-    if (hq == 0) {
-      slot[8192 + qq * 32 + rq] = empty ? -INFINITY : mu;
-      slot[8256 + qq * 32 + rq] = empty ? 0.0f : lt;
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<f32x4*>(st + ((qw * 16 + (2 * pair + e) * 4 + j) * 64 + lq % 64) * 4) =
+            f32x4{R[e][4 * j], R[e][4 * j + 1], R[e][4 * j + 2], R[e][4 * j + 3]};
+    if (pair == 0 && hq == 0) {
+      st[8192 + qw * 32 + rq] = mu;
+      st[8256 + qw * 32 + rq] = lt;
     }
     return;
   }
   const float inv = 1.0f / lt;
-  uint16_t* op = p.out + (long long)(t * 64 + qq * 32 + rq) * p.q_tok + (long long)h * p.q_head + 4 * hq;
+  uint16_t* op = p.out + (long long)(t * 64 + qw * 32 + rq) * p.q_tok + (long long)h * p.q_head + 64 * pair + 4 * hq;
 #pragma unroll
-  for (int dt = 0; dt < 4; ++dt) {
+  for (int e = 0; e < 2; ++e) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      float o[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) o[c] = (O[dt][4 * j + c] * a0 + d[(16 * dt + 4 * j + c) * 64] * a1) * inv;
-      const u32x2 w = {pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
-      *reinterpret_cast<u32x2*>(op + 32 * dt + 8 * j) = w;
+      const u32x2 w = {pack_bf16(R[e][4 * j] * inv, R[e][4 * j + 1] * inv),
+                       pack_bf16(R[e][4 * j + 2] * inv, R[e][4 * j + 3] * inv)};
+      *reinterpret_cast<u32x2*>(op + 32 * e + 8 * j) = w;
     }
   }
 }
