@@ -1060,73 +1060,54 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
 // split tile s (tile g = s % NB of workgroup split_from + s / NB) for queries
 // 32 qw .. 32 qw + 31 and dims 32 dt .. 32 dt + 31 (O = sum_j O_j 2^(m_j - M),
 // l likewise, M = max_j m_j, in piece order) and writes out = O / l.  Lane l
-// holds the epilogue's lane layout.  Bound by the latency of its loads: the
-// m and l of every piece are requested together, then the O of kMergeAhead
-// pieces at a time, and a tile spreads over 8 waves.  MAXP: the most pieces
-// an instance takes.
+// holds the epilogue's lane layout; wave jj takes its item jj of every piece.
+// Bound by the latency of its loads, so all of them -- m, l and one 16-byte
+// item of each piece per lane -- go out before the first use.  A wave per
+// block with four items of four pieces at a time, m and l ahead of them, took
+// two to four latencies: 9 pieces of 24 tiles 15.6 -> 14.9 us a call, 3 of 144
+// 32.7 -> 32.3.  MAXP: the most pieces an instance takes.
 constexpr int kMaxPieces = 16;
-constexpr int kMergeAhead = 4;
 
 template <int NB, int MAXP>
-__global__ __launch_bounds__(64) void merge_kernel(const float* part, uint16_t* out, int split_from, int pieces,
-                                                   int T, long long q_tok, long long q_head) {
-  const int lane = threadIdx.x, s = blockIdx.x >> 3, qw = (blockIdx.x >> 2) & 1, dt = blockIdx.x & 3;
+__global__ __launch_bounds__(kThreads) void merge_kernel(const float* part, uint16_t* out, int split_from, int pieces,
+                                                         int T, long long q_tok, long long q_head) {
+  const int lane = threadIdx.x & 63, jj = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int s = blockIdx.x >> 3, qw = (blockIdx.x >> 2) & 1, dt = blockIdx.x & 3;
   const int r = lane & 31, hh = lane >> 5;
-  const int TB = T / NB, g = s % NB;
-  const int work = split_from + s / NB;
-  const int h = work / TB, t = (work % TB) * NB + g;
+  const int g = s % NB;
   const float* const base = part + ((long long)(s / NB) * pieces * NB + g) * kPieceFloats;
   auto piece = [&](int j) { return base + (long long)j * (NB * kPieceFloats); };
-  constexpr int kAhead = MAXP < kMergeAhead ? MAXP : kMergeAhead;
-  f32x4 v[kAhead][4];
-  auto load = [&](int j0) {
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) {
-      // past the last piece: re-read it, its weight is zero
-      const float* sj = piece(min(j0 + j, pieces - 1)) + ((qw * 16 + dt * 4) * 64 + lane) * 4;
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) v[j][jj] = *reinterpret_cast<const f32x4*>(sj + jj * 256);
-    }
-  };
   float w[MAXP], lj[MAXP];
+  f32x4 v[MAXP];
 #pragma unroll
   for (int j = 0; j < MAXP; ++j) {
     // a uniform branch: the loads of all pieces go out before the first use
     w[j] = -INFINITY;
     lj[j] = 0.0f;
+    v[j] = f32x4{};
     if (j < pieces) {
       w[j] = piece(j)[8192 + qw * 32 + r];
       lj[j] = piece(j)[8256 + qw * 32 + r];
+      v[j] = *reinterpret_cast<const f32x4*>(piece(j) + ((qw * 16 + dt * 4 + jj) * 64 + lane) * 4);
     }
   }
+  const int TB = T / NB, work = split_from + s / NB;
+  const int h = work / TB, t = (work % TB) * NB + g;
   float M = w[0];
 #pragma unroll
   for (int j = 1; j < MAXP; ++j) M = fmaxf(M, w[j]);
   float L = 0.0f;
+  f32x4 acc = {};
 #pragma unroll
   for (int j = 0; j < MAXP; ++j) {
     w[j] = __builtin_amdgcn_exp2f(w[j] - M);
     L += lj[j] * w[j];
-  }
-  f32x4 acc[4] = {};
 #pragma unroll
-  for (int j0 = 0; j0 < MAXP; j0 += kAhead) {
-    if (j0 >= pieces) break;
-    load(j0);
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j)
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[jj][c] += v[j][jj][c] * w[j0 + j];
+    for (int c = 0; c < 4; ++c) acc[c] += v[j][c] * w[j];
   }
   const float inv = 1.0f / L;
-  uint16_t* op = out + (long long)(t * 64 + qw * 32 + r) * q_tok + (long long)h * q_head + 4 * hh;
-#pragma unroll
-  for (int jj = 0; jj < 4; ++jj) {
-    const u32x2 o = {pack_bf16(acc[jj][0] * inv, acc[jj][1] * inv), pack_bf16(acc[jj][2] * inv, acc[jj][3] * inv)};
-    *reinterpret_cast<u32x2*>(op + 32 * dt + 8 * jj) = o;
-  }
+  uint16_t* op = out + (long long)(t * 64 + qw * 32 + r) * q_tok + (long long)h * q_head + 32 * dt + 8 * jj + 4 * hh;
+  *reinterpret_cast<u32x2*>(op) = u32x2{pack_bf16(acc[0] * inv, acc[1] * inv), pack_bf16(acc[2] * inv, acc[3] * inv)};
 }
 
 // Detail operand tiles of one head per block row: rops[h, rt] for the
@@ -1141,13 +1122,16 @@ __global__ __launch_bounds__(kRepOpChunks) void rep_operands_kernel(const uint16
 // Merges `pieces` pieces of each of `tiles` split tiles (NB per workgroup).
 template <int NB>
 void launch_merge(const AttnParams& p, int tiles, int split_from, int pieces, hipStream_t stream) {
-  const dim3 grid(8 * tiles), block(64);
+  const dim3 grid(8 * tiles), block(kThreads);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, p.part, p.out, split_from, pieces, p.T, p.q_tok, p.q_head);
+  };
   if (pieces <= 2)
-    hipLaunchKernelGGL((merge_kernel<NB, 2>), grid, block, 0, stream, p.part, p.out, split_from, pieces, p.T, p.q_tok,
-                       p.q_head);
+    launch(merge_kernel<NB, 2>);
+  else if (pieces <= 4)
+    launch(merge_kernel<NB, 4>);
   else
-    hipLaunchKernelGGL((merge_kernel<NB, kMaxPieces>), grid, block, 0, stream, p.part, p.out, split_from, pieces, p.T,
-                       p.q_tok, p.q_head);
+    launch(merge_kernel<NB, kMaxPieces>);
 }
 
 // The split a call runs: the workgroups past the last multiple of the CU
