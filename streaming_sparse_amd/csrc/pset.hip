@@ -871,7 +871,9 @@ struct ScoreSmem {
 // so a lane scores 4 pairs per probe, its sums in registers.  Bound by the
 // chain of dependent steps per probe, two probes per wave at two waves per
 // SIMD.  3 heads x 72 blocks, kernel trace: 48 us (all 512 pairs, three fp64
-// products per pair and dim, four probes per wave) -> 27 us.
+// products per pair and dim, four probes per wave) -> 27 us; with its LDS reads
+// in groups (a read behind a write or a lane's condition waited for itself) the
+// correction call went from 147.7 to 145.5 us.
 __global__ __launch_bounds__(kScoreThreads) void pset_scores_kernel(PsetParams p) {
   __shared__ ScoreSmem s;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -990,24 +992,26 @@ __global__ __launch_bounds__(kScoreThreads) void pset_scores_kernel(PsetParams p
     // per candidate: endpoint vector, its E . V and its share of the swap
     // denominator (leave-one-out sums over the other candidates of its group)
     if (lane < kCand) {
-      double ev = 0.0;
+      double ev = 0.0, x[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const double x = D * (c[2 + e] - s.Hs[w][e]) + EX * rp_of(c, e);
-        s.V[w][e][lane] = x;
-        ev = fma(s.Hs[w][16 + e], x, ev);
+        x[e] = D * (c[2 + e] - s.Hs[w][e]) + EX * rp_of(c, e);
+        ev = fma(s.Hs[w][16 + e], x[e], ev);
       }
+      // written once all is read: reads stay behind the writes before them
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s.V[w][e][lane] = x[e];
       s.EV[w][lane] = ev;
+      // every entry is read and the lane's own left out of the sum: a read
+      // under a condition of the lane waits for itself
+      const int g0 = lane < 16 ? 0 : 16, gn = lane < 16 ? 16 : 32, col = lane < 16 ? 0 : 1;
+      double others[32];
+#pragma unroll
+      for (int k = 0; k < 32; ++k) others[k] = s.ex[w][min(g0 + k, kCand - 1)][col];
       double loo = 0.0;
-      if (lane < 16) {
 #pragma unroll
-        for (int k = 0; k < 16; ++k) loo += k != lane ? s.ex[w][k][0] : 0.0;
-        s.S[w][lane] = B + loo + LM;
-      } else {
-#pragma unroll
-        for (int k = 16; k < kCand; ++k) loo += k != lane ? s.ex[w][k][1] : 0.0;
-        s.S[w][lane] = loo + EX;
-      }
+      for (int k = 0; k < 32; ++k) loo += k < gn && g0 + k != lane ? others[k] : 0.0;
+      s.S[w][lane] = lane < 16 ? B + loo + LM : loo + EX;
     }
     wave_fence();
     uint32_t badmask = 0u;
