@@ -72,6 +72,7 @@ struct AttnParams {
   // split_from = H * T / NB: no split.
   float* part;
   int split_from, split_k;
+  int split_inv;               // ceil(2^20 / split_k)
 };
 
 // Per piece of a split tile: O [qw][dt * 4 + j][64 lanes][4] fp32 (the
@@ -546,22 +547,28 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
     work = xcd_remap(blockIdx.x, p.split_from);
   } else {
     const int b = blockIdx.x - p.split_from;
-    work = p.split_from + b / p.split_k;
-    piece = b % p.split_k;
+    // b / split_k, and below list lengths / (2 split_k), by the multiplied
+    // inverse: exact for b < 4096 and 544 units in up to kMaxPieces pieces
+    const int w = b * p.split_inv >> 20;
+    work = p.split_from + w;
+    piece = b - w * p.split_k;
     nparts = p.split_k;
   }
-  const int h = work / TB, t = (work % TB) * NB + grp;
-  // the table entries first: the unit list waits for them alone, not for
-  // the query rows requested after them
+  // the table entries first (a tile's table row is its index): the unit list
+  // waits for them alone, not for the query rows requested after them.  No
+  // division stands before their request or after the list (four of them did:
+  // 24 tiles of 36 units 15.0 -> 14.9 us, 144 of 45 32.6 -> 32.4, 185 of 83
+  // 61.9 -> 61.4, captured).
   int lut[kLutRows];
   if (NB == 1) {
-    const int32_t* row = p.ids + ((long long)h * p.T + t) * p.C;
+    const int32_t* row = p.ids + (long long)work * p.C;
 #pragma unroll
     for (int j = 0; j < kLutRows; ++j) {
       lut[j] = -1;
       if (64 * j < p.C && 64 * j + lane < p.C) lut[j] = row[64 * j + lane];
     }
   }
+  const int h = work / TB, t = (work % TB) * NB + grp;
   // query operand: lane's query row, dims 16*st + 8*hh + [0,8); its latency
   // overlaps the unit list
   const int r = lane & 31, hh = lane >> 5;
@@ -589,8 +596,9 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   // this workgroup's units [ibeg, iend): a piece of the list when split,
   // starting at an even unit (so the slot of every step stays known at
   // compile time)
-  const int ibeg = STAGE ? 0 : 2 * (nunits * piece / (2 * nparts));
-  const int iend = (STAGE || piece + 1 == nparts) ? nunits : 2 * (nunits * (piece + 1) / (2 * nparts));
+  auto bound = [&](int pc) { return 2 * (nunits * pc * p.split_inv >> 21); };     // 2 (nunits pc / (2 nparts))
+  const int ibeg = STAGE || piece == 0 ? 0 : bound(piece);
+  const int iend = STAGE || piece + 1 == nparts ? nunits : bound(piece + 1);
   if (nparts > 1 && iend <= ibeg) {
     // no unit of this piece (a list shorter than the pieces) or stage (a
     // table that selects every page, or lists none in the window): the empty
@@ -1284,6 +1292,7 @@ int ssa_attention(const void* q, const void* k, const void* v, const void* keys,
   p.part = nullptr;
   p.split_from = wgs;
   p.split_k = 1;
+  p.split_inv = 1 << 20;
   // with a workspace of ssa_attention_workspace_bytes, the workgroups past
   // the last multiple of the CU count run as pieces, merged by merge_kernel
   int r = 0, pieces = 1;
@@ -1308,6 +1317,7 @@ int ssa_attention(const void* q, const void* k, const void* v, const void* keys,
     p.part = (float*)workspace;
     p.split_from = wgs - r;
     p.split_k = pieces;
+    p.split_inv = ((1 << 20) + pieces - 1) / pieces;
   }
   const dim3 grid(p.split_from + (wgs - p.split_from) * p.split_k);
   if (dense) {
