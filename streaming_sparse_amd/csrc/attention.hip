@@ -1148,35 +1148,44 @@ void launch_merge(const AttnParams& p, int tiles, int split_from, int pieces, hi
 // workspace bytes.
 //
 // The chip holds `slots` workgroups at once (the general call two per CU, the
-// two-block call one).  The last round holds wgs mod slots of them; where
-// that leaves a whole CU's worth of work the first `cus` run whole.  k is the
-// most pieces that still start together: a piece that waits for a slot costs
-// its prologue, its state (33 KB) and a second latency-bound walk.  Measured
-// (captured in a graph; W workgroups, units each; k = 1, 2 and the rule's):
-// general W 24 x 36: 31.5, 24.7, 16.6 us (k 9); W 48 x 91: 70.9, 45.9, 28.4
-// (k 10, with 11: 37.0); W 144 x 46: 39.3, 40.0, 34.3 (k 3, with 4: 44.0);
-// W 288 x 91: 105.2, 92.6, 89.5 (k 8); W 432 x 46: 64.3 (the rule's k 1),
-// 76.8; W 504 x 91: 132.0 (k 1), 142.0; W 576 x 91: 192.3, 164.9, 158.4;
-// W 864 x 91: 241.7, 227.7 (k 2), with 3: 235.8.  Two-block W 22 x 308:
-// 217.0, 117.4, 41.4 (k 11, with 12: 60.9); W 216 x 432: 378.4 (k 1), 391.7;
-// W 432 x 72: 135.4 (k 1), 152.2, with 4: 148.5.
-// Pieces hold at least kMinUnits units (W 24 x 36: 2 units each 20.8 us, 4
-// units 16.6).
-constexpr int kMinUnits = 4;
-
+// two-block call one), and the last round holds wgs mod slots of them.  A
+// piece costs its start, its state (33 KB) and its share of the merge, and one
+// that waits for a slot a second latency-bound walk, so k is never more than
+// start together; and two pieces on a CU are little faster than one, so where
+// one piece per CU already cuts a list in three, or in two after a full round,
+// k is cus / r.  Otherwise it is the most that start together.  Measured
+// (captured in a graph, us; W workgroups of U units; k = 1, the rule's, and
+// the other side of the line):
+// general  W 24 U 36 31.2, 14.3 (k 10);  W 24 U 66 -, 17.0 (10), 20.8 (two per
+// CU: 16);  W 30 U 73 -, 17.6 (8), 22.4 (16);  W 48 U 91 71.0, 25.2 (5), 26.5
+// (10);  W 60 U 63 -, 22.7 (4), 26.0 (8);  W 72 U 46 -, 22.6 (3), 25.4 (7), but
+// single-term U 91 30.4 and 29.8;  W 100 U 64 -, 33.2 (5), 34.5 (one per CU:
+// 2);  W 120 U 91 -, 43.3 (4), 45.7 (2);  W 144 U 46 38.5, 31.0 (3), 39.9 (4);
+// W 288 U 91 104.1, 86.9 (8), 104.2 (15);  W 432 U 46 63.3 (1), 71.9 (2);
+// W 504 U 91 128.1 (1), 135.6 (2);  W 544 U 46 -, 76.6 (8), 84.0 (two per CU:
+// 16);  W 576 U 91 187.4, 147.2 (4), 154.5 (8);  W 608 U 46 98.8, 87.5 (2),
+// 88.8 (5);  W 648 U 64 136.1, 125.0 (3);  W 864 U 91 234.4, 219.7 (2), 224.5
+// (3).
+// two-block  W 22 U 308 210.2, 38.2 (11), 55.9 (12);  W 216 U 432 358.3 (1),
+// 370.1 (2);  W 288 U 288 463.8, 312.6 (8);  W 432 U 72 130.4 (1), 144.8 (2),
+// 141.0 (4).
+// Pieces hold at least min_units units: general W 24 U 36 14.9 (4 units), 14.3
+// (3), 16.1 (12 pieces, which no longer start alone); W 12 U 36 12.7, 11.9;
+// W 4 U 35 12.3, 11.4.
 int split_plan(int wgs, int nb, int units, int* split_wgs, int* k, long long* bytes) {
   int cus = 0;
   const int e = device_cus(&cus);
   if (e != (int)hipSuccess) return e;
-  const int slots = nb == 1 ? 2 * cus : cus;
+  const int slots = nb == 1 ? 2 * cus : cus, min_units = nb == 1 ? 3 : 4;
   const int last = wgs % slots, r = wgs % cus;
   int pieces = 1;
   if (r > 0) {
-    pieces = (last >= cus ? slots - cus : slots) / r;
-    pieces = std::min(std::min(pieces, kMaxPieces), std::max(1, units / kMinUnits));
+    const int alone = cus / r;
+    pieces = alone >= (wgs > slots ? 2 : 3) ? alone : (last >= cus ? slots - cus : slots) / r;
+    pieces = std::min(std::min(pieces, kMaxPieces), std::max(1, units / min_units));
     // a long two-block list whose last round fills at most 3/4 of the CUs:
-    // its quarters run in three quarter rounds (W 432: 432 units 750.7 ->
-    // 741.0 us, 72 units 135.4 -> 148.5)
+    // its quarters run in three quarter rounds (W 432: 432 units 714.4 ->
+    // 702.3 us, 72 units 130.4 -> 141.0)
     if (nb == 2 && pieces == 1 && 4 * r <= 3 * cus && units >= 288) pieces = 4;
   }
   *split_wgs = pieces > 1 ? r : 0;

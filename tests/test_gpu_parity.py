@@ -641,11 +641,14 @@ def test_attention_split_short_lists(device):
 
 
 @pytest.mark.parametrize("heads,blocks,pages,count,pieces", [
-    (1, 1, 40, 9, 3),       # 12 units at most: pieces of kMinUnits = 4
+    (1, 1, 40, 9, 4),       # 12 units at most: pieces of at least 3
     (1, 3, 290, 61, 16),    # 80 units: the most pieces a merge takes, five units each
-    (1, 23, 97, 20, 6),     # an odd window: 27 units, pieces of 4 and 6
+    (1, 23, 97, 20, 9),     # an odd window: 27 units, pieces of 2 and 4
+    (1, 72, 100, 14, 3),    # one piece per CU
+    (2, 50, 100, 14, 5),    # two per CU, where one would leave two pieces
     (3, 57, 100, 14, 2),    # 171 tiles: two pieces each
-    (2, 150, 96, 12, 4),    # 300 tiles: the 44 past the CU count, bounded by their units
+    (2, 150, 96, 12, 5),    # 300 tiles: the 44 past the CU count
+    (4, 152, 96, 12, 2),    # 608 tiles: after a full round one piece per CU
 ])
 def test_attention_many_pieces(device, heads, blocks, pages, count, pieces):
     """Calls that leave CUs idle split every tile into the pieces that start
