@@ -1153,7 +1153,9 @@ void launch_merge(const AttnParams& p, int tiles, int split_from, int pieces, hi
 // that waits for a slot a second latency-bound walk, so k is never more than
 // start together; and two pieces on a CU are little faster than one, so where
 // one piece per CU already cuts a list in three, or in two after a full round,
-// k is cus / r.  Otherwise it is the most that start together.  Measured
+// k is cus / r.  Otherwise it is the most that start together, and no more
+// than kBesideWhole where whole workgroups run in the same round: they set its
+// length, and each piece slows one of them.  Measured
 // (captured in a graph, us; W workgroups of U units; k = 1, the rule's, and
 // the other side of the line):
 // general  W 24 U 36 31.2, 14.3 (k 10);  W 24 U 66 -, 17.0 (10), 20.8 (two per
@@ -1161,7 +1163,10 @@ void launch_merge(const AttnParams& p, int tiles, int split_from, int pieces, hi
 // (10);  W 60 U 63 -, 22.7 (4), 26.0 (8);  W 72 U 46 -, 22.6 (3), 25.4 (7), but
 // single-term U 91 30.4 and 29.8;  W 100 U 64 -, 33.2 (5), 34.5 (one per CU:
 // 2);  W 120 U 91 -, 43.3 (4), 45.7 (2);  W 144 U 46 38.5, 31.0 (3), 39.9 (4);
-// W 288 U 91 104.1, 86.9 (8), 104.2 (15);  W 432 U 46 63.3 (1), 71.9 (2);
+// W 264 U 46 54.1, 46.0 (4), 45.9 (8);  W 264 U 91 100.9, 83.4 (4), 82.5 (8);
+// W 282 U 34 (single-term) 38.3, 32.8 (4), 34.3 (9);  W 288 U 46 55.4, 48.5
+// (4), 49.3 (8);  W 288 U 91 (single-term) 78.1, 71.1 (4), 72.6 (8);  W 300 U
+// 46 56.8, 50.3 (4), 51.3 (5);  W 432 U 46 63.3 (1), 71.9 (2);
 // W 504 U 91 128.1 (1), 135.6 (2);  W 544 U 46 -, 76.6 (8), 84.0 (two per CU:
 // 16);  W 576 U 91 187.4, 147.2 (4), 154.5 (8);  W 608 U 46 98.8, 87.5 (2),
 // 88.8 (5);  W 648 U 64 136.1, 125.0 (3);  W 864 U 91 234.4, 219.7 (2), 224.5
@@ -1172,6 +1177,8 @@ void launch_merge(const AttnParams& p, int tiles, int split_from, int pieces, hi
 // Pieces hold at least min_units units: general W 24 U 36 14.9 (4 units), 14.3
 // (3), 16.1 (12 pieces, which no longer start alone); W 12 U 36 12.7, 11.9;
 // W 4 U 35 12.3, 11.4.
+constexpr int kBesideWhole = 4;
+
 int split_plan(int wgs, int nb, int units, int* split_wgs, int* k, long long* bytes) {
   int cus = 0;
   const int e = device_cus(&cus);
@@ -1182,6 +1189,7 @@ int split_plan(int wgs, int nb, int units, int* split_wgs, int* k, long long* by
   if (r > 0) {
     const int alone = cus / r;
     pieces = alone >= (wgs > slots ? 2 : 3) ? alone : (last >= cus ? slots - cus : slots) / r;
+    if (last >= cus) pieces = std::min(pieces, kBesideWhole);
     pieces = std::min(std::min(pieces, kMaxPieces), std::max(1, units / min_units));
     // a long two-block list whose last round fills at most 3/4 of the CUs:
     // its quarters run in three quarter rounds (W 432: 432 units 714.4 ->

@@ -647,7 +647,7 @@ def test_attention_split_short_lists(device):
     (1, 72, 100, 14, 3),    # one piece per CU
     (2, 50, 100, 14, 5),    # two per CU, where one would leave two pieces
     (3, 57, 100, 14, 2),    # 171 tiles: two pieces each
-    (2, 150, 96, 12, 5),    # 300 tiles: the 44 past the CU count
+    (2, 150, 96, 12, 4),    # 300 tiles: the 44 past the CU count, beside whole ones
     (4, 152, 96, 12, 2),    # 608 tiles: after a full round one piece per CU
 ])
 def test_attention_many_pieces(device, heads, blocks, pages, count, pieces):
