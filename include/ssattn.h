@@ -90,11 +90,11 @@ int ssa_rep_operands(const void* detail, void* rep_ops, int heads, int pages, in
  * not matter), the stand-in for the reference's Workspace
  * (VR/attention.py:7-13).  With it, the
  * workgroups past the last multiple of the device's compute-unit count run
- * as pieces of their unit lists (two per (query block, head) tile in a
- * general call, four per two-block workgroup in a dense one), so the last
- * round spreads over every CU, and a second kernel merges the pieces'
- * states into out; NULL (or too small): every workgroup in one piece.  Results agree within the
- * call's tolerance, not bit for bit, between the two; each is
+ * as pieces of their unit lists, no more than start together with the last
+ * round's other workgroups (at most 16, of at least 3 units each; none where
+ * fewer than two would), and a second kernel merges the pieces' states into
+ * out; NULL (or too small): every workgroup in one piece.  Results agree
+ * within the call's tolerance, not bit for bit, between the two; each is
  * deterministic.  Calls that share a workspace must not overlap (one
  * stream, or ordered). */
 int ssa_attention(const void* q, const void* k, const void* v, const void* keys, const void* mean, const void* basis,
@@ -273,8 +273,9 @@ int ssa_encode_layers(int layers, const void* const* keys, const void* const* me
  * the best legal same-partition swap is applied to mask [H,blocks,pages]
  * (0/1 bytes) iff its gain > 0 and every legal score is finite, and the row
  * of ids [H,blocks,count] is rebuilt (own first, then descending risk).
- * Caller-owned scratch: cand n_heads*blocks*16*48*34 fp64, rows
- * n_heads*blocks*16*2*52 fp64, pool n_heads*blocks*64 int32.  Per-row outputs:
+ * Caller-owned scratch: cand n_heads*blocks*16*48*34 fp64 (candidate data
+ * and the background's partial sums), rows n_heads*blocks*16*2*52 fp64 (not
+ * written), pool n_heads*blocks*64 int32.  Per-row outputs:
  * gain [n_heads,blocks] fp64, info [n_heads,blocks,3] int32 = (executed, best
  * pair index remove*32+add, non-finite legal scores); scores
  * [n_heads,blocks,16,32] fp64 (illegal pairs -1e30) or NULL; stats [3]

@@ -21,8 +21,8 @@ COEF_STRIDE = 128      # bf16 per page: co[85] | 0 x 11 | A[32]
 COEF_A = 96
 CAND = 48
 CAND_VALS = 34
-ROW_VALS = 52
-ROW_SPLIT = 2          # page ranges per pair of query blocks in the rows kernel
+ROW_VALS = 52          # the ABI's row scratch (the kernels keep their partial sums behind the candidates)
+ROW_SPLIT = 2
 POOL_INTS = 64
 
 
