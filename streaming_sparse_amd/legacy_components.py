@@ -131,7 +131,7 @@ def attention(q, k, v, s, basis, ids, workspace, *, bf16_av=True, single_av=None
     has them (route(..., rep_out=...) writes them on the side); otherwise
     they are computed here.  ``split=False`` runs every tile in one piece
     (no split workspace; the tiles past the last multiple of the CU count
-    otherwise run as two pieces each).  ``staged=True`` runs the exact pages
+    otherwise run as pieces, two or more each).  ``staged=True`` runs the exact pages
     and the compensation as two launches whose states a merge kernel
     combines (the reference's exact kernel + tail + merge), so a profiler
     shows the two stages apart; not with ``all_pages``."""
