@@ -516,7 +516,9 @@ __device__ __forceinline__ UnitCounts own_units(const AttnParams& p, int lane, c
 // exact pages, then the compensation's rep tiles -- each leaving its state
 // in part[2 tile + STAGE - 1] for merge_kernel, the reference's split into
 // an exact kernel, a tail and a merge (RV/tuned_attention.py:20-81).
-template <bool PRECISE, int NB, int STAGE = 0>
+// SPREAD: a page step's loads go out between its first products instead of
+// ahead of them (always so in the two-block call).
+template <bool PRECISE, int NB, int STAGE = 0, bool SPREAD = NB == 2>
 __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams p) {
   static_assert(STAGE == 0 || NB == 1, "staged calls are general calls");
   // LDS ring: K rows of units i (slot i & 1) run two units ahead of use, V
@@ -671,8 +673,8 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
 #pragma unroll
       for (int st = 0; st < 8; ++st) {
         Sn = mfma32(ka[st], qop[st], Sn);
-        if (NB == 2 && st == 0) issue_rows<NB, K>(p, src, u2, 0, wave, lane, page_off, rep_off, kslot(cur));
-        if (NB == 2 && st == 3) issue_rows<NB, K>(p, src, u1, 1, wave, lane, page_off, rep_off, vslot(cur ^ 1));
+        if (SPREAD && st == 0) issue_rows<NB, K>(p, src, u2, 0, wave, lane, page_off, rep_off, kslot(cur));
+        if (SPREAD && st == 3) issue_rows<NB, K>(p, src, u1, 1, wave, lane, page_off, rep_off, vslot(cur ^ 1));
         if (st < 4)
           ka[st + 4] = k_read(kb, kl, st + 4);
         else
@@ -727,8 +729,8 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
 #pragma unroll
       for (int st = 0; st < 8; ++st) {
         Sn = mfma32(ka[st], qop[st], Sn);
-        if (NB == 2 && st == 0) issue_rows<NB, K>(p, src, u2, 0, wave, lane, page_off, rep_off, kslot(cur));
-        if (NB == 2 && st == 3) issue_rows<NB, K>(p, src, u1, 1, wave, lane, page_off, rep_off, vslot(cur ^ 1));
+        if (SPREAD && st == 0) issue_rows<NB, K>(p, src, u2, 0, wave, lane, page_off, rep_off, kslot(cur));
+        if (SPREAD && st == 3) issue_rows<NB, K>(p, src, u1, 1, wave, lane, page_off, rep_off, vslot(cur ^ 1));
         if (st < 4)
           ka[st + 4] = k_read(kb, kl, st + 4);
         else
@@ -877,9 +879,8 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
     constexpr int cur = decltype(parity)::value;   // i & 1: every paired loop keeps i even
     const int u3 = __builtin_amdgcn_readfirstlane(u3raw);
     ATTN_TICK(8 + 3 * (i - ibeg));
-    // the general call issues its loads first; the two-block call (8 waves,
-    // half the loads each) spreads them over the first products
-    if (NB == 1) {
+    // loads first; with SPREAD a page step sends them between its products
+    if (!SPREAD || (NB == 1 && KP == 1)) {
       issue_rows<NB, K>(p, src, u2, 0, wave, lane, page_off, rep_off, kslot(cur));
       issue_rows<NB, K>(p, src, u1, 1, wave, lane, page_off, rep_off, vslot(cur ^ 1));
     }
@@ -1202,6 +1203,20 @@ int split_plan(int wgs, int nb, int units, int* split_wgs, int* k, long long* by
   return (int)hipSuccess;
 }
 
+// Whether a two-term general call spreads its page steps' loads over their
+// products: where a full round of two workgroups per CU runs, the loads' eight
+// instructions ahead of the products hold the matrix pipe up for the other
+// workgroup too; with fewer, getting them out first counts for more.  Measured
+// (captured, us; loads first, spread):  W 144 U 46 32.4, 32.9;  W 185 U 83 60.7,
+// 61.2;  W 432 U 46 64.0, 64.1;  W 504 U 91 129.0, 128.9;  W 576 U 64 107.7,
+// 106.9;  W 640 U 71 128.4, 127.5;  W 720 U 91 189.6, 188.4;  W 864 U 46 116.6,
+// 115.3;  W 864 U 91 219.5, 216.6.  Single-term calls gain 0.5% at W 864 and
+// lose 1 to 2% at W 504 and 768, so they keep the loads first.
+bool spread_loads(int wgs) {
+  int cus = 0;
+  return device_cus(&cus) == (int)hipSuccess && wgs >= 2 * cus;
+}
+
 // Flag bits of ssa_attention.
 constexpr int kTwoTerm = 1, kDense = 2, kStaged = 4;
 
@@ -1344,7 +1359,9 @@ int ssa_attention(const void* q, const void* k, const void* v, const void* keys,
       hipLaunchKernelGGL((attn_kernel<false, 2>), grid, dim3(2 * kThreads), 0, stream, p);
     if (p.split_k > 1) launch_merge<2>(p, 2 * (wgs - p.split_from), p.split_from, p.split_k, stream);
   } else {
-    if (flags & kTwoTerm)
+    if ((flags & kTwoTerm) && spread_loads(wgs))
+      hipLaunchKernelGGL((attn_kernel<true, 1, 0, true>), grid, dim3(kThreads), 0, stream, p);
+    else if (flags & kTwoTerm)
       hipLaunchKernelGGL((attn_kernel<true, 1>), grid, dim3(kThreads), 0, stream, p);
     else
       hipLaunchKernelGGL((attn_kernel<false, 1>), grid, dim3(kThreads), 0, stream, p);

@@ -774,6 +774,34 @@ def test_attention_split_boundary(device, blocks):
     check_out(out[:, rows], want[:, rows], f"{blocks} tiles")
 
 
+@pytest.mark.parametrize("pages,count", [(96, 1), (97, 15), (130, 65)])
+def test_attention_full_round(device, pages, count):
+    """512 tiles fill two workgroups on each of 256 CUs and take the kernel
+    whose page steps send their loads between the products, 511 tiles the one
+    that sends them first: the same values bit for bit (every tile runs whole
+    in both), with one, an odd and an even number of exact pages, -1 padding
+    and a window that ends inside a rep tile."""
+    gen = torch.Generator().manual_seed(pages)
+    q = torch.randn(1, 64 * 512, 1, 128, generator=gen).bfloat16().to(device)
+    k = torch.randn(1, 64 * pages, 1, 128, generator=gen).bfloat16()
+    v = torch.randn(1, 64 * pages, 1, 128, generator=gen).bfloat16()
+    vp = v[0].transpose(0, 1).reshape(1, pages, 64, 128)
+    basis = workload.pca_basis(vp.float())
+    s = workload.kmeans_summaries(k[0].transpose(0, 1).reshape(1, pages, 64, 128), vp, basis,
+                                  torch.Generator().manual_seed(8))
+    gd = Summary(*(getattr(s, f).to(device) for f in Summary.FIELDS))
+    ids = torch.stack([torch.randperm(pages, generator=gen)[:count] for _ in range(512)])[None].int()
+    ids[:, 5::7, count // 2 + 1:] = -1
+    args = (k.to(device), v.to(device), gd, basis.to(device))
+    a = attention(q, *args, ids.to(device), Workspace())
+    b = attention(q[:, :64 * 511].contiguous(), *args, ids[:, :511].contiguous().to(device), Workspace())
+    assert torch.equal(a[:, :64 * 511].view(torch.int16), b.view(torch.int16))
+    tiles = [0, 5, 510]
+    want = ref.selected_attention(q.cpu(), k, v, s, basis, ids, tiles=tiles).bfloat16()
+    rows = torch.cat([torch.arange(t * 64, (t + 1) * 64) for t in tiles])
+    check_out(a[:, rows.to(device)], want[:, rows], f"512 tiles, {count} of {pages} pages")
+
+
 @pytest.mark.parametrize("single", [False, True])
 def test_attention_staged(device, single):
     """A staged call (the exact pages of every tile in one launch, the
