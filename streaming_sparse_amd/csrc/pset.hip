@@ -587,10 +587,14 @@ __device__ __forceinline__ Const<T>* scalar(const T* p) {
 // which the scores kernel completes with the candidates.  Bound by vector
 // issue: ~440 fp32 and fp64 instructions per page and 64 probes, the fp64 ones
 // at half rate (with the page data always in the scalar cache the kernel is
-// 12% faster).  432 pages, 3 heads x 72 blocks, kernel trace: 94 us (32 probes
+// 12% faster).  The scalar cache reads whole 4-byte words and drops the low
+// bits of an address, so coefficients that start between two words (a view at
+// an odd element; the encode kernel writes those too) take the instance
+// without WORDS, which reads them one by one.  432 pages, 3 heads x 72 blocks, kernel trace: 94 us (32 probes
 // per wave, page data broadcast from LDS, three accumulated mixtures, 369
 // registers at one wave per SIMD) -> 54 us; the trace runs below the load
 // clock.
+template <bool WORDS>
 __global__ __launch_bounds__(64 * kRowWaves, 2) void pset_rows_kernel(PsetParams p) {
   __shared__ RowsSmem s;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -683,10 +687,17 @@ __global__ __launch_bounds__(64 * kRowWaves, 2) void pset_rows_kernel(PsetParams
   // one page, its 4 rep logits of this lane's probe in z
   auto page_step = [&](int page, const float (&zr)[4]) {
     const long long pe = (long long)h * p.EP + page;
-    Const<uint32_t>* cw = scalar(reinterpret_cast<const uint32_t*>(p.coef + pe * kCoefStride));
+    const uint16_t* const cf = p.coef + pe * kCoefStride;
     Const<double>* mb = scalar(p.mean_b + pe * 16);
     Const<double>* db = scalar(p.detail_b + pe * 48);
-    auto coef = [&](int i) { return i & 1 ? bf16_hi(cw[i >> 1]) : bf16_lo(cw[i >> 1]); };
+    auto coef = [&](int i) {
+      if constexpr (WORDS) {
+        const uint32_t w = scalar(reinterpret_cast<const uint32_t*>(cf))[i >> 1];
+        return i & 1 ? bf16_hi(w) : bf16_lo(w);
+      } else {
+        return bf16_to_f32(cf[i]);
+      }
+    };
     // rep softmax of the page (fp32), page log mass in fp64
     float z[4], w[4];
 #pragma unroll
@@ -1306,7 +1317,11 @@ int pset_launch(const void* q, long long q_head_stride, long long q_block_stride
   p.C = count;
   const int groups = (blocks + kRowBlocks - 1) / kRowBlocks;
   hipLaunchKernelGGL(pset_pool_kernel, dim3(n_heads * blocks), dim3(kMaxPages), 0, stream, p);
-  hipLaunchKernelGGL(pset_rows_kernel, dim3(n_heads * groups * kSplit), dim3(64 * kRowWaves), 0, stream, p);
+  const dim3 rows_grid(n_heads * groups * kSplit), rows_block(64 * kRowWaves);
+  if (((uintptr_t)coef & 3) == 0)
+    hipLaunchKernelGGL(pset_rows_kernel<true>, rows_grid, rows_block, 0, stream, p);
+  else
+    hipLaunchKernelGGL(pset_rows_kernel<false>, rows_grid, rows_block, 0, stream, p);
   hipLaunchKernelGGL(pset_scores_kernel, dim3(n_heads * blocks), dim3(kScoreThreads), 0, stream, p);
   return (int)hipGetLastError();
 }

@@ -338,3 +338,32 @@ def test_pset_ragged_groups_match_oracle(device, blocks, pages):
     ex_g = rows['executed'].cpu().bool()
     assert bool(((ex_g == orow['executed']) & (~ex_g | (rows['argmax'].cpu().long() == orow['argmax'])) | ties).all())
     assert bool(((mask.cpu()[scoped] == want_mask[scoped]).all(-1) | ties).all())
+
+
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_pset_coefficients_between_words(device, offset):
+    """Encodings whose bf16 coefficients start 2, 4 or 6 bytes past a word
+    boundary of their storage (views of one flat buffer), encoded and
+    corrected there: scores, tables and the swap count equal those of aligned
+    ones bit for bit."""
+    x, w, _, _ = inputs(9)
+    heads, pages, n = 2, 130, 30
+    s = type(x.summary)(*(getattr(x.summary, f)[:heads, :pages].contiguous().to(device) for f in x.summary.FIELDS))
+    q = x.q[:, -64 * 5:, :heads].contiguous().to(device)
+    reader = pset.Reader(w, device)
+    lse = torch.empty(heads, 5, 16, device=device)
+
+    def corrected(enc):
+        pset.encode(s, x.basis[:heads].to(device), reader, out=enc)
+        ids, mask, risk, _ = route(q, s, x.theta[:heads].to(device), tier='intersection', n=n, lse_out=lse,
+                                   current_slots=torch.full((heads,), 24, dtype=torch.int32))
+        stats, rows = pset.correct(q, s, enc, reader, risk, lse, mask, ids, None, [0, 1], want_scores=True)
+        return ids, mask, rows['scores'], stats
+
+    want = corrected(pset.Encoding.empty(heads, pages, device))
+    assert int(want[3][0]) > 0
+    e = pset.Encoding.empty(heads, pages, device)
+    flat = torch.zeros(e.coef.numel() + 4, device=device, dtype=torch.bfloat16)
+    e.coef = flat[offset:offset + e.coef.numel()].view(e.coef.shape)
+    for got, ref_v in zip(corrected(e), want):
+        assert torch.equal(got, ref_v)
