@@ -89,13 +89,12 @@ def ptrs(tensors):
 
 def stream_handle(device=None):
     """The current stream of `device` (default: the current device), as an
-    int.  A device with an index is asked for its raw stream directly: the
+    int.  A torch.device with an index is asked for its raw stream directly: the
     Stream object that torch.cuda.current_stream makes costs more than a
     kernel launch."""
-    index = getattr(device, 'index', None)
-    if index is None:
-        return torch.cuda.current_stream(device).cuda_stream
-    return _raw_stream(index)
+    if isinstance(device, torch.device) and device.index is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def check(status: int, name: str):

@@ -274,3 +274,17 @@ def test_batch_graphs_checks_call_shape():
     bg.current_slots = torch.full((H,), 10)
     with pytest.raises(ValueError):                                  # Full_Pset without reader / encoding
         bg.get(torch.zeros(H, 72, 64, D), s, None, torch.ones(H, 4), None, None, True, [3])
+
+
+@pytest.mark.parametrize("device,handle", [(torch.device("cuda:1"), 101), (torch.device("cuda"), 7), ("cuda:1", 7),
+                                           ("cuda", 7), (0, 7), (None, 7)])
+def test_stream_handle_takes_every_device_form(monkeypatch, device, handle):
+    """A torch.device with an index is asked for its raw stream; a name, an
+    index or no device goes to torch.cuda.current_stream, as it is."""
+    from streaming_sparse_amd import _lib
+    asked = []
+    monkeypatch.setattr(_lib, "_raw_stream", lambda i: 100 + i)
+    monkeypatch.setattr(torch.cuda, "current_stream",
+                        lambda d=None: asked.append(d) or type("Stream", (), {"cuda_stream": 7}))
+    assert _lib.stream_handle(device) == handle
+    assert asked == ([device] if handle == 7 else [])
