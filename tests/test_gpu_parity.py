@@ -802,6 +802,38 @@ def test_attention_full_round(device, pages, count):
     check_out(a[:, rows.to(device)], want[:, rows], f"512 tiles, {count} of {pages} pages")
 
 
+@pytest.mark.parametrize("heads,blocks", [(1, 1), (1, 7), (1, 9), (3, 141)])
+def test_ragged_grids_cover_every_tile(device, heads, blocks):
+    """Grids of no multiple of eight workgroups (8 XCDs): risk, table and every
+    output row equal, bit for bit, those of the same blocks padded to a multiple of
+    eight (more blocks of the same queries)."""
+    pages, count = 40, 9
+    gen = torch.Generator().manual_seed(blocks)
+    more = -(-blocks // 16) * 16
+    q = torch.randn(1, 64 * more, heads, 128, generator=gen).bfloat16().to(device)
+    k = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    v = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    vp = v[0].transpose(0, 1).reshape(heads, pages, 64, 128)
+    basis = workload.pca_basis(vp.float())
+    s = workload.kmeans_summaries(k[0].transpose(0, 1).reshape(heads, pages, 64, 128), vp, basis,
+                                  torch.Generator().manual_seed(9))
+    gd = Summary(*(getattr(s, f).to(device) for f in Summary.FIELDS))
+    theta = torch.tensor([1.0, 1.0, 1.0, 0.5], device=device).expand(heads, 4).contiguous()
+    own = (torch.arange(more, device=device) % pages).int().expand(heads, -1).contiguous()
+    kv = (k.to(device), v.to(device), gd, basis.to(device))
+    got = []
+    for n in (blocks, more):
+        qn, on = q[:, :64 * n].contiguous(), own[:, :n].contiguous()
+        ids, mask, risk, _ = route(qn, gd, theta, tier='topk', own=on)
+        ids = torch.stack([(on + i * 7) % pages for i in range(count)], -1).int().contiguous()
+        out = attention(qn, *kv, ids, Workspace(), split=False)
+        got.append((risk.clone(), mask.clone(), out.clone()))
+    torch.cuda.synchronize()
+    for a, b in zip(got[0][:2], got[1][:2]):
+        assert torch.equal(a, b[:, :blocks])
+    assert torch.equal(got[0][2].view(torch.int16), got[1][2][:, :64 * blocks].view(torch.int16))
+
+
 @pytest.mark.parametrize("single", [False, True])
 def test_attention_staged(device, single):
     """A staged call (the exact pages of every tile in one launch, the

@@ -281,7 +281,6 @@ def test_batch_graphs_checks_call_shape():
 def test_stream_handle_takes_every_device_form(monkeypatch, device, handle):
     """A torch.device with an index is asked for its raw stream; a name, an
     index or no device goes to torch.cuda.current_stream, as it is."""
-    from streaming_sparse_amd import _lib
     asked = []
     monkeypatch.setattr(_lib, "_raw_stream", lambda i: 100 + i)
     monkeypatch.setattr(torch.cuda, "current_stream",
