@@ -73,6 +73,10 @@ struct AttnParams {
   float* part;
   int split_from, split_k;
   int split_inv;               // ceil(2^20 / split_k)
+  // Grid order of the pieces: 0: the pieces of a tile next to each other; else
+  // ceil(2^20 / split tiles): each XCD takes a contiguous range of the list
+  // piece 0 of every tile, piece 1 of every tile, ...
+  int group_inv;
 };
 
 // Per piece of a split tile: O [qw][dt * 4 + j][64 lanes][4] fp32 (the
@@ -548,12 +552,18 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   } else if ((int)blockIdx.x < p.split_from) {
     work = xcd_remap(blockIdx.x, p.split_from);
   } else {
-    const int b = blockIdx.x - p.split_from;
-    // b / split_k, and below list lengths / (2 split_k), by the multiplied
-    // inverse: exact for b < 4096 and 544 units in up to kMaxPieces pieces
-    const int w = b * p.split_inv >> 20;
-    work = p.split_from + w;
+    const int b = blockIdx.x - p.split_from, tiles = p.H * TB - p.split_from;
+    // b / split_k, b / tiles, and below list lengths / (2 split_k), by the
+    // multiplied inverse: exact for b < 4096 and 544 units in up to kMaxPieces
+    // pieces
+    int w = b * p.split_inv >> 20;
     piece = b - w * p.split_k;
+    if (p.group_inv) {
+      const int i = xcd_remap(b, tiles * p.split_k);
+      piece = i * p.group_inv >> 20;
+      w = i - piece * tiles;
+    }
+    work = p.split_from + w;
     nparts = p.split_k;
   }
   // the table entries first (a tile's table row is its index): the unit list
@@ -1217,6 +1227,17 @@ bool spread_loads(int wgs) {
   return device_cus(&cus) == (int)hipSuccess && wgs >= 2 * cus;
 }
 
+// Whether a general call's pieces are grouped by XCD: where every tile lists
+// every page.  Tiles of a head then walk the same pages, and pieces of one
+// index the same part of them; in tile order each XCD gets every piece of every
+// head unless the pieces divide 8.  Short lists fit the L2s either way and
+// start sooner in tile order, and the tables of a sparse call share little
+// (captured, us, single-term; tile order, grouped; W tiles, U pages):  W 140 in 3
+// pieces U 32 33.0, 33.4;  U 40 36.2, 35.8;  U 72 56.4, 44.6;  U 300 164, 115;
+// W 105 in 4 U 32 30.3, 31.0;  U 48 34.2, 33.7;  W 245 in 2 U 40 63.4, 44.4;  W 852
+// U 300 580, 567;  sparse W 100 U 36 30.0, 31.7;  W 144 U 91 55.2, 56.2.
+bool group_pieces(int pages, int count) { return count == pages && pages >= 40; }
+
 // Flag bits of ssa_attention.
 constexpr int kTwoTerm = 1, kDense = 2, kStaged = 4;
 
@@ -1325,6 +1346,7 @@ int ssa_attention(const void* q, const void* k, const void* v, const void* keys,
   p.split_from = wgs;
   p.split_k = 1;
   p.split_inv = 1 << 20;
+  p.group_inv = 0;
   // with a workspace of ssa_attention_workspace_bytes, the workgroups past
   // the last multiple of the CU count run as pieces, merged by merge_kernel
   int r = 0, pieces = 1;
@@ -1350,6 +1372,7 @@ int ssa_attention(const void* q, const void* k, const void* v, const void* keys,
     p.split_from = wgs - r;
     p.split_k = pieces;
     p.split_inv = ((1 << 20) + pieces - 1) / pieces;
+    if (!dense && group_pieces(pages, count)) p.group_inv = ((1 << 20) + r - 1) / r;
   }
   const dim3 grid(p.split_from + (wgs - p.split_from) * p.split_k);
   if (dense) {

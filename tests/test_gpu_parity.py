@@ -749,6 +749,40 @@ def test_dense_many_pieces(device, heads, blocks, pages, pieces):
     check_out(out[:, rows], want, f"dense {heads}x{blocks} blocks, {pieces} pieces")
 
 
+@pytest.mark.parametrize("heads,blocks,pieces", [(1, 1, 16), (1, 27, 9), (4, 35, 3), (7, 35, 2), (9, 35, 4), (12, 71, 3)])
+@pytest.mark.parametrize("pages", [40, 67])
+def test_attention_grouped_pieces(device, heads, blocks, pieces, pages):
+    """Tables as long as the window are cut into pieces in another grid order
+    than shorter ones.  A table of every page but one and a -1 is the same
+    unit list as that table without the -1: equal outputs bit for bit, whatever
+    the order, in single- and two-term calls; and within the bar of the same
+    call run whole."""
+    from streaming_sparse_amd import _lib
+    gen = torch.Generator().manual_seed(heads * blocks)
+    n = 64 * blocks
+    q = torch.randn(1, n, heads, 128, generator=gen).bfloat16().to(device)
+    k = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    v = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    vp = v[0].transpose(0, 1).reshape(heads, pages, 64, 128)
+    basis = workload.pca_basis(vp.float())
+    s = workload.kmeans_summaries(k[0].transpose(0, 1).reshape(heads, pages, 64, 128), vp, basis,
+                                  torch.Generator().manual_seed(9))
+    gd = Summary(*(getattr(s, f).to(device) for f in Summary.FIELDS))
+    args = (q, k.to(device), v.to(device), gd, basis.to(device))
+    own = torch.arange(blocks, device=device) % pages
+    every = ((torch.arange(pages, device=device) + own[:, None]) % pages).int().expand(heads, -1, -1).contiguous()
+    every[..., -1] = -1
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        need = _lib.lib().ssa_attention_workspace_bytes(n, heads, pages, pages, 1)
+        assert need == heads * blocks % 256 * min(pieces, (pages + (pages + 15) // 16) // 3) * 33280
+    for single in (False, True):
+        a = attention(*args, every, Workspace(), single_av=single).clone()
+        b = attention(*args, every[..., :-1].contiguous(), Workspace(), single_av=single)
+        whole = attention(*args, every, Workspace(), single_av=single, split=False)
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+        assert ref.rel_l2(a.float().cpu(), whole.float().cpu()) <= (5e-3 if single else 1e-3)
+
+
 @pytest.mark.parametrize("blocks", [256, 257])
 def test_attention_split_boundary(device, blocks):
     """Tile counts at the CU-count boundary (256 CUs): 256 tiles run whole,
