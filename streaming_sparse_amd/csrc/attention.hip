@@ -1202,10 +1202,13 @@ int split_plan(int wgs, int nb, int units, int* split_wgs, int* k, long long* by
     pieces = alone >= (wgs > slots ? 2 : 3) ? alone : (last >= cus ? slots - cus : slots) / r;
     if (last >= cus) pieces = std::min(pieces, kBesideWhole);
     pieces = std::min(std::min(pieces, kMaxPieces), std::max(1, units / min_units));
-    // a long two-block list whose last round fills at most 3/4 of the CUs:
-    // its quarters run in three quarter rounds (W 432: 432 units 714.4 ->
-    // 702.3 us, 72 units 130.4 -> 141.0)
-    if (nb == 2 && pieces == 1 && 4 * r <= 3 * cus && units >= 288) pieces = 4;
+    // a long two-block list whose last round fills at most 3/4 of the CUs: its
+    // quarters run in three quarter rounds.  Whole and quarters, us: W 132 U 144
+    // 123.5, 122.1;  U 180 151.5, 143.3;  U 252 198.6, 185.4;  W 144 U 180 152.3,
+    // 144.1;  U 288 226.6, 206.3;  W 385 U 180 315.5, 311.3;  U 252 432.1, 413.3;
+    // W 432 U 144 259.0, 263.4;  U 180 320.5, 321.2;  U 216 379.7, 381.4;  U 252
+    // 438.2, 429.9;  U 288 505.3, 491.2;  U 432 742.5, 715.5.
+    if (nb == 2 && pieces == 1 && 4 * r <= 3 * cus && units >= 180) pieces = 4;
   }
   *split_wgs = pieces > 1 ? r : 0;
   *k = pieces;

@@ -718,11 +718,12 @@ def test_attention_list_lengths(device, pages, count):
 
 
 @pytest.mark.parametrize("heads,blocks,pages,pieces", [(1, 2, 7, 1), (1, 6, 70, 16), (2, 22, 60, 11), (8, 72, 24, 6),
-                                                       (12, 72, 290, 4)])
+                                                       (12, 72, 290, 4), (11, 24, 179, 1), (11, 24, 180, 4),
+                                                       (8, 36, 216, 4), (11, 70, 252, 4)])
 def test_dense_many_pieces(device, heads, blocks, pages, pieces):
     """The two-block kernel's pieces: a list too short to split, the most
-    pieces, one round of eleven, a tail bounded by its units, and the long
-    list whose tail runs in quarters; against dense attention on the first
+    pieces, one round of eleven, a tail bounded by its units, and long
+    lists, from 180 pages, whose tail of 129 to 192 workgroups runs in quarters; against dense attention on the first
     and last block, and against the same call run whole."""
     from streaming_sparse_amd import _lib
     gen = torch.Generator().manual_seed(heads * 100 + blocks)
