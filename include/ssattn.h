@@ -274,8 +274,8 @@ int ssa_encode_layers(int layers, const void* const* keys, const void* const* me
  * (0/1 bytes) iff its gain > 0 and every legal score is finite, and the row
  * of ids [H,blocks,count] is rebuilt (own first, then descending risk).
  * Caller-owned scratch: cand n_heads*blocks*16*48*34 fp64 (candidate data
- * and the background's partial sums), rows n_heads*blocks*16*2*52 fp64 (not
- * written), pool n_heads*blocks*64 int32.  Per-row outputs:
+ * and the background's partial sums), pool n_heads*blocks*64 int32; rows is
+ * neither read nor written and may be NULL.  Per-row outputs:
  * gain [n_heads,blocks] fp64, info [n_heads,blocks,3] int32 = (executed, best
  * pair index remove*32+add, non-finite legal scores); scores
  * [n_heads,blocks,16,32] fp64 (illegal pairs -1e30) or NULL; stats [3]
@@ -362,8 +362,8 @@ int ssa_group_order(const void* k, const void* v, long long layer_stride, long l
                     const int32_t* page_dst, int first_chunk, int layers, int heads, double* scratch_x,
                     int32_t* scratch_ids, int32_t* order, hipStream_t stream);
 
-/* ssa_pset without the caller-owned scratch (cand, rows, pool): the library
- * keeps that scratch in a file-scope device array of 48.05 MB per device
+/* ssa_pset without the caller-owned scratch (cand, pool): the library
+ * keeps that scratch in a file-scope device array of 45.18 MB per device
  * (held until the process ends), sized for n_heads * blocks <= 216 scoped rows
  * (3 heads x 72 query blocks); larger calls return hipErrorInvalidValue.
  * Allocates nothing (no hipMalloc, no allocating library routine); the first

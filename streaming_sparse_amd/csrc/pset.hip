@@ -337,7 +337,7 @@ struct PsetParams {
   const int32_t* own;
   const int32_t* heads;
   int HS;
-  double *cand, *rows;
+  double* cand;
   int32_t* pool;
   double* gain;
   int32_t* info;
@@ -537,8 +537,6 @@ constexpr int kRowWaves = 8;
 constexpr int kPartVals = 35;      // B[16], T[16], their masses sB and sT, max log mass
 constexpr int kPartAt = 16 * kCand * kCandStride;     // [kSplit][kPartVals][16 probes], in a row's scratch
 static_assert(kPartAt + kSplit * kPartVals * 16 <= kRowDoubles, "the partials fit behind the candidates");
-// the caller's row buffer (unused: the partials lie behind the candidates)
-constexpr int kRowsSplit = 2, kRowsVals = 52;
 
 struct RowsSmem {
   uint8_t sel[kRowBlocks][kMaxPages];
@@ -1272,8 +1270,8 @@ int pset_launch(const void* q, long long q_head_stride, long long q_block_stride
                 int gathered, const void* keys, int head_pages, const void* coef, const double* mean_b,
                 const double* detail_b, int enc_pages, const float* wq, const float* risk, const float* probe_lse,
                 uint8_t* mask, int32_t* ids, const int32_t* own, const int32_t* heads, int n_heads, double* cand,
-                double* rows, int32_t* pool, double* gain, int32_t* info, double* scores, long long* stats,
-                int total_heads, int blocks, int pages, int count, hipStream_t stream) {
+                int32_t* pool, double* gain, int32_t* info, double* scores, long long* stats, int total_heads,
+                int blocks, int pages, int count, hipStream_t stream) {
   // a 72-page window (the first chunk) or a window beyond the anchor frame
   // and the current chunk; any table size (an add slot past the spare pages
   // is an empty candidate)
@@ -1281,8 +1279,8 @@ int pset_launch(const void* q, long long q_head_stride, long long q_block_stride
   if (n_heads <= 0 || n_heads > total_heads || blocks <= 0 || pages > kMaxPages ||
       (!first && pages <= kAnchors + kCurrent) || head_pages < pages ||
       enc_pages < pages || count < (first ? kAnchors : 1) || count > pages ||
-      heads == nullptr || probe_lse == nullptr || cand == nullptr || rows == nullptr || pool == nullptr ||
-      gain == nullptr || info == nullptr || stats == nullptr)
+      heads == nullptr || probe_lse == nullptr || cand == nullptr || pool == nullptr || gain == nullptr ||
+      info == nullptr || stats == nullptr)
     return (int)hipErrorInvalidValue;
   PsetParams p;
   p.q = (const uint16_t*)q;
@@ -1305,7 +1303,6 @@ int pset_launch(const void* q, long long q_head_stride, long long q_block_stride
   p.heads = heads;
   p.HS = n_heads;
   p.cand = cand;
-  p.rows = rows;
   p.pool = pool;
   p.gain = gain;
   p.info = info;
@@ -1326,21 +1323,19 @@ int pset_launch(const void* q, long long q_head_stride, long long q_block_stride
   return (int)hipGetLastError();
 }
 
-// Scratch of the allocation-free entry point: for at most kScratchRows
-// scoped (head, query block) rows, the candidate endpoint data
-// [rows,16,48,34] fp64, then the split row partials [rows,16,2,52] fp64, then
-// the pools [rows,64] int32, each region at a fixed offset (48.05 MB in all).
+// Scratch of the allocation-free entry point: for at most kScratchRows scoped
+// (head, query block) rows, the candidate scratch [rows, kRowDoubles] fp64 (a
+// row's candidates, then its partials), then the pools [rows,64] int32, each
+// region at a fixed offset (45.18 MB in all).
 // Every entry a call reads is written earlier in the same call (the pool
 // kernel writes all 48 slots of each row, the rows kernel the candidates'
-// endpoint data and every row partial), so nothing in it must start at zero.
+// endpoint data and every partial), so nothing in it must start at zero.
 constexpr int kScratchRows = 216;   // 3 heads x 72 query blocks
-constexpr size_t kCandRowBytes = (size_t)16 * kCand * kCandVals * sizeof(double);
-constexpr size_t kRowsRowBytes = (size_t)16 * kRowsSplit * kRowsVals * sizeof(double);
+constexpr size_t kCandRowBytes = (size_t)kRowDoubles * sizeof(double);
 constexpr size_t kPoolRowBytes = (size_t)kPoolInts * sizeof(int32_t);
-constexpr size_t kScratchRowsOff = kScratchRows * kCandRowBytes;
-constexpr size_t kScratchPoolOff = kScratchRowsOff + kScratchRows * kRowsRowBytes;
+constexpr size_t kScratchPoolOff = kScratchRows * kCandRowBytes;
 constexpr size_t kScratchBytes = kScratchPoolOff + kScratchRows * kPoolRowBytes;
-static_assert(kCandRowBytes % 256 == 0 && kRowsRowBytes % 256 == 0, "regions stay 256-byte aligned");
+static_assert(kCandRowBytes % 256 == 0, "regions stay 256-byte aligned");
 
 }  // namespace
 
@@ -1380,9 +1375,10 @@ int ssa_pset(const void* q, long long q_head_stride, long long q_block_stride, l
              uint8_t* mask, int32_t* ids, const int32_t* own, const int32_t* heads, int n_heads, double* cand,
              double* rows, int32_t* pool, double* gain, int32_t* info, double* scores, long long* stats,
              int total_heads, int blocks, int pages, int count, hipStream_t stream) {
+  (void)rows;
   return pset_launch(q, q_head_stride, q_block_stride, q_row_stride, gathered, keys, head_pages, coef, mean_b,
-                     detail_b, enc_pages, wq, risk, probe_lse, mask, ids, own, heads, n_heads, cand, rows, pool, gain,
-                     info, scores, stats, total_heads, blocks, pages, count, stream);
+                     detail_b, enc_pages, wq, risk, probe_lse, mask, ids, own, heads, n_heads, cand, pool, gain, info,
+                     scores, stats, total_heads, blocks, pages, count, stream);
 }
 
 int ssa_pset_noalloc(const void* q, long long q_head_stride, long long q_block_stride, long long q_row_stride,
@@ -1397,8 +1393,8 @@ int ssa_pset_noalloc(const void* q, long long q_head_stride, long long q_block_s
   if (e != (int)hipSuccess) return e;
   return pset_launch(q, q_head_stride, q_block_stride, q_row_stride, gathered, keys, head_pages, coef, mean_b,
                      detail_b, enc_pages, wq, risk, probe_lse, mask, ids, own, heads, n_heads, (double*)base,
-                     (double*)(base + kScratchRowsOff), (int32_t*)(base + kScratchPoolOff), gain, info, scores,
-                     stats, total_heads, blocks, pages, count, stream);
+                     (int32_t*)(base + kScratchPoolOff), gain, info, scores, stats, total_heads, blocks, pages, count,
+                     stream);
 }
 
 }  // extern "C"

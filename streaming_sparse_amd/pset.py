@@ -21,8 +21,6 @@ COEF_STRIDE = 128      # bf16 per page: co[85] | 0 x 11 | A[32]
 COEF_A = 96
 CAND = 48
 CAND_VALS = 34
-ROW_VALS = 52          # the ABI's row scratch (the kernels keep their partial sums behind the candidates)
-ROW_SPLIT = 2
 POOL_INTS = 64
 
 
@@ -204,8 +202,7 @@ def correct(q, summary: Summary, encoding: Encoding, reader: Reader, risk, lse, 
         _lib.check(_lib.lib().ssa_pset_noalloc(*head, *tail), "ssa_pset_noalloc")
     else:
         cand = buf('cand', (n, t, 16, CAND, CAND_VALS), torch.float64)
-        rows = buf('rows', (n, t, 16, ROW_SPLIT, ROW_VALS), torch.float64)
         pool = buf('pool', (n, t, POOL_INTS), torch.int32)
-        _lib.check(_lib.lib().ssa_pset(*head, _lib.ptr(cand), _lib.ptr(rows), _lib.ptr(pool), *tail), "ssa_pset")
+        _lib.check(_lib.lib().ssa_pset(*head, _lib.ptr(cand), None, _lib.ptr(pool), *tail), "ssa_pset")
     return stats, dict(gain=gain, executed=info[..., 0], argmax=info[..., 1], nonfinite=info[..., 2],
                        scores=scores, pool=pool)
