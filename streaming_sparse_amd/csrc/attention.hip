@@ -93,8 +93,8 @@ constexpr int kPieceFloats = 2 * 16 * 64 * 4 + 2 * 64;
 // exchanged, 6 npages | nunits << 16 | ibeg << 32 | (end of the paired
 // steps) << 48, 7 HW_ID | XCC_ID << 32; then per paired step k (unit ibeg + k)
 // three stamps: step start (after the previous barrier), body and max update
-// done, loads waited for (before the barrier).  The product library compiles
-// the stamps out.
+// done, loads waited for (before the barrier).  A workgroup without units (an
+// empty piece) leaves zeros.  The product library compiles the stamps out.
 constexpr int kAStampWGs = 1024, kAStampSteps = 96, kAStampRec = 8 + 3 * kAStampSteps;
 #ifdef SSA_ATTN_STAMPS
 __device__ unsigned long long attn_stamps[kAStampWGs * 4 * kAStampRec];
@@ -617,6 +617,11 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
     // state m = -inf, l = 0, O = 0
     float* const st = p.part + pslot;
     for (int i = tid & (kThreads - 1); i < kPieceFloats; i += kThreads) st[i] = i >= 8192 && i < 8256 ? -INFINITY : 0.0f;
+#ifdef SSA_ATTN_STAMPS
+    // an empty record, not an earlier call's
+    if (NB == 1 && blockIdx.x < kAStampWGs)
+      for (int k = lane; k < kAStampRec; k += 64) attn_stamps[((long long)blockIdx.x * 4 + wave) * kAStampRec + k] = 0;
+#endif
     return;
   }
   lds_u8* const kbase = (lds_u8*)ring;

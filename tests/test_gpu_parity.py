@@ -750,7 +750,39 @@ def test_dense_many_pieces(device, heads, blocks, pages, pieces):
     check_out(out[:, rows], want, f"dense {heads}x{blocks} blocks, {pieces} pieces")
 
 
-@pytest.mark.parametrize("heads,blocks,pieces", [(1, 1, 16), (1, 27, 9), (4, 35, 3), (7, 35, 2), (9, 35, 4), (12, 71, 3)])
+def test_empty_pieces_leave_no_stamps(device):
+    """Measurement build: a piece without units records zeros, where an earlier
+    call's piece of the same workgroup had left its steps."""
+    import os
+    from streaming_sparse_amd import _lib, attn_steps, build
+    if not os.path.exists(build.STAMPS_LIB):
+        pytest.skip("libssattn_stamps.so not built")
+    pages, count = 40, 9
+    gen = torch.Generator().manual_seed(3)
+    q = torch.randn(1, 64, 1, 128, generator=gen).bfloat16().to(device)
+    kv = torch.randn(1, 64 * pages, 1, 128, generator=gen).bfloat16().to(device)
+    z = lambda *shape: torch.zeros(1, pages, *shape, device=device, dtype=torch.bfloat16)
+    s = Summary(z(4, 128), z(128), z(3, 8), z(4, 12))
+    basis = torch.zeros(1, 128, 8, device=device, dtype=torch.bfloat16)
+    product = _lib.lib()
+    try:
+        if _lib.use(build.STAMPS_LIB).ssa_attention_workspace_bytes(64, 1, pages, count, 1) != 4 * 33280:
+            pytest.skip("another compute unit count cuts the list differently")
+        for listed in (count, 1):       # 12 units, then 4: pieces [0, 0), [0, 2), [2, 2), [2, 4)
+            ids = torch.full((1, 1, count), -1, dtype=torch.int32, device=device)
+            ids[..., :listed] = torch.arange(listed, device=device)
+            attention(q, kv, kv, s, basis, ids, Workspace())
+            torch.cuda.synchronize()
+            st = attn_steps.read_stamps()[:4]
+            used = [bool((st[g, :, 0] != 0).all()) for g in range(4)]
+            assert used == ([True] * 4 if listed == count else [False, True, False, True])
+            assert all(used[g] or not st[g].any() for g in range(4))
+    finally:
+        _lib._lib = product
+
+
+@pytest.mark.parametrize("heads,blocks,pieces", [(1, 1, 16), (1, 27, 9), (4, 35, 3), (7, 35, 2), (9, 35, 4),
+                                                 (12, 71, 3)])
 @pytest.mark.parametrize("pages", [40, 67])
 def test_attention_grouped_pieces(device, heads, blocks, pieces, pages):
     """Tables as long as the window are cut into pieces in another grid order
