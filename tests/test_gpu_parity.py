@@ -78,8 +78,9 @@ def test_route_wide_and_narrow_workgroups(device, blocks, pages):
     """One head with a grid of at most one workgroup per CU (256 CUs: 512
     blocks) runs the router with 8 waves, 514 blocks with 4: windows that
     leave waves of either kind without a tile, end in a partial tile (of one
-    page, as a wave's first tile: 9, 57 and 25) or fill it, odd block counts; risk within 1e-4 of the float64 oracle and the
-    top-k table ranked by that risk, own first, ties to the lower page."""
+    page, as a wave's first tile: 9, 57 and 25) or fill it, odd block counts;
+    risk within 1e-4 of the float64 oracle and the top-k table ranked by that
+    risk, own first, ties to the lower page."""
     x = call_inputs(0, 9)
     sub = x.summary.slice(0, pages)
     s = Summary(*(getattr(sub, f)[:1].contiguous() for f in sub.FIELDS))
@@ -263,6 +264,49 @@ def test_route_writes_rep_operands(device, cfg, frames):
     a = attention(g.q, g.k, g.v, g.summary, basis, ids, ws).clone()
     b = attention(g.q, g.k, g.v, g.summary, basis, ids, ws, rep_ops=slab)
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("tier", ["base", "intersection"])
+@pytest.mark.parametrize("heads,blocks,pages", [(1, 1, 167), (2, 9, 425), (5, 72, 301), (7, 72, 300)])
+def test_wide_router_tiers_ties_and_operands(device, heads, blocks, pages, tier):
+    """Grids of at most one workgroup per CU (8 waves each), whose operand
+    tiles are written by blocks of twice the threads, up to a grid that they
+    take past the CU count (7 x 36 router workgroups and 17 more): tiles equal
+    to the standalone kernel's, those past the window untouched; tables,
+    masks and the near-tie report exactly those of the risk it returns, which
+    is within 1e-4 of the float64 oracle."""
+    from types import SimpleNamespace
+
+    from streaming_sparse_amd.legacy_components import rep_operands
+    x = call_inputs(1, 18)
+    s = Summary(*(getattr(x.summary, f)[:heads, :pages].contiguous() for f in Summary.FIELDS))
+    gs = Summary(*(getattr(s, f).to(device) for f in Summary.FIELDS))
+    q = x.q[:, -64 * blocks:, :heads].contiguous()
+    own = (torch.arange(blocks) + pages - blocks)[None].expand(heads, -1).contiguous()
+    tiles = (pages + 15) // 16
+    slab = torch.full((heads, tiles + 1, 512), float("nan"), device=device, dtype=torch.bfloat16)
+    want_ops = rep_operands(gs, pages, torch.empty(heads, tiles, 512, device=device, dtype=torch.bfloat16))
+    rows = torch.full((heads * blocks,), -1, dtype=torch.int32, device=device)
+    cnt = torch.full((1,), 12345, dtype=torch.int32, device=device)
+    a, n = torch.arange(heads) % 7 * 3 + 5, 41
+    kw = dict(current_slots=a.to(device), n=n) if tier == 'intersection' else {}
+    ids, mask, risk, _ = route(q.to(device), gs, x.theta[:heads].to(device), tier=tier, own=own.to(device),
+                               rep_out=slab, ties=(rows, cnt), tie_eps=1e-3, **kw)
+    ids, mask, risk = ids.cpu(), mask.cpu(), risk.cpu()
+    assert torch.equal(slab[:, :tiles].view(torch.int16), want_ops.view(torch.int16))
+    assert bool(slab[:, tiles:].isnan().all())
+    pr = ref.probes(q)
+    want = ref.risk(pr, ref.route_logits(pr, s.keys, torch.float64), s.stats, x.theta[:heads], dtype=torch.float64)
+    assert float(((risk.double() - want).abs() / want.abs().clamp_min(1e-30)).max()) < 1e-4
+    if tier == 'base':
+        assert torch.equal(ids, ref.select_base(risk, own, ids.shape[-1]))
+        assert torch.equal(mask, ref.mask_from_ids(ids, pages))
+    else:
+        want_mask = ref.quota_mask(risk, own, a, n)
+        assert torch.equal(mask, want_mask) and torch.equal(ids, ref.lut(risk, want_mask, own, ids.shape[-1]))
+    listed = rows[:int(cnt)].cpu().sort().values
+    expected = _expected_ties(risk, SimpleNamespace(own=own), tier, a, n).flatten().nonzero()[:, 0].int()
+    assert torch.equal(listed, expected) and bool((rows[int(cnt):] == -1).all())
 
 
 @pytest.mark.parametrize("single", [False, True])
