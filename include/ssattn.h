@@ -90,10 +90,12 @@ int ssa_rep_operands(const void* detail, void* rep_ops, int heads, int pages, in
  * not matter), the stand-in for the reference's Workspace
  * (VR/attention.py:7-13).  With it, the
  * workgroups past the last multiple of the device's compute-unit count run
- * as pieces of their unit lists, no more than start together with the last
- * round's other workgroups (at most 16, of at least 3 units each; none where
- * fewer than two would), and a second kernel merges the pieces' states into
- * out; NULL (or too small): every workgroup in one piece.  Results agree
+ * as up to 16 pieces of their unit lists (of the longest possible list, 3
+ * units a piece on average, two-block 4; pieces begin at even units and may be
+ * shorter or empty), no more than start together with the last round's other
+ * workgroups, none where fewer than two would -- but for the quarters of a
+ * dense call's lists of 180 units and more -- and a second kernel merges the
+ * pieces' states into out; NULL (or too small): every workgroup in one piece.  Results agree
  * within the call's tolerance, not bit for bit, between the two; each is
  * deterministic.  Calls that share a workspace must not overlap (one
  * stream, or ordered). */

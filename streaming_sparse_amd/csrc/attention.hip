@@ -641,9 +641,8 @@ __global__ __launch_bounds__(kThreads * NB, 2 / NB) void attn_kernel(AttnParams 
   issue_rows<NB>(p, src, unit(ibeg), 0, wave, lane, page_off, rep_off, kslot(ibeg & 1));
   issue_rows<NB>(p, src, unit(ibeg), 1, wave, lane, page_off, rep_off, vslot(ibeg & 1));
   issue_rows<NB>(p, src, unit(min(ibeg + 1, iend - 1)), 0, wave, lane, page_off, rep_off, kslot((ibeg + 1) & 1));
-  // the loads of unit ibeg's K have landed when no more than the later ones
-  // are left (a wave issues 4 / NB of its K rows, as many of a page's V rows,
-  // fewer of a rep tile's)
+  // all three: a wait for the first K rows alone, S before the others have
+  // landed, gained nothing
   wait_loads();
   __syncthreads();
   f32x16 S0 = s_tile(kslot(ibeg & 1), pair, lane, qop), S1;
@@ -1166,8 +1165,9 @@ void launch_merge(const AttnParams& p, int tiles, int split_from, int pieces, hi
 // The chip holds `slots` workgroups at once (the general call two per CU, the
 // two-block call one), and the last round holds wgs mod slots of them.  A
 // piece costs its start, its state (33 KB) and its share of the merge, and one
-// that waits for a slot a second latency-bound walk, so k is never more than
-// start together; and two pieces on a CU are little faster than one, so where
+// that waits for a slot a second latency-bound walk, so k is no more than start
+// together (but for the quarters of long two-block lists, below); and two
+// pieces on a CU are little faster than one, so where
 // one piece per CU already cuts a list in three, or in two after a full round,
 // k is cus / r.  Otherwise it is the most that start together, and no more
 // than kBesideWhole where whole workgroups run in the same round: they set its
@@ -1190,9 +1190,11 @@ void launch_merge(const AttnParams& p, int tiles, int split_from, int pieces, hi
 // two-block  W 22 U 308 210.2, 38.2 (11), 55.9 (12);  W 216 U 432 358.3 (1),
 // 370.1 (2);  W 288 U 288 463.8, 312.6 (8);  W 432 U 72 130.4 (1), 144.8 (2),
 // 141.0 (4).
-// Pieces hold at least min_units units: general W 24 U 36 14.9 (4 units), 14.3
-// (3), 16.1 (12 pieces, which no longer start alone); W 12 U 36 12.7, 11.9;
-// W 4 U 35 12.3, 11.4.
+// Pieces of the longest possible list hold min_units units on average (they
+// begin at even units, so 27 units in 9 pieces are pieces of 2 and 4, and a
+// list shortened by -1 entries may leave some empty): general W 24 U 36 14.9 (4
+// units), 14.3 (3), 16.1 (12 pieces, which no longer start alone); W 12 U 36
+// 12.7, 11.9;  W 4 U 35 12.3, 11.4.
 constexpr int kBesideWhole = 4;
 
 int split_plan(int wgs, int nb, int units, int* split_wgs, int* k, long long* bytes) {
@@ -1287,7 +1289,8 @@ long long ssa_attention_workspace_bytes(int n_tokens, int heads, int pages, int 
   const int nb = dense_call(flags, count, pages, n_tokens) ? 2 : 1;
   int r = 0, k = 1;
   long long bytes = 0;
-  if (split_plan(heads * (n_tokens / 64) / nb, nb, unit_bound(pages, count, nb), &r, &k, &bytes) != (int)hipSuccess) return -1;
+  if (split_plan(heads * (n_tokens / 64) / nb, nb, unit_bound(pages, count, nb), &r, &k, &bytes) != (int)hipSuccess)
+    return -1;
   return bytes;
 }
 

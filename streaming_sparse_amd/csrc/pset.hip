@@ -554,9 +554,10 @@ __device__ __forceinline__ float recip(float x) {
   return fmaf(fmaf(-x, r, 1.0f), r, r);
 }
 
-// tanh to within 1.6 ulp: below 0.625 an odd polynomial (a weighted
-// least-squares fit of (tanh x / x - 1) / x^2, 7e-9 relative), above it
-// 1 - 2 / (e^2x + 1).
+// tanh to within 1.6 ulp (just above the split, where the exponent's argument
+// is rounded once), in the form of the Cephes library's tanhf: below 0.625 an
+// odd polynomial, above it 1 - 2 / (e^2x + 1).  The coefficients are a weighted
+// least-squares fit of (tanh x / x - 1) / x^2 of our own, 7e-9 relative.
 __device__ __forceinline__ float tanh_f32(float x) {
   const float a = fabsf(x), t = x * x;
   const float pl = fmaf(fmaf(fmaf(fmaf(-0.005515433382242918f, t, 0.020469674840569496f), t, -0.05368810519576073f), t,

@@ -46,7 +46,7 @@ constexpr int kStampBlocks = 1024, kStampSlots = 16;
 __device__ unsigned long long route_stamps[kStampBlocks * 4 * kStampSlots];
 #define ROUTE_STAMP(k)                                                                       \
   do {                                                                                       \
-    if ((threadIdx.x & 63) == 0 && threadIdx.x < 256 && blockIdx.x < kStampBlocks)                                \
+    if ((threadIdx.x & 63) == 0 && threadIdx.x < 256 && blockIdx.x < kStampBlocks)           \
       route_stamps[(blockIdx.x * 4 + (threadIdx.x >> 6)) * kStampSlots + (k)] = __builtin_amdgcn_s_memtime(); \
   } while (0)
 #else
@@ -214,8 +214,11 @@ __device__ __forceinline__ void sort512_desc(unsigned long long (&key)[KPT], int
 }
 
 // Detail operand tiles written on the side by workgroups of their own,
-// appended to the router's grid: they take the slots of the CUs that hold
-// one router workgroup.  Thread c of block r writes chunk r * threads + c
+// appended to the router's grid: beside 4-wave workgroups they take the slots
+// of the CUs that hold one of them.  No 8-wave workgroup leaves room for
+// another on its CU, so those that find no free CU run after the first router
+// workgroups: up to 1.3 us (7 heads x 72 blocks, 480 pages 26.8 -> 27.7; with 4
+// waves 29.3 and 29.5).  Thread c of block r writes chunk r * threads + c
 // of the flat (head, tile, chunk) range.
 __device__ __forceinline__ void rep_operand_block(const RouteParams& p, int r, int threads) {
   const int tiles = (p.P + 15) >> 4;
@@ -553,9 +556,10 @@ __global__ __launch_bounds__(64 * NW, 2) void route_kernel(RouteParams p) {
 
   // ---------------------------------------------------------------- select
   Sel& sl = *reinterpret_cast<Sel*>(&s.ring[0][0][0]);
-  // Row b is sorted by its half of the threads, 512 64-bit keys, descending.  Key = (group << 62) | (orderable risk << 30) | (1023 - page):
-  // risk descending, ties -> lower page, and the group field orders the
-  // partitions (base / top-k: one group).
+  // Row b is sorted by its half of the threads, 512 64-bit keys, descending.
+  // Key = (group << 62) | (orderable risk << 30) | (1023 - page): risk
+  // descending, ties -> lower page, and the group field orders the partitions
+  // (base / top-k: one group).
   const int b = tid / kRowThreads, bt = tid % kRowThreads;
   int own[2];
   // own pages outside the window are clamped into it (memory safety of the
@@ -877,7 +881,10 @@ int ssa_route(const void* q, long long q_head_stride, long long q_block_stride, 
   // head x 8 blocks, 180 pages 18.1 -> 12.7 us, 2 x 72, 432 pages 22.0 -> 18.0,
   // 7 x 72, 300 pages 19.8 -> 18.1); beyond that two 4-wave workgroups share a
   // CU, which 8 waves of either kind fill with their registers, and the wide
-  // ones would run one after the other.
+  // ones would run one after the other.  The operand tiles' workgroups do not
+  // count: where they take the grid past the CUs 8 waves are still as fast
+  // or faster (quota route with tiles, 4 and 8 waves: 7 x 72 blocks, 200 pages
+  // 22.2, 22.0, 300 25.3, 24.4, 480 29.5, 27.7; 8 x 64, 480 29.7, 28.3).
   int cus = 0;
   const int e = device_cus(&cus);
   if (e != (int)hipSuccess) return e;
