@@ -92,9 +92,10 @@ def stream_handle(device=None):
     int.  A torch.device with an index is asked for its raw stream directly: the
     Stream object that torch.cuda.current_stream makes costs more than a
     kernel launch."""
-    if isinstance(device, torch.device) and device.index is not None:
-        return _raw_stream(device.index)
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index if isinstance(device, torch.device) else None
+    if index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(index)
 
 
 def check(status: int, name: str):
