@@ -1237,17 +1237,6 @@ bool spread_loads(int wgs) {
   return device_cus(&cus) == (int)hipSuccess && wgs >= 2 * cus;
 }
 
-// Whether a general call's pieces are grouped by XCD: where every tile lists
-// every page.  Tiles of a head then walk the same pages, and pieces of one
-// index the same part of them; in tile order each XCD gets every piece of every
-// head unless the pieces divide 8.  Short lists fit the L2s either way and
-// start sooner in tile order, and the tables of a sparse call share little
-// (captured, us, single-term; tile order, grouped; W tiles, U pages):  W 140 in 3
-// pieces U 32 33.0, 33.4;  U 40 36.2, 35.8;  U 72 56.4, 44.6;  U 300 164, 115;
-// W 105 in 4 U 32 30.3, 31.0;  U 48 34.2, 33.7;  W 245 in 2 U 40 63.4, 44.4;  W 852
-// U 300 580, 567;  sparse W 100 U 36 30.0, 31.7;  W 144 U 91 55.2, 56.2.
-bool group_pieces(int pages, int count) { return count == pages && pages >= 40; }
-
 // Flag bits of ssa_attention.
 constexpr int kTwoTerm = 1, kDense = 2, kStaged = 4;
 
@@ -1259,6 +1248,33 @@ bool dense_call(int flags, int count, int pages, int n_tokens) {
 
 // Units of a tile's list, at most: the listed pages and the rep tiles.
 int unit_bound(int pages, int count, int nb) { return nb == 2 ? pages : count + (pages + 15) / 16; }
+
+// Whether a general call's r split tiles (of a T-block call) run their k
+// pieces grouped by XCD.  In tile order each XCD gets pieces of every tile, so
+// of every head; only a k that is a power of two gives it the same piece
+// indices each time.
+// - Where every tile lists every page, tiles of a head walk the same pages, and
+//   pieces of one index the same part of them: grouped at any k, from 40 pages
+//   on (shorter lists fit the L2s either way and start sooner in tile order).
+//   Captured, us, single-term; tile order, grouped; W tiles, U pages:  W 140 in 3
+//   pieces U 32 33.0, 33.4;  U 40 36.2, 35.8;  U 72 56.4, 44.6;  U 300 164, 115;
+//   W 105 in 4 U 32 30.3, 31.0;  U 48 34.2, 33.7;  W 245 in 2 U 40 63.4, 44.4;  W 852
+//   U 300 580, 567.
+// - Sparse tables of one head overlap, too: with the tiles of eight heads or
+//   more in as many pieces as are no power of two, the L2s hold too little of
+//   each.  Heads x blocks, listed of window, single-term and two-term:  12 x 14
+//   in 3, 44 of 100 42.8, 37.4 and 44.5, 42.6;  80 of 470 76.4, 57.9 and 79.4,
+//   69.2;  8 x 20 in 3, 44 of 100 37.7, 35.9 and 42.6, 40.8;  10 x 9 in 5, 54 of
+//   220 41.5, 33.8 and 41.6, 36.2;  12 x 4 in 5, 80 of 470 38.5, 32.4 and 39.0,
+//   34.2.  With fewer heads short lists lose what long ones gain:  2 x 72 in 3, 44
+//   of 100 32.5, 34.0 and 36.5, 38.5;  80 of 470 55.0, 53.4 and 63.2, 63.0;  7 x
+//   24 in 3, 44 of 100 38.0, 38.5 and 42.9, 43.8.  So do the shortest pieces:  8
+//   x 3 in 10, 51 units 20.4, 20.5 and 20.8, 21.1.  In two pieces nothing is
+//   gained:  12 x 17, 80 of 220 61.5, 62.0 and 76.5, 76.2.
+bool group_pieces(int pages, int count, int r, int T, int k) {
+  if (count == pages) return pages >= 40;
+  return (k & (k - 1)) != 0 && r > 7 * T && unit_bound(pages, count, 1) >= 6 * k;
+}
 
 // Workspace bytes of a staged call: two piece states per tile.
 long long staged_bytes(int wgs) { return (long long)wgs * 2 * kPieceFloats * 4; }
@@ -1383,7 +1399,7 @@ int ssa_attention(const void* q, const void* k, const void* v, const void* keys,
     p.split_from = wgs - r;
     p.split_k = pieces;
     p.split_inv = ((1 << 20) + pieces - 1) / pieces;
-    if (!dense && group_pieces(pages, count)) p.group_inv = ((1 << 20) + r - 1) / r;
+    if (!dense && group_pieces(pages, count, r, p.T, pieces)) p.group_inv = ((1 << 20) + r - 1) / r;
   }
   const dim3 grid(p.split_from + (wgs - p.split_from) * p.split_k);
   if (dense) {

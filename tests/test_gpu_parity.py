@@ -794,6 +794,39 @@ def test_dense_many_pieces(device, heads, blocks, pages, pieces):
     check_out(out[:, rows], want, f"dense {heads}x{blocks} blocks, {pieces} pieces")
 
 
+@pytest.mark.parametrize("heads,blocks,pieces", [(12, 12, 3), (10, 9, 5), (8, 20, 3)])
+def test_attention_grouped_heads(device, heads, blocks, pieces):
+    """Tiles of eight heads and more in pieces of no power of two run in another
+    grid order; half the heads make as many pieces per tile and keep tile order:
+    equal outputs bit for bit in single- and two-term calls, with -1 padding."""
+    from streaming_sparse_amd import _lib
+    pages, count = 64, 30
+    gen = torch.Generator().manual_seed(heads)
+    n, half = 64 * blocks, heads // 2
+    q = torch.randn(1, n, heads, 128, generator=gen).bfloat16().to(device)
+    k = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    v = torch.randn(1, 64 * pages, heads, 128, generator=gen).bfloat16()
+    vp = v[0].transpose(0, 1).reshape(heads, pages, 64, 128)
+    basis = workload.pca_basis(vp.float()).to(device)
+    s = workload.kmeans_summaries(k[0].transpose(0, 1).reshape(heads, pages, 64, 128), vp, basis.cpu(),
+                                  torch.Generator().manual_seed(9))
+    gd = Summary(*(getattr(s, f).to(device) for f in Summary.FIELDS))
+    k, v = k.to(device), v.to(device)
+    ids = torch.stack([torch.randperm(pages, generator=gen)[:count] for _ in range(heads * blocks)])
+    ids = ids.reshape(heads, blocks, count).int().to(device)
+    ids[:, ::3, count // 2:] = -1
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        for h in (heads, half):
+            assert _lib.lib().ssa_attention_workspace_bytes(n, h, pages, count, 1) == h * blocks * pieces * 33280
+    for single in (False, True):
+        got = attention(q, k, v, gd, basis, ids, Workspace(), single_av=single)
+        for at in (slice(0, half), slice(half, heads)):
+            sub = Summary(*(getattr(gd, f)[at].contiguous() for f in Summary.FIELDS))
+            want = attention(*(t[:, :, at].contiguous() for t in (q, k, v)), sub, basis[at], ids[at], Workspace(),
+                             single_av=single)
+            assert torch.equal(got[:, :, at].contiguous().view(torch.int16), want.view(torch.int16))
+
+
 def test_empty_pieces_leave_no_stamps(device):
     """Measurement build: a piece without units records zeros, where an earlier
     call's piece of the same workgroup had left its steps."""
