@@ -33,9 +33,9 @@
 //   frames_kernel    grid (B): the first chunk's stable partition by frame
 // 30 layers x 12 heads: 5.26 ms (a workgroup per row and seven passes over its
 // rows per level, sums over rows through serial LDS walks, bitonic sorts in
-// LDS) -> 1.92 ms: project 0.58, totals 0.01, features 0.24, level 0 0.24
-// (direction 0.014, keys 0.11, sort 0.11), level 1 0.20, level 2 0.17, fused
-// levels 0.48.  One layer x 12 heads: 862 -> 249 us.
+// LDS) -> 1.92 ms: project 0.59, totals 0.01, features 0.24, level 0 0.24
+// (direction 0.014, keys 0.11, sort 0.12), level 1 0.20, level 2 0.17, fused
+// levels 0.49.  One layer x 12 heads: 862 -> 249 us.
 #include "common.h"
 
 #include <type_traits>
@@ -149,7 +149,7 @@ __device__ __forceinline__ Stat xor_stat(const Stat& s) {
 // k order of the product is free, so no LDS staging is needed).  Bound by the
 // fp64 pipe: 27.2 GFLOP per 30-layer batch, 0.39 ms at the 70 TFLOP/s a loop
 // of these products reaches, and the operands' conversions (to 0.51 ms) and
-// the statistics (to 0.58 ms) share it; as fp64 vector FMAs with a conversion
+// the statistics (to 0.59 ms) share it; as fp64 vector FMAs with a conversion
 // per operand the projections alone took 1.01 ms.
 __global__ __launch_bounds__(256, 2) void project_kernel(GroupParams p) {
   __shared__ double sh[2][16][kStatVals];
@@ -805,8 +805,8 @@ __global__ __launch_bounds__(THREADS) void level_kernel(GroupParams p, int src) 
 // where a block spans waves, one LDS round with one barrier each.  The sort
 // runs one element per thread, by lane exchanges up to distance 32.  The last
 // level writes the final order.  Bound by fp64 vector issue, two workgroups
-// per CU: per 30-layer batch 0.48 ms, half of it power steps (with level 2 in
-// here too, 512 rows and one workgroup per CU: 0.77 ms against 0.48 + 0.17; at
+// per CU: per 30-layer batch 0.49 ms, half of it power steps (with level 2 in
+// here too, 512 rows and one workgroup per CU: 0.77 ms against 0.49 + 0.17; at
 // the start 1.65 ms, with every pass from LDS and its sums through a 64-deep
 // serial LDS walk).
 constexpr int kFuse = 256;

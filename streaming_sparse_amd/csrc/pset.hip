@@ -115,12 +115,12 @@ union EncSmem {
 // products and sums).  Layer 1: wave w takes hidden units 64 (w % 4) .. + 63
 // over half w / 4 of the 712 features; lane (c = l % 16, g = l / 16) loads
 // units 4 c .. 4 c + 3 of a feature's weight row (256 bytes per row and
-// wave), well ahead, each item one product.  Bound by the fp32 matrix rate,
-// 9.5 us per workgroup, on the 108 CUs that 72 x 12 pages fill, then by the
-// latency of the steps around it.  72 x 12 pages, as part of a correction
-// call: 42 us (4 pages and both MLPs per workgroup as vector FMAs at one wave
-// per SIMD, layer 2 as 256-long serial dot products, meanB after it) -> 17;
-// 432 x 12 pages 126 -> 80.
+// wave), well ahead, each item one product.  Products take 9.5 us of a
+// workgroup's time (the fp32 matrix pipe is 37% busy on the 108 CUs that 72 x
+// 12 pages fill), the latency of the steps around them the rest.  72 x 12
+// pages, kernel trace of a correction call: 42 us (4 pages and both MLPs per
+// workgroup as vector FMAs at one wave per SIMD, layer 2 as 256-long serial dot
+// products, meanB after it) -> 29;  432 x 12 pages, captured, 136 -> 80.
 template <class Layers>
 __global__ __launch_bounds__(kEncThreads) void encode_kernel(EncodeParams p, Layers layers) {
   if constexpr (std::is_same_v<Layers, EncodeLayers>) {
@@ -375,7 +375,7 @@ struct PoolSmem {
 // pages other than own; the unselected pages by descending risk, then the
 // selected pages in page order; the movable removes x the first 16 add
 // slots are legal.  One key per thread; 3 heads x 72 blocks, kernel trace:
-// 9.5 us (two keys per thread, every step through LDS) -> 7.8 us.
+// 9.5 us (two keys per thread, every step through LDS) -> 8.3 us.
 __global__ __launch_bounds__(kMaxPages) void pset_pool_kernel(PsetParams p) {
   __shared__ PoolSmem s;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -583,10 +583,11 @@ __device__ __forceinline__ Const<T>* scalar(const T* p) {
 // the readout (rp, beta) and the summary approximation; candidate pages write
 // their endpoint data, the background pages (in no pool slot) enter the
 // mixture sums B (the current selection's weights) and T (every page exact),
-// which the scores kernel completes with the candidates.  Bound by vector
-// issue: ~440 fp32 and fp64 instructions per page and 64 probes, the fp64 ones
-// at half rate (with the page data always in the scalar cache the kernel is
-// 12% faster).  The scalar cache reads whole 4-byte words and drops the low
+// which the scores kernel completes with the candidates.  Vector issue
+// takes about two thirds of the time a CU holds a workgroup (~440 fp32 and
+// fp64 instructions per page and 64 probes, the fp64 ones at half rate), and
+// waves wait 47% of theirs, mostly for scalar loads (with the page data always
+// in the scalar cache the kernel is 12% faster).  The scalar cache reads whole 4-byte words and drops the low
 // bits of an address, so coefficients that start between two words (a view at
 // an odd element; the encode kernel writes those too) take the instance
 // without WORDS, which reads them one by one.  432 pages, 3 heads x 72 blocks, kernel trace: 94 us (32 probes
@@ -882,8 +883,8 @@ struct ScoreSmem {
 // chain of dependent steps per probe, two probes per wave at two waves per
 // SIMD.  3 heads x 72 blocks, kernel trace: 48 us (all 512 pairs, three fp64
 // products per pair and dim, four probes per wave) -> 27 us; with its LDS reads
-// in groups (a read behind a write or a lane's condition waited for itself) the
-// correction call went from 147.7 to 145.5 us.
+// in groups (a read behind a write or a lane's condition waited for itself) ->
+// 25 us, the correction call 147.7 -> 145.5.
 __global__ __launch_bounds__(kScoreThreads) void pset_scores_kernel(PsetParams p) {
   __shared__ ScoreSmem s;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;

@@ -26,8 +26,8 @@
 // ascending token order.  LDS stays under 40 KB so four workgroups share a
 // CU.
 //
-// Vector instructions bound it (the vector pipes are about two thirds busy
-// over the kernel's life), not the 1 KB per row that it moves: 72 pages of
+// Vector instructions take most of it (the vector pipes are 71% busy while a
+// CU holds a workgroup), not the 1 KB per row that it moves: 72 pages of
 // 12 heads written through take 23.1 us, 11.3 us of it for their bytes.
 // Lane masks of the cluster sums are picked once per Lloyd step instead of
 // once per matrix step, and the detail formed once per wave instead of once
